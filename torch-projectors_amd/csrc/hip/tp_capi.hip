@@ -257,16 +257,17 @@ tp::TileSpec2 tile_spec2(const tp::Geom& g, bool cubic) {
     };
     tiles_within(rho_unit + 1.0, ts.kr0, ts.nr, ts.nc);
     tiles_within(rho, ts.kr0_2, ts.nr_2, ts.nc_2);
-    // Every pose reaches every tile of the disc: split the poses into ranges until there are
-    // about 65536 work items, keeping >= 128 poses a range.  A workgroup's item is long (all of
-    // its range's poses cross its tile), so many short items balance the CUs far better than the
-    // partial tiles' extra float atomics cost: c5's backprojection (1360 tiles, 4096 poses)
-    // took 13.07 ms at about 4096 items (4 ranges), 11.72 at 8192, 10.18 at 32768 and 10.03
-    // at 32 ranges of 128 poses; ranges of 84 poses 10.05, of 43 poses 10.23 ms (A/B medians;
-    // its reconstruction gradient 16.50 -> 13.54 ms).
+    // Every pose reaches every tile of the disc: split the poses into ranges until there are about
+    // 32768 work items, keeping >= 32 poses a range.  A workgroup's item is long (all of its range's
+    // poses cross its tile), so many short items balance the CUs far better than the partial tiles'
+    // extra float atomics cost: 8 images of 100 x 100 with 500 poses each (112 tiles) took 1.11 ms
+    // in ranges of 167 poses (336 items), 0.43 ms of 64, 0.36 of 32 and 0.33 of 16; 16 x 512 poses of
+    // 256 x 256 (1440 tiles, a cubic step) 2.84 / 2.81 / 2.83 ms with ranges of 64 / 32 / 16, and
+    // 16 x 4096 of them 10.18 ms at 16384 items, 9.7 at 32768 and 65536.  Ranges of 16 pay only while
+    // the items are few (below about 4096); past that they cost up to 3 % by their fixed work.
     const int64_t tiles = g.B * int64_t(ts.nr) * ts.nc;
-    const int64_t want = tiles > 0 ? (65536 + tiles - 1) / tiles : 1;
-    const int64_t most = std::max<int64_t>(1, g.P / 128);
+    const int64_t want = tiles > 0 ? (32768 + tiles - 1) / tiles : 1;
+    const int64_t most = std::max<int64_t>(1, g.P / (tiles * (g.P / 32) < 4096 ? 16 : 32));
     ts.ksplit = int(std::max<int64_t>(1, std::min(want, most)));
     ts.prange = int((g.P + ts.ksplit - 1) / ts.ksplit);
     ts.rho = float(rho);

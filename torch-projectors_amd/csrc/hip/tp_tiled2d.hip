@@ -173,10 +173,14 @@ __device__ __forceinline__ void cull2(const float* __restrict__ rotb, int pend, 
 }
 
 // LDS layout of the accumulators: cell (lc, lr) sits at
-// lr * TC + ((lc + swizzle2(lr)) mod TC).  Samples stepping along r land two
-// rows apart; the rotation by lr / 2 spreads them over different banks (an
-// fp64 cell spans two of the 64 four-byte banks).
-__device__ __forceinline__ int swizzle2(int lr) { return (lr >> 1) & (TC - 1); }
+// lr * TC + ((lc + swizzle2(lr)) mod TC).  An fp64 cell spans two of the 64
+// four-byte banks, so a row of TC = 32 cells covers them all and neighbouring
+// rows must be rotated against each other.  The rotation by 5 lr spreads a
+// window's lanes best over random in-plane angles: counted on the CPU, the
+// busiest bank of 32 lanes takes 2.65 of them at oversampling 1 (2.5 at 1.25),
+// against 4.7 (4.1) with a rotation by lr / 2.  8 images of 100 x 100, 500
+// poses each, linear with weights: 0.445 -> 0.365 ms (same pose ranges).
+__device__ __forceinline__ int swizzle2(int lr) { return (5 * lr) & (TC - 1); }
 
 // Per-pass constants: local cell of tap j on axis a is sgn * floor(x_a) + off[a] + sgn * j
 // (sgn = -1 for the flipped taps), valid in [lmin[a], S_a).
@@ -243,21 +247,27 @@ __device__ __forceinline__ void scatter_sample2(const Geom& g, const Slot2& sd, 
 // lie in distinct cells: the lanes of one tap never share a cell.  A wave's
 // LDS operations execute in order; the signal fence keeps the compiler from
 // moving one tap's read above the previous tap's write (another lane's tap
-// may have written that cell).  The private tile has rows of PS = TC + 1
-// cells (the odd stride spreads a column over the banks) and one row more: a
-// tap outside the tile goes to that row or to a row's last cell, which are
+// may have written that cell).  The private tile has rows of priv_stride
+// cells (an odd stride spreads a column over the banks) and one row more: a
+// tap outside the tile goes to that row or to a row's cell TC, which are
 // never written out, so every tap runs without a test or branch (lanes that
-// share those cells only lose garbage).  v * wr is rounded as the reference
+// share those cells only lose garbage).  The cubic stencil's 16 taps are
+// bound by LDS: a stride of TC + 5 leaves the busiest bank of 32 lanes 2.65
+// lanes at oversampling 2 (TC + 1: 3.4; counted on the CPU), 16 x 512 poses of
+// 256 x 256 in a step 2.84 -> 2.81 ms.  The linear stencil's four taps are not,
+// and lose more by the larger tile (1.44 against 1.50 ms for 7 x 3561 poses
+// of 84 x 84, forward and backward), so they keep TC + 1.  v * wr is rounded as the reference
 // forms it; the product with wc is fused into the fp32 sum (and the weight
 // tap wpix * |wr * wc| into its sum as (wpix * |wr|) * |wc|), one rounding per
 // tap fewer than the reference's order, far below the per-cell bar, and still
 // exactly 0 where every tap weight is.
-constexpr int PS = TC + 1, PT = (TR + 1) * PS;  // private tile: row stride, cells
+template <bool CUBIC> constexpr int priv_stride = TC + (CUBIC ? 5 : 1);            // private tile: row stride
+template <bool CUBIC> constexpr int priv_cells = (TR + 1) * priv_stride<CUBIC>;  // and cells
 template <bool CUBIC, int MODE, bool WEIGHTS>
 __device__ __forceinline__ void scatter_sample2_priv(const Geom& g, const Slot2& sd, int rr, int cc, Cx<float> v,
                                                      float wpix, bool shifted, bool flip, const TapMap2& tm,
                                                      float2* pc, float* pw) {
-    constexpr int K = CUBIC ? 4 : 2;
+    constexpr int K = CUBIC ? 4 : 2, PS = priv_stride<CUBIC>;
     const float fr = float(rr), fc = float(cc);
     float x[2];
     rotate_pix(sd.R, fr, fc, g.os, x);
@@ -321,7 +331,7 @@ __global__ __launch_bounds__(kThreads) void k_scatter2_tiled(Geom g, TileSpec2 t
     constexpr int RPS = 64 / KP;
     constexpr int NW = kThreads / 64;
     static_assert(!PRIV || KP == 1, "private accumulation needs one pose per window");
-    constexpr int TS = PRIV ? 1 : T2, TP = PRIV ? PT : 1;
+    constexpr int PS = priv_stride<CUBIC>, TS = PRIV ? 1 : T2, TP = PRIV ? priv_cells<CUBIC> : 1;
     __shared__ double acc_re[TS], acc_im[TS];
     __shared__ double acc_w[WEIGHTS ? TS : 1];
     __shared__ float2 pacc[NW][TP];
