@@ -15,6 +15,15 @@ pytestmark = pytest.mark.gpu
 
 def _cases():
     out, seed = [], 771000
+    # 3D: tiles in one, two and three levels of pieces (few and many poses for the box), one-pose pieces
+    for op in ("project_3d_to_2d_forw", "project_3d_to_2d_back", "backproject_2d_to_3d_forw",
+               "backproject_2d_to_3d_back"):
+        for interp, os_ in (("linear", 2.0), ("cubic", 1.0), ("linear", 1.5)):
+            for n, P in ((16, 47), (16, 49), (32, 130), (48, 260)):
+                seed += 1
+                out.append(_case(f"{op}_{interp}_n{n}_os{os_:g}_P{P}", op, interp=interp, os=os_,
+                                 cutoff=11.0 if n == 32 else None, B=2, P=P, n=n, B_rot=2, seed=seed,
+                                 weights=(seed % 2 == 0)))
     for op in ("backproject_2d_forw", "project_2d_back"):
         for interp, os_ in (("linear", 1.0), ("cubic", 1.0), ("cubic", 2.0)):
             for n, P in ((32, 1), (32, 15), (30, 31), (48, 33), (40, 65)):

@@ -131,18 +131,83 @@ int scatter_poses_per_batch(double w, double eps, double os) {
     return rows <= 14 ? 6 : (rows <= 21 ? 4 : (rows <= 32 ? 3 : 1));
 }
 
-// Poses per range of the forward projection's rotation kernel's core tiles: 2048 at oversampling 2
+// Poses per piece of the forward projection's rotation kernel in large calls: 2048 at oversampling 2
 // and above, fewer as the oversampling (and so the spacing of a pose's samples) shrinks, so that a
-// range holds about as many samples: at oversampling 1 a core tile holds four times the samples
+// piece holds about as many samples: at oversampling 1 a core tile holds four times the samples
 // per pose, and unsplit core tiles became the critical path there (the published rows' linear
 // batch-1 forward 0.50 -> 0.86 ms at 2048), so it takes 512 like the rest.
 int64_t forw_poses_per_range(double os) {
     const double r = 2048.0 * (os / 2.0) * (os / 2.0);
     return r >= 2048.0 ? 2048 : (r <= 512.0 || !(r == r) ? 512 : int64_t(r));
 }
-// pkf: poses per range of the rotation forward-family kernels' core tiles (forward projections
-// take forw_poses_per_range, their backward ops the scatter's 512).
-tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, int64_t pkf = 512) {
+
+// Most pieces of split tiles of one scatter call (12-18 KB of workspace each: up to 2.4 GB) and of one
+// gather call (which needs none); a call of more takes longer pieces.
+constexpr double kMaxScatterPieces = double(1 << 17), kMaxGatherPieces = double(1 << 30);
+
+// Pose ranges of a 3D tile grid (tp::PoseSplit): n tiles per axis (d, r, c) of `edge` voxels from the
+// signed coordinate `org`, for samples within `reach` of the origin; `stencil` voxels more per axis
+// belong to a tile's box.
+//   A random slice plane crosses a tile at distance x with probability h / x, h the mean half width of
+// its box, so a call crosses about `cross` (pose, tile) pairs (half of the ball: a pose's samples
+// fill half of its plane).  A tile's pieces hold about `target` expected poses:
+//   - cross / per_slot over the 1024 workgroups that run at once, at least `least` (a piece's fixed
+//     work: staging or clearing its tile, its cull, its write-out), in levels of growing distance.  With
+//     the whole pose list in one workgroup the centre tiles were small calls' critical path: 2 x 333
+//     poses of 90 x 90 at oversampling 1.5, cubic forward and backward 1.59 -> 0.84 ms; 1000 poses of
+//     64 x 64 at 2, linear: backprojection 0.211 -> 0.124, projection with all gradients 0.549 -> 0.279 ms;
+//     1000 of 64 x 64 at 1, cubic backprojection 3.34 -> 0.65 ms.
+//   - in calls where that is 512 poses or more (and without `levels`: when the call can have no list
+//     of its pieces), one level of 40 voxels with `range` poses per piece: there the levels measured
+//     slower (the headline backprojection 1.33 -> 1.39 ms: less of the projections' rows is shared
+//     by the pieces that run together).
+tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const int org[3], const int edge[3],
+                         double stencil, double per_slot, double least, int64_t range, double most, bool levels) {
+    constexpr double kSlots = 1024.0, kLongRange = 512.0;
+    const double h = 0.25 * (edge[0] + edge[1] + edge[2] + 3.0 * stencil);
+    const double vt = double(edge[0]) * edge[1] * edge[2], R = std::max(reach, h);
+    const double cross =
+        double(g.B) * double(g.P) * 2.0 * M_PI / vt * (h * h * h / 3.0 + h * (R * R - h * h) / 2.0);
+    double target = std::max(least, cross / (kSlots * per_slot));
+    const bool one_level = !levels || target >= kLongRange;
+    if (one_level) target = double(range);
+    tp::PoseSplit ps{};
+    double r = one_level ? 40.0 : 16.0, p = 1.0;  // this level's half width; share of the poses that cross its tiles
+    double total = 0.0;
+    for (int l = 0; l < (one_level ? 1 : tp::kSplitLevels); ++l, r *= 2.0) {
+        const int64_t k = int64_t(std::ceil(double(g.P) * p / target));
+        if (k <= 1) break;
+        tp::PoseSplit::Level& v = ps.lv[l];
+        int64_t tiles = 1;
+        for (int a = 0; a < 3; ++a) {
+            const double rc = std::min(r, reach);
+            v.lo[a] = std::max(0, int(std::floor((-rc - org[a]) / edge[a])));
+            const int hi = std::max(v.lo[a], std::min(n[a], int(std::floor((rc - org[a]) / edge[a])) + 1));
+            v.ext |= unsigned(hi - v.lo[a]) << (10 * a);
+            tiles *= hi - v.lo[a];
+        }
+        total += double(g.B) * double(tiles) * double(k);
+        if (total > most || k > tp::kMaxTilePieces || double(ps.pieces) + double(tiles) * double(k) > double(INT32_MAX))  // (twice as long until they fit)
+            return pose_split(g, reach, n, org, edge, stencil, per_slot / 2.0, 2.0 * target, 2 * int64_t(target), most,
+                              levels);
+        v.k = int(k);
+        v.pieces = int(tiles * k);
+        ps.n = l + 1;
+        ps.pieces += v.pieces;
+        if (r >= reach) break;
+        p = std::min(1.0, h / (r + 6.0));
+    }
+    return ps;
+}
+
+// The op a TileSpec is for: its pose ranges differ.
+enum class TileOp { project, gradients, backproject };
+// The pose ranges of a call's tile grids (forward, the other poses' wider forward grid, scatter): in
+// levels, and in the one level of a call without a list of its pieces.
+struct Splits {
+    tp::PoseSplit f[2], f2[2], s[2];
+};
+tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, Splits& sp) {
     constexpr int L = tp::kTileEdge;
     tp::TileSpec ts{};
     // radius bound of the active pixels: the cutoff disc, within the pixel grid
@@ -168,38 +233,29 @@ tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, int64_t pkf = 512) {
     ts.ntd = (g.N + tp::kScTD - 1) / tp::kScTD;
     ts.ntr = (g.N + tp::kScTR - 1) / tp::kScTR;
     ts.ntc = (g.H + tp::kScTC - 1) / tp::kScTC;
-    // Every random slice plane crosses the tiles around the origin, so those
-    // carry up to P poses each; they are split into pose ranges so that no
-    // single workgroup holds the critical path.  Core = tiles within `rc`
-    // voxels of the origin on every axis.
-    const int rc = 40;
-    ts.fc0 = std::max(0, (-rc - ts.org) / L);
-    ts.fc1 = std::min(ts.nt, (rc - ts.org) / L + 1);
-    ts.fd0 = std::max(0, (-rc - ts.orgd) / tp::kTileEdgeD);
-    ts.fd1 = std::min(ts.ntfd, (rc - ts.orgd) / tp::kTileEdgeD + 1);
-    ts.fc0_2 = std::max(0, (-rc - ts.org2) / L);
-    ts.fc1_2 = std::min(ts.nt2, (rc - ts.org2) / L + 1);
-    ts.fd0_2 = std::max(0, (-rc - ts.orgd2) / tp::kTileEdgeD);
-    ts.fd1_2 = std::min(ts.ntfd2, (rc - ts.orgd2) / tp::kTileEdgeD + 1);
-    ts.sd0 = std::max(0, (-rc + half - 1) / tp::kScTD);
-    ts.sd1 = std::min(ts.ntd, (rc + half - 1) / tp::kScTD + 1);
-    ts.sr0 = std::max(0, (-rc + half - 1) / tp::kScTR);
-    ts.sr1 = std::min(ts.ntr, (rc + half - 1) / tp::kScTR + 1);
-    ts.sc1 = std::min(ts.ntc, rc / tp::kScTC + 1);
-    // poses per range: the scatter's core tiles carry the most work of its grid and split at 512
-    // (at 1024 the headline backprojection took 1.41 ms against 1.34; backprojection_ranges
-    // lengthens them for calls of more than 2048 poses), as do the kernels of the
-    // other tiled poses and the gradient modes (1-4 % slower at 2048); the rotation forward
-    // projection's split at pkf (at oversampling 2, c2's forward 0.317 ms at 512 against 0.299 at
-    // 2048, the headline's the same)
-    const int64_t pk = 512;
-    ts.ksplit = int(std::max<int64_t>(1, (g.P + pk - 1) / pk));
-    ts.prange = int((g.P + ts.ksplit - 1) / ts.ksplit);
-    ts.fksplit = int(std::max<int64_t>(1, (g.P + pkf - 1) / pkf));
-    ts.fprange = int((g.P + ts.fksplit - 1) / ts.fksplit);
-    if (ts.ksplit == 1)  // nothing to split
-        ts.fc1_2 = ts.fc0_2 = ts.fd1_2 = ts.fd0_2 = ts.sd1 = ts.sd0 = ts.sr1 = ts.sr0 = ts.sc1 = 0;
-    if (ts.fksplit == 1) ts.fc1 = ts.fc0 = ts.fd1 = ts.fd0 = 0;
+    // Pieces of the tiles' poses.  Measured targets (calls in pose_split's comment): the gathers stage
+    // their tile once per piece and do best with half as many pieces as slots would take; the
+    // scatters' pieces, above all the cubic ones, hold more work per pose.  In large calls the
+    // scatter's core tiles carry the most work of its grid and take 512 poses per piece (at 1024 the
+    // headline backprojection took 1.41 ms against 1.34), the backprojection of more than 2048 poses
+    // about four pieces of up to 2048 (8192 poses of 128 x 128: 1.369 ms at 512, 1.347 at 2048); the
+    // gradient modes and the kernels of the other tiled poses 512 (1-4 % slower at 2048); the forward
+    // projection's rotation kernel forw_poses_per_range (at oversampling 2, 4096 poses of 128 x 128 take
+    // 0.317 ms at 512 against 0.299 at 2048, the headline the same).
+    const int nf[3] = {ts.ntfd, ts.nt, ts.nt}, of[3] = {ts.orgd, ts.org, ts.org}, ef[3] = {tp::kTileEdgeD, L, L};
+    const int nf2[3] = {ts.ntfd2, ts.nt2, ts.nt2}, of2[3] = {ts.orgd2, ts.org2, ts.org2};
+    const int nsc[3] = {ts.ntd, ts.ntr, ts.ntc}, osc[3] = {1 - half, 1 - half, 0},
+              esc[3] = {tp::kScTD, tp::kScTR, tp::kScTC};
+    const double flo = op == TileOp::project ? 64.0 : 32.0;
+    for (int i = 0; i < 2; ++i) {
+        const bool lv = i == 0;
+        sp.f[i] = pose_split(g, rho_unit, nf, of, ef, 0.0, 0.5, flo,
+                             op == TileOp::project ? forw_poses_per_range(g.os) : 512, kMaxGatherPieces, lv);
+        sp.f2[i] = pose_split(g, rho_unit, nf2, of2, ef, 0.0, 0.5, flo, 512, kMaxGatherPieces, lv);
+        sp.s[i] = pose_split(g, rho_unit, nsc, osc, esc, cubic ? 3.0 : 1.0, cubic ? 1.5 : 1.0, cubic ? 16.0 : 48.0,
+                             op == TileOp::backproject ? std::min<int64_t>(2048, std::max<int64_t>(512, g.P / 4)) : 512,
+                             kMaxScatterPieces, lv);
+    }
     ts.rho = float(rho);
     ts.rho_unit = float(rho_unit);
     ts.os = float(g.os);
@@ -218,17 +274,6 @@ tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, int64_t pkf = 512) {
     ts.rmin = std::max(g.n / 2 + 1 - g.n, -cl);
     ts.rmax = std::min(g.n / 2, cl);
     return ts;
-}
-
-// Pose ranges of the backprojection's core tiles: about four per call, from 512 up to 2048
-// poses each (512 for up to 2048 poses, as tile_spec sets them).  With more poses a range of
-// 512 left the core's global float atomics the larger cost: c3's shape (8192 poses) took
-// 1.369 ms at 512, 1.347 ms at 2048 and 1.372 ms at 1024 poses per range (A/B medians).  The
-// reconstruction-gradient scatter keeps 512 (the cubic one was slower with longer ranges).
-void backprojection_ranges(const tp::Geom& g, tp::TileSpec& ts) {
-    const int64_t pk = std::min<int64_t>(2048, std::max<int64_t>(512, g.P / 4));
-    ts.ksplit = int(std::max<int64_t>(1, (g.P + pk - 1) / pk));
-    ts.prange = int((g.P + ts.ksplit - 1) / ts.ksplit);
 }
 
 // fp32 2D operators take the tile-owner kernels (tp_tiled2d.hip) for tiled poses (pose_tiled2).
@@ -345,17 +390,17 @@ struct StreamScratch {
     // until the process ends; growth is geometric, so these stay a small multiple of the last).
     bool bins_captured = false;
     std::vector<void*> bins_retired;
-    // The rotation forward kernels' lists of work items in reach (tp::TileSpec::flist) of the
-    // last few geometries; a list that a capture has used is retired in the same way.
+    // Lists of work items (tp::TileSpec::flist, tp::SplitView::list) of the last few geometries; a
+    // list that a capture has used is retired in the same way.
     struct ForwList {
         std::vector<int64_t> key;
-        int* p = nullptr;
+        tp::TileItem* p = nullptr;
         size_t cap = 0;
         int64_t count = 0;
         bool captured = false;
         uint64_t used = 0;
     };
-    ForwList flists[4];
+    ForwList flists[12];  // (a projection with gradients uses four)
     uint64_t flist_tick = 0;
     std::vector<void*> flist_retired;
 };
@@ -451,13 +496,13 @@ struct CallScratch {
         if (capturing) area->bins_captured = true;
         return area->bins;
     }
-    // The rotation forward kernels' list of work items in reach for the geometry of g and ts
-    // (tp::forw_reach_items), or nullptr (the kernels then take every work item of their grid).
-    // The area keeps the lists of its last four geometries; another geometry is listed on the host
-    // and copied in on the call's stream, which is then synchronised (once per new geometry). A
-    // stream under graph capture takes a list that the area holds for its geometry, else none, and
-    // a list that a capture has used is retired, never rewritten or freed.
-    const int* forw_list(const tp::Geom& g, const tp::TileSpec& ts, hipStream_t st, int64_t& count) {
+    // The list of work items with this key (everything it depends on), or nullptr (the kernels then
+    // take every work item of their grid, split in one level).  The area keeps the last twelve; another
+    // one is listed on the host (`build` appends it) and copied in on the call's stream, which is then
+    // synchronised (once per new key).  A stream under graph capture takes a list that the area holds,
+    // else none, and a list that a capture has used is retired, never rewritten or freed.
+    template <typename F>
+    const tp::TileItem* item_list(const std::vector<int64_t>& key, hipStream_t st, int64_t& count, F&& build) {
         if (static_area || !area) return nullptr;
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
@@ -465,12 +510,6 @@ struct CallScratch {
             return nullptr;
         }
         const bool capturing = cs != hipStreamCaptureStatusNone;
-        uint32_t rho_bits = 0, eps_bits = 0;
-        std::memcpy(&rho_bits, &ts.rho_unit, 4);
-        std::memcpy(&eps_bits, &ts.eps, 4);
-        // everything the list depends on (the pose count only through fksplit)
-        const std::vector<int64_t> key{g.B, ts.nt, ts.org, ts.ntfd, ts.orgd, ts.fc0, ts.fc1, ts.fd0, ts.fd1,
-                                       ts.fksplit, int64_t(rho_bits), int64_t(eps_bits)};
         StreamScratch::ForwList* victim = nullptr;
         for (StreamScratch::ForwList& f : area->flists) {
             if (f.p && f.key == key) {
@@ -482,10 +521,9 @@ struct CallScratch {
             if (!victim || (victim->p && (!f.p || f.used < victim->used))) victim = &f;
         }
         if (capturing) return nullptr;
-        std::vector<int> host;
-        const int64_t items = tp::forw_reach_items(g, ts, host);
-        if (items > int64_t(INT32_MAX) || host.empty()) return nullptr;
-        const size_t need = host.size() * sizeof(int);
+        std::vector<tp::TileItem> host;
+        if (!build(host) || host.empty()) return nullptr;
+        const size_t need = host.size() * sizeof(tp::TileItem);
         // queued work may still read the list that is replaced
         if (hipStreamSynchronize(st) != hipSuccess) {
             (void)hipGetLastError();
@@ -561,7 +599,7 @@ struct CallScratch {
 };
 
 // Summary of the call's poses for its tiled kernels (tp::launch_call_poses), which also clears the
-// counts of the pose bins that plan_bins laid out in ts (if any).
+// counts of the pose bins that plan_scatter laid out in ts (if any).
 int call_poses(int dim, const tp::Geom& g, const void* rot, float rho_unit, CallScratch& sc, hipStream_t s,
                const tp::TileSpec* ts = nullptr) {
     TP_TRY(sc.get(s));
@@ -571,40 +609,72 @@ int call_poses(int dim, const tp::Geom& g, const void* rot, float rho_unit, Call
                     "pose summary launch");
 }
 
-// Pose bins of the tiled 3D scatter's tile grid for this call (tp::BinGrid), in 2 x 2 x 2 tiles:
-// plan_bins lays them out in the stream's workspace (ts.sbins; the pose summary then clears their
-// counts) and fill_bins fills them after the summary.  None below kBinsMinPoses poses, from 65536
-// poses (list entries are 16-bit), beyond kBinsMaxBytes or tp::kBinMaxGroups workgroups of the
-// pre-pass, and none without a workspace: the scatter then culls every pose of each tile.
+// A split as the kernels take it: its pieces listed when it has several levels, or the one-level
+// split (`ps` then becomes that) when the call's (device, stream) area can hold no list.
+tp::SplitView split_view(tp::PoseSplit& ps, const tp::PoseSplit& one, int64_t B, CallScratch& sc, hipStream_t s) {
+    const tp::TileItem* list = nullptr;
+    if (ps.n > 1) {
+        std::vector<int64_t> key{1, B};
+        for (int l = 0; l < ps.n; ++l) {
+            const tp::PoseSplit::Level& v = ps.lv[l];
+            key.insert(key.end(), {v.lo[0], v.lo[1], v.lo[2], int64_t(v.ext), v.k});
+        }
+        int64_t count = 0;
+        list = sc.item_list(key, s, count, [&](std::vector<tp::TileItem>& out) {
+            tp::split_items(ps, B, out);
+            return true;
+        });
+        if (!list) ps = one;
+    }
+    tp::SplitView v{};
+    if (ps.n > 0) v.box = ps.lv[ps.n - 1];
+    v.pieces = ps.pieces;
+    v.list = list;
+    return v;
+}
+
+// Workspace of the tiled 3D scatter for this call: the slots of the split tiles' pieces
+// (tp::TileSpec::part), and the pose bins of its tile grid (tp::BinGrid) in 2 x 2 x 2 tiles, which
+// plan_scatter lays out (the pose summary then clears their counts) and fill_bins fills after the
+// summary.  No bins below kBinsMinPoses poses, from 65536 poses (list entries are 16-bit), beyond
+// kBinsMaxBytes or tp::kBinMaxGroups workgroups of the pre-pass; without a workspace (a failed
+// allocation, or growth under graph capture) no bins and no split tiles: every tile then takes all
+// of the call's poses itself.
 constexpr int64_t kBinsMinPoses = 16;
 constexpr size_t kBinsMaxBytes = size_t(1) << 30;
-int plan_bins(const tp::Geom& g, tp::TileSpec& ts, CallScratch& sc, hipStream_t s) {
+int plan_scatter(const tp::Geom& g, tp::TileSpec& ts, Splits& sp, bool weights, CallScratch& sc, hipStream_t s) {
     ts.sbins = tp::BinGrid{};
     TP_TRY(sc.get(s));
-    if (g.P < kBinsMinPoses || g.P >= 65536) return TP_OK;
+    ts.ssplit = split_view(sp.s[0], sp.s[1], g.B, sc, s);
+    auto align = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t slots = align(size_t(g.B) * size_t(ts.ssplit.pieces) * size_t(tp::slot_bytes(weights)));
     tp::BinGrid sb{};
     sb.nb[0] = (ts.ntc + 1) / 2;
     sb.nb[1] = (ts.ntr + 1) / 2;
     sb.nb[2] = (ts.ntd + 1) / 2;
     sb.n = sb.nb[0] * sb.nb[1] * sb.nb[2];
-    auto align = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t cells = size_t(g.B_rot) * size_t(sb.n);
-    const size_t counts = align(cells * sizeof(int)), lists = align(cells * size_t(g.P) * sizeof(unsigned short));
-    if (counts + lists > kBinsMaxBytes) return TP_OK;
-    if (g.B_rot * int64_t(sb.nb[1]) * sb.nb[2] * ((g.P + tp::kBinPoses - 1) / tp::kBinPoses) > tp::kBinMaxGroups)
+    size_t counts = align(cells * sizeof(int)), lists = align(cells * size_t(g.P) * sizeof(unsigned short));
+    if (g.P < kBinsMinPoses || g.P >= 65536 || counts + lists > kBinsMaxBytes ||
+        g.B_rot * int64_t(sb.nb[1]) * sb.nb[2] * ((g.P + tp::kBinPoses - 1) / tp::kBinPoses) > tp::kBinMaxGroups)
+        counts = lists = 0;
+    const size_t need = slots + counts + lists;
+    char* w = need ? static_cast<char*>(sc.bins(need, s)) : nullptr;
+    if (!w) {
+        ts.ssplit = tp::SplitView{};
+        sp.s[0] = tp::PoseSplit{};
         return TP_OK;
-    char* w = static_cast<char*>(sc.bins(counts + lists, s));
-    if (!w) return TP_OK;
-    sb.count = reinterpret_cast<int*>(w);
-    sb.list = reinterpret_cast<unsigned short*>(w + counts);
-    ts.sbins = sb;
+    }
+    ts.part = w;
+    if (counts) {
+        sb.count = reinterpret_cast<int*>(w + slots);
+        sb.list = reinterpret_cast<unsigned short*>(w + slots + counts);
+        ts.sbins = sb;
+    }
     return TP_OK;
 }
-// The bins' pre-pass, which also zeroes the core tiles' cells of dst and wdst (dst null: not; the
-// scatter then zeroes them itself).
-int fill_bins(bool cubic, const tp::Geom& g, tp::TileSpec& ts, const void* rot, void* dst, void* wdst,
-              CallScratch& sc, hipStream_t s) {
-    ts.core_zeroed = false;
+int fill_bins(bool cubic, const tp::Geom& g, const tp::TileSpec& ts, const void* rot, CallScratch& sc,
+              hipStream_t s) {
     if (!ts.sbins.list) return TP_OK;
     // a bin's box holds its tiles' box-1 boxes (the tile dilated by the stencil and the slack) with
     // half a voxel to spare
@@ -613,18 +683,29 @@ int fill_bins(bool cubic, const tp::Geom& g, tp::TileSpec& ts, const void* rot, 
     const tp::BinBox bb{{0.f, -half + 1.f, -half + 1.f},
                         {2.f * tp::kScTC, 2.f * tp::kScTR, 2.f * tp::kScTD},
                         sl + ts.eps + pad, sh + ts.eps + pad, ts.rho_unit + 1.0f};
-    TP_TRY(launched(tp::launch_pose_bins(g, rot, ts.sbins, bb, sc.p, s, ts, dst, wdst), "pose-bin launch"));
-    ts.core_zeroed = dst != nullptr;
-    return TP_OK;
+    return launched(tp::launch_pose_bins(g, rot, ts.sbins, bb, sc.p, s), "pose-bin launch");
 }
 
-// The rotation forward kernels' work items in reach (tp::TileSpec::flist), when the call's
-// (device, stream) area can hold them.
-int use_forw_list(const tp::Geom& g, tp::TileSpec& ts, CallScratch& sc, hipStream_t s) {
+// The forward kernels' splits, and the rotation kernels' work items in reach (tp::TileSpec::flist)
+// when the call's (device, stream) area can hold them.
+int use_forw_lists(const tp::Geom& g, tp::TileSpec& ts, Splits& sp, CallScratch& sc, hipStream_t s) {
     TP_TRY(sc.get(s));
+    uint32_t rho_bits = 0, eps_bits = 0;
+    std::memcpy(&rho_bits, &ts.rho_unit, 4);
+    std::memcpy(&eps_bits, &ts.eps, 4);
+    std::vector<int64_t> key{0, g.B, ts.nt, ts.org, ts.ntfd, ts.orgd, int64_t(rho_bits), int64_t(eps_bits)};
+    for (int l = 0; l < sp.f[0].n; ++l) {
+        const tp::PoseSplit::Level& v = sp.f[0].lv[l];
+        key.insert(key.end(), {v.lo[0], v.lo[1], v.lo[2], int64_t(v.ext), v.k});
+    }
+    ts.fsplit2 = split_view(sp.f2[0], sp.f2[1], g.B, sc, s);
+    ts.fsplit.pieces = sp.f[0].pieces;  // (the grid's item count, should the list have it)
     int64_t count = 0;
-    ts.flist = sc.forw_list(g, ts, s, count);
+    ts.flist = sc.item_list(key, s, count, [&](std::vector<tp::TileItem>& out) {
+        return tp::forw_reach_items(g, ts, sp.f[0], out) <= int64_t(INT32_MAX);
+    });
     ts.fcount = ts.flist ? count : 0;
+    if (!ts.flist) ts.fsplit = split_view(sp.f[1], sp.f[1], g.B, sc, s);
     return TP_OK;
 }
 
@@ -653,9 +734,10 @@ int project_forw(int dim, int dtype, const void* rec, int64_t B, int64_t D, int6
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool cubic = interp == TP_CUBIC;
     if (use_tiles(dim, dt, os, n)) {
-        tp::TileSpec ts = tile_spec(g, cubic, forw_poses_per_range(os));
+        Splits sp{};
+        tp::TileSpec ts = tile_spec(g, cubic, TileOp::project, sp);
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s));
-        TP_TRY(use_forw_list(g, ts, sc, s));
+        TP_TRY(use_forw_lists(g, ts, sp, sc, s));
         TP_TRY(launched(tp::launch_project3_forw_tiled(cubic, g, ts, rec, rot, shifts, out, sc.p, 0, s, rec_half),
                         "tiled projection launch"));
         return launched(tp::launch_project_forw(dim, kdt, cubic, g, rec, rot, shifts, out, s, true),
@@ -709,12 +791,13 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     TP_TRY(need(rot, "rotations"));
     CallScratch sc;
     if (tiles) {
-        tp::TileSpec ts = tile_spec(g, cubic);
-        TP_TRY(plan_bins(g, ts, sc, s));
+        Splits sp{};
+        tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, sp);
+        TP_TRY(plan_scatter(g, ts, sp, false, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, &ts));
-        TP_TRY(fill_bins(cubic, g, ts, rot, grec, nullptr, sc, s));
-        TP_TRY(use_forw_list(g, ts, sc, s));
-        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 1, g, ts, gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
+        TP_TRY(fill_bins(cubic, g, ts, rot, sc, s));
+        TP_TRY(use_forw_lists(g, ts, sp, sc, s));
+        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 1, g, ts, sp.s[0], gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
                                                   s),
                         "tiled reconstruction-gradient launch"));
         TP_TRY(launched(tp::launch_grads3_tiled(cubic, g, ts, gproj, rec, rot, shifts, grot, gshift, sc.p, 1, s,
@@ -764,12 +847,12 @@ int backproject_forw(int dim, int dtype, const void* proj, int64_t B, int64_t P,
     TP_TRY(need(rot, "rotations"));
     CallScratch sc;
     if (tiles) {
-        tp::TileSpec ts = tile_spec(g, cubic);
-        backprojection_ranges(g, ts);
-        TP_TRY(plan_bins(g, ts, sc, s));
+        Splits sp{};
+        tp::TileSpec ts = tile_spec(g, cubic, TileOp::backproject, sp);
+        TP_TRY(plan_scatter(g, ts, sp, weights != nullptr, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, &ts));
-        TP_TRY(fill_bins(cubic, g, ts, rot, data, weights ? wrec : nullptr, sc, s));
-        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 0, g, ts, proj, weights, rot, shifts, data, wrec, sc.p, 0, s),
+        TP_TRY(fill_bins(cubic, g, ts, rot, sc, s));
+        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 0, g, ts, sp.s[0], proj, weights, rot, shifts, data, wrec, sc.p, 0, s),
                         "tiled backprojection launch"));
     }
     if (tiles2) {
@@ -814,9 +897,10 @@ int backproject_back(int dim, int dtype, const void* gdata, const void* gw, int6
     }
     CallScratch sc;
     if (tiles) {
-        tp::TileSpec ts = tile_spec(g, cubic);
+        Splits sp{};
+        tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, sp);
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s));
-        TP_TRY(use_forw_list(g, ts, sc, s));
+        TP_TRY(use_forw_lists(g, ts, sp, sc, s));
         TP_TRY(launched(tp::launch_bpback3_tiled(cubic, g, ts, gdata, gw, proj, rot, shifts, gproj, gweights, grot,
                                                  gshift, sc.p, 0, s),
                         "tiled backprojection backward launch"));

@@ -63,17 +63,58 @@ struct BinBox {
     float org[3], edge[3];
     float lo_pad, hi_pad, reach;
 };
+
+// Pose ranges of a 3D tile grid.  Tiles near the origin are crossed by every pose, tiles at distance
+// x by about h / x of them (h a tile's half width), so the tiles within nested boxes around the origin
+// are split into pieces, more of them further in: level l (0 innermost) holds the tiles [lo, hi) along
+// d, r, c that no inner level holds, k pieces each.  Tiles outside every level are one piece.
+constexpr int kSplitLevels = 3;
+struct PoseSplit {
+    int n;  // levels in use
+    struct Level {
+        int lo[3];       // tile box along d, r, c: first tile
+        unsigned ext;    // and its extents, 10 bits each
+        int k;           // pieces per tile
+        int pieces;      // k times the box's tiles: work items of one batch item
+        __host__ __device__ int size(int a) const { return int(ext >> (10 * a)) & 1023; }
+        __host__ __device__ bool holds(int d, int r, int c) const {
+            return unsigned(d - lo[0]) < unsigned(size(0)) && unsigned(r - lo[1]) < unsigned(size(1)) &&
+                   unsigned(c - lo[2]) < unsigned(size(2));
+        }
+    } lv[kSplitLevels];  // (pieces 0 past the levels in use)
+    int pieces;          // of every level, for one batch item
+};
+// A work item of the rotation kernels' forward tile grid, decoded: piece j of k of tile (d, r, c) of
+// batch item b.
+struct alignas(16) TileItem {
+    unsigned short d, r, c, k;
+    int b, j;
+};
+static_assert(sizeof(TileItem) == 16, "one 16-byte load per workgroup");
+constexpr int kMaxTilePieces = 65535;
+// A split as the tile kernels see it: work items 0 .. B * pieces - 1 are the levels' pieces, listed in
+// device memory (level by level, batch item by batch item; the levels themselves in kernel arguments
+// cost the kernels 60 scalar registers), or without a list the pieces of one level, `box`.  Then come
+// the tiles of the whole grid, where those of `box`, the outermost level, are skipped.
+struct SplitView {
+    PoseSplit::Level box;
+    int pieces;
+    const TileItem* list;
+};
+
+// Bytes of one split tile's piece in the scatter's workspace.
+__host__ __device__ constexpr int64_t slot_bytes(bool weights) {
+    return int64_t(kScTC) * kScTR * kScTD * (weights ? 12 : 8);
+}
+
 struct TileSpec {
     int nt, org;              // forward: tiles along c and r, and the signed origin of the grid there,
                               // laid out for unit-scale poses (|x| <= rho_unit + 1)
-    int fc0, fc1;             // forward core tiles (split by pose range): [fc0, fc1) along c and r
-    int ntfd, orgd, fd0, fd1;  // forward: the same along d (tiles of kTileEdgeD)
+    int ntfd, orgd;           // forward: the same along d (tiles of kTileEdgeD)
     int nt2, org2, ntfd2, orgd2;  // forward: the grid that the other tiled poses reach (|x| <= rho)
-    int fc0_2, fc1_2, fd0_2, fd1_2;  // and its core tiles (the same voxels as fc0.. fd1)
+    SplitView fsplit, fsplit2;    // forward: pose ranges on the two grids
     int ntd, ntr, ntc;        // scatter: tiles along d, r, c of the stored half volume
-    int sd0, sd1, sr0, sr1, sc1;  // scatter core tiles: [sd0, sd1) x [sr0, sr1) x [0, sc1)
-    int ksplit, prange;       // pose ranges per core tile, poses per range (the scatters, GEN gathers)
-    int fksplit, fprange;     // the same for the rotation forward-family kernels (fc0.. fd1)
+    SplitView ssplit;         // scatter: pose ranges
     float rho;                // bound on |x| of every active sample of a tiled pose (singular values <= kScaleMax)
     float rho_unit;           // the same for singular values <= 1, less the +1 voxel margin
     float eps;                // slack (voxels) added to every enumeration box
@@ -89,15 +130,19 @@ struct TileSpec {
     // forward: the rotation kernels' work items whose tiles the rotations' samples can reach, in
     // work-item order (forw_reach_items), fcount of them; flist null: every work item of the grid
     // (about half of the headline's tiles lie outside that sphere)
-    const int* flist;
+    const TileItem* flist;
     int64_t fcount;
-    bool core_zeroed;         // scatter: the bin pre-pass has zeroed the core tiles' cells
+    // scatter: a slot of slot_bytes per piece of the split tiles (B * ssplit.pieces: the tile's values, then
+    // its weights), which k_finish3 sums into the volume
+    char* part;
 };
 
-// The work items of the rotation kernels' forward tile grid (ts's nt, ntfd, core tiles and
-// fksplit) whose tiles lie within rho_unit + 1 (and a margin) of the origin, in increasing order,
+// The pieces of split ps in work-item order, appended to `out` (k = 0: a tile that an inner level
+// holds, which the kernels skip).  Host code, for SplitView::list.
+void split_items(const PoseSplit& ps, int64_t B, std::vector<TileItem>& out);
+// The work items of the rotation kernels' forward tile grid (ts's nt, ntfd and split ps) whose tiles lie within rho_unit + 1 (and a margin) of the origin, in increasing order,
 // appended to `out`; returns the grid's item count.  Host code, for TileSpec::flist.
-int64_t forw_reach_items(const Geom& g, const TileSpec& ts, std::vector<int>& out);
+int64_t forw_reach_items(const Geom& g, const TileSpec& ts, const PoseSplit& ps, std::vector<TileItem>& out);
 
 // Tile-owner kernels of the fp32 2D operators (tp_tiled2d.hip).
 constexpr int kTile2C = 32, kTile2R = 16;  // scatter tile edges (c, r): fp64 accumulators
@@ -147,10 +192,9 @@ hipError_t launch_call_poses(int dim, int64_t poses, const void* rot, float rho_
 // Fill the pose bins bg (list and count allocated by the caller, the counts zeroed by
 // launch_call_poses, which has also filled *cp) of the scatter tile grid whose bin boxes bb
 // describes, for the B_rot * P poses at rot (bins beyond the reach of the call's tiled poses stay
-// empty, bb.reach being the rotations').  With dst, the same workgroups zero the scatter's core
-// tiles' cells of dst (and wdst) that ts describes, which the core pieces then add into.
+// empty, bb.reach being the rotations').
 hipError_t launch_pose_bins(const Geom& g, const void* rot, const BinGrid& bg, const BinBox& bb, const CallPoses* cp,
-                            hipStream_t s, const TileSpec& ts, void* dst, void* wdst);
+                            hipStream_t s);
 
 constexpr int kBlock = 256;
 constexpr int64_t kMaxGrid = int64_t(1) << 22;
@@ -202,7 +246,8 @@ hipError_t launch_bpback3_tiled(bool cubic, const Geom& g, const TileSpec& ts, c
                                 void* grot, void* gshift, CallPoses* cp, int gl, hipStream_t s);
 // mode 0: backprojection into data (+ weights), with the x = 0 Hermitian completion;
 // mode 1: reconstruction gradient of the projection.
-hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const void* src,
+// `ps`: the split of ts.ssplit.
+hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src,
                                  const void* weights, const void* rot, const void* shifts, void* dst, void* wdst,
                                  CallPoses* cp, int gl, hipStream_t s);
 

@@ -12,7 +12,7 @@
 // tile (one lane per (pose, row) computes the row's column interval, a wave
 // prefix sum packs the samples of several poses densely onto the lanes).
 // The tiles around the origin are crossed by nearly every pose; they are
-// split into pose ranges ("core" work items) that are dispatched first.
+// split into pieces of their poses (PoseSplit), which are dispatched first.
 //
 //   k_forw3_tiled     forward projection.  The tile plus its stencil halo is
 //                     staged in LDS holding exactly the value the reference's
@@ -26,10 +26,12 @@
 //                     accumulated in fp64 LDS (gfx950's LDS fp32 atomic add
 //                     runs at ~0.3 lanes/clk/CU, fp64 at ~7.7) and every
 //                     stored cell of the tile is written once with a plain
-//                     store: no zero fill and no global atomics, except for
-//                     the split core tiles, which add their partial tiles
-//                     into a zeroed region.  The Hermitian x = 0 mirror of
-//                     the backprojection is applied afterwards by k_mirror_x0.
+//                     store: no zero fill and no global atomics.  The pieces
+//                     of a split tile go to a workspace, and k_finish3 sums
+//                     them (with the Hermitian x = 0 mirror of the
+//                     backprojection): float atomics into a zeroed region
+//                     left 2 x 333 poses of 90 x 90 (cubic, oversampling 1.5,
+//                     eleven pieces) at 0.94 ms a step, the sums take it to 0.84.
 //
 // Poses whose first two matrix columns a, b have singular values in
 // [kScaleMin, kScaleMax] take this path (pose_tiled3); the per-pixel kernels
@@ -54,6 +56,7 @@
 //                sc >= 0 that can reach a box; the grid reaches samples up to
 //                kScaleMax times farther out.  Scatters add their tiles into
 //                the volume.
+#include <algorithm>
 #include <type_traits>
 
 #include "tp_device.hh"
@@ -254,46 +257,60 @@ __device__ __forceinline__ void load_pose(const float* __restrict__ rotb, const 
 constexpr int kRunForw = 64, kRunScatter = 128;  // measured at the headline
 constexpr int kForwFlatKP = 5;  // forward poses per wave batch for poses of up to 16 rows (about 11 rows each)
 
-// Work items: first the core tiles, one item per (batch, tile, pose range),
-// then every tile of every batch with all poses (core tiles skipped there).
+// Work items: the pieces of the split tiles (innermost level first, so that the longest items
+// start first), then every tile [0, n) of every batch item, offset by `off` (the split ones are
+// skipped there).  Axes are d, r, c.
 struct Item {
     int64_t b;
     int kd, kr, kc;
-    int p0, p1;
-    bool core, skip;
+    int j, k;   // piece j of k of the tile's poses
+    bool skip;  // a split tile
 };
-__device__ __forceinline__ Item item_of(int64_t w, int64_t B, int P, int nd, int nr, int nc, int d0, int d1, int r0,
-                                        int r1, int c0, int c1, int ksplit, int prange) {
+__device__ __forceinline__ Item listed_item(const TileItem* __restrict__ list, int64_t w) {
+    const TileItem f = list[w];
+    return Item{f.b, f.d, f.r, f.c, f.j, f.k, f.k == 0};
+}
+__device__ __forceinline__ Item item_of(int64_t w, int64_t B, int nd, int nr, int nc, int offd, int off,
+                                        const SplitView& sp) {
     Item it;
-    const int cd = d1 - d0, cr = r1 - r0, cc = c1 - c0;
-    const int64_t ncore = int64_t(cd) * cr * cc * ksplit;
-    it.skip = false;
-    if (w < B * ncore) {
-        it.core = true;
-        it.b = w / ncore;
-        int64_t q = w - it.b * ncore;
-        const int j = int(q % ksplit);
-        q /= ksplit;
-        it.kc = c0 + int(q % cc);
-        it.kr = r0 + int((q / cc) % cr);
-        it.kd = d0 + int(q / (int64_t(cc) * cr));
-        it.p0 = j * prange;
-        it.p1 = min(P, it.p0 + prange);
+    const int64_t split = B * sp.pieces;
+    const PoseSplit::Level& v = sp.box;
+    if (w < split) {
+        if (sp.list) return listed_item(sp.list, w);
+        it.b = w / sp.pieces;
+        const int q = int(w - it.b * sp.pieces), t = q / v.k, nc_ = v.size(2), nr_ = v.size(1);
+        it.j = q - t * v.k;
+        it.k = v.k;
+        it.kc = v.lo[2] + t % nc_;
+        it.kr = v.lo[1] + (t / nc_) % nr_;
+        it.kd = v.lo[0] + t / (nc_ * nr_);
+        it.skip = false;
     } else {
-        it.core = false;
         const int64_t per_b = int64_t(nd) * nr * nc;
-        const int64_t q = w - B * ncore;
-        it.b = q / per_b;
-        const int t = int(q - it.b * per_b);
-        it.kc = t % nc;
-        it.kr = (t / nc) % nr;
-        it.kd = t / (nc * nr);
-        it.p0 = 0;
-        it.p1 = P;
-        it.skip = ksplit > 1 && it.kd >= d0 && it.kd < d1 && it.kr >= r0 && it.kr < r1 && it.kc >= c0 && it.kc < c1;
+        w -= split;
+        it.b = w / per_b;
+        const int t = int(w - it.b * per_b);
+        it.kc = off + t % nc;
+        it.kr = off + (t / nc) % nr;
+        it.kd = offd + t / (nc * nr);
+        it.j = 0;
+        it.k = 1;
+        it.skip = v.holds(it.kd, it.kr, it.kc);
     }
     return it;
 }
+// The same in scalar registers (every lane holds the same item; a listed one comes by a vector load).
+__device__ __forceinline__ Item uniform(Item it) {
+    it.kd = __builtin_amdgcn_readfirstlane(it.kd);
+    it.kr = __builtin_amdgcn_readfirstlane(it.kr);
+    it.kc = __builtin_amdgcn_readfirstlane(it.kc);
+    it.j = __builtin_amdgcn_readfirstlane(it.j);
+    it.k = __builtin_amdgcn_readfirstlane(it.k);
+    it.b = __builtin_amdgcn_readfirstlane(int(it.b));
+    return it;
+}
+// Start of piece j of k of n poses.
+__device__ __forceinline__ int piece_at(int n, int j, int k) { return int(unsigned(n) / unsigned(k)) * j + min(j, int(unsigned(n) % unsigned(k))); }
 
 // Poses culled per phase: each lane tests kChunk / NT of them, the survivors'
 // indices (relative to the phase) go to an LDS list.
@@ -429,12 +446,10 @@ __device__ __forceinline__ void cull_chunk_boxes(const float* __restrict__ rotb,
     n2 = pcnt[1];
 }
 
-// Pose bin of scatter tile (kc, kr, kd) in the grid with bins bg (tiles outside the core): its list
-// and count for rotation batch item rb, or lst = nullptr when there are no bins.
+// Pose bin of scatter tile (kc, kr, kd) in the grid with bins bg: its list
+// and count for rotation batch item rb (unchanged when there are no bins).
 __device__ __forceinline__ void tile_bin(const BinGrid& bg, int64_t rb, int64_t P, int kc, int kr, int kd,
                                          const unsigned short*& lst, int& cnt) {
-    lst = nullptr;
-    cnt = 0;
     if (!bg.list) return;
     const int64_t bi = rb * bg.n + (int64_t(kd >> 1) * bg.nb[1] + (kr >> 1)) * bg.nb[0] + (kc >> 1);
     lst = bg.list + bi * P;
@@ -611,28 +626,24 @@ __attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>())))
     const bool all_rot = !GEN && call_flag(&cp->all_rot);
     float rho_k = ts.rho_unit + 1.0f;
     int nt = ts.nt, ntd = ts.ntfd, org = ts.org, orgd = ts.orgd;
-    int fc0 = ts.fc0, fc1 = ts.fc1, fd0 = ts.fd0, fd1 = ts.fd1;
+    const SplitView& ps = GEN ? ts.fsplit2 : ts.fsplit;
+    int off = 0, offd = 0;  // first tile of the part of the wide grid that the reach needs
     if constexpr (GEN) {
         rho_k = fminf(ts.rho, cp->gen_reach);
         if (!(rho_k > 0.f)) return;  // no such pose in this call
         const int h = half_tiles_for(rho_k, L, ts.nt2 / 2), hd = half_tiles_for(rho_k, LD, ts.ntfd2 / 2);
-        const int off = ts.nt2 / 2 - h, offd = ts.ntfd2 / 2 - hd;
+        off = ts.nt2 / 2 - h;
+        offd = ts.ntfd2 / 2 - hd;
         nt = 2 * h;
         ntd = 2 * hd;
-        org = ts.org2 + off * L;
-        orgd = ts.orgd2 + offd * LD;
-        fc0 = min(nt, max(0, ts.fc0_2 - off));
-        fc1 = min(nt, max(fc0, ts.fc1_2 - off));
-        fd0 = min(ntd, max(0, ts.fd0_2 - offd));
-        fd1 = min(ntd, max(fd0, ts.fd1_2 - offd));
+        org = ts.org2;
+        orgd = ts.orgd2;
     }
     const float rho2 = rho_k * rho_k;
-    // core tiles in pose ranges: the rotation kernels' split, or the other poses' (the scatter's)
-    const int ksplit = GEN ? ts.ksplit : ts.fksplit, prange = GEN ? ts.prange : ts.fprange;
-    int64_t items = g.B * (int64_t(fc1 - fc0) * (fc1 - fc0) * (fd1 - fd0) * ksplit + int64_t(nt) * nt * ntd);
+    int64_t items = g.B * (ps.pieces + int64_t(nt) * nt * ntd);
     // rotations: the slots may index the list of the work items in reach (the others' workgroups
     // would only start and leave)
-    const int* __restrict__ flist = GEN ? nullptr : ts.flist;
+    const TileItem* __restrict__ flist = GEN ? nullptr : ts.flist;
     if (flist) items = ts.fcount;
     const float cut2 = float(g.cut2);
     const int N = g.N, H = g.H;
@@ -642,12 +653,11 @@ __attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>())))
         const int64_t slot_i = sl.s;
         const int64_t wi = xcd_item<kRunForw>(slot_i);
         if (wi >= items) continue;
-        const int64_t w = flist ? int64_t(flist[wi]) : wi;
-        const Item it = item_of(w, g.B, int(g.P), ntd, nt, nt, fd0, fd1, fc0, fc1, fc0, fc1, ksplit, prange);
+        const Item it = uniform(flist ? listed_item(flist, wi) : item_of(wi, g.B, ntd, nt, nt, offd, off, ps));
         if (it.skip) continue;
         const int64_t b = it.b;
         const int tc = org + it.kc * L, tr = org + it.kr * L, td = orgd + it.kd * LD;
-        const int p0 = it.p0, p1 = it.p1;
+        const int p0 = piece_at(int(g.P), it.j, it.k), p1 = piece_at(int(g.P), it.j + 1, it.k);
         // samples owned by this tile: floor(x) in [t, t + edge) on every axis (+ slack)
         const float lo[3] = {float(tc) - ts.eps, float(tr) - ts.eps, float(td) - ts.eps};
         const float hi[3] = {float(tc + L) + ts.eps, float(tr + L) + ts.eps, float(td + LD) + ts.eps};
@@ -1077,8 +1087,7 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool pose_lane = lane < KP;  // lane k holds pose k of the wave's batch
     const int N = g.N, H = g.H, half = N / 2;
-    const int64_t items = g.B * (int64_t(ts.sd1 - ts.sd0) * (ts.sr1 - ts.sr0) * ts.sc1 * ts.ksplit +
-                                 int64_t(ts.ntd) * ts.ntr * ts.ntc);
+    const int64_t items = g.B * (ts.ssplit.pieces + int64_t(ts.ntd) * ts.ntr * ts.ntc);
     const float cut2 = float(g.cut2);
     // samples lie within |x| <= rho_k: rotations reach rho_unit + 1, GEN poses the call's own
     // reach (up to kScaleMax times farther).  Without rotations in the call the rotation kernel
@@ -1095,9 +1104,9 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
         const int64_t slot_i = sl.s;
         const int64_t w = xcd_item<kRunScatter>(slot_i);
         if (w >= items) continue;
-        const Item it = item_of(w, g.B, int(g.P), ts.ntd, ts.ntr, ts.ntc, ts.sd0, ts.sd1, ts.sr0, ts.sr1, 0, ts.sc1,
-                                ts.ksplit, ts.prange);
+        const Item it = uniform(item_of(w, g.B, ts.ntd, ts.ntr, ts.ntc, 0, 0, ts.ssplit));
         if (it.skip) continue;
+        const bool split = w < g.B * ts.ssplit.pieces;  // a piece, whose slot of the workspace is w
         const int64_t b = it.b;
         // stored cells of this tile, signed coordinates: d, r in [-N/2+1, N/2], c in [0, N/2]
         const int tc = it.kc * SC, tr = -half + 1 + it.kr * SR, td = -half + 1 + it.kd * SD;
@@ -1122,10 +1131,9 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
             dist2 += q * q;
         }
         // (a rotation kernel without rotations in the call only stores zeros)
-        const int pend = (dist2 > rho_k * rho_k || (!GEN && !any_rot)) ? it.p0 : it.p1;
         // a tile that no pose can reach stores zeros without its accumulators (about half of the
         // tiles of a volume lie beyond the samples' sphere)
-        const bool empty = pend == it.p0;
+        const bool empty = dist2 > rho_k * rho_k || (!GEN && !any_rot);
         if (!empty)
             for (int e = tid; e < S3; e += NT) {
                 acc_re[e] = 0.0;
@@ -1135,11 +1143,12 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
 
         const float* shb = shifts ? shifts + sb * g.P * 2 : nullptr;
         bool touched = false;  // GEN: some pose reaches the tile
-        // candidates: the tile's pose range, or (outside the core) its bin's poses
+        // candidates: a split tile's piece of all poses (all pieces j run at about the same time, on the
+        // same poses' projections), or the poses of the tile's bin
         const unsigned short* lst = nullptr;
-        int lcnt = 0;
-        if (!it.core && pend > it.p0) tile_bin(ts.sbins, rb, g.P, it.kc, it.kr, it.kd, lst, lcnt);
-        const int c_begin = lst ? 0 : it.p0, c_end = lst ? lcnt : pend;
+        int lcnt = int(g.P);
+        if (!empty && !split) tile_bin(ts.sbins, rb, g.P, it.kc, it.kr, it.kd, lst, lcnt);
+        const int c_begin = empty ? 0 : piece_at(lcnt, it.j, it.k), c_end = empty ? 0 : piece_at(lcnt, it.j + 1, it.k);
         for (int pbase = c_begin; pbase < c_end; pbase += kChunkSc) {
             int n1, n2;
             cull_chunk_boxes<NT, GEN>(rotb, c_end, pbase, lo1, hi1, lo2, hi2, plist, pcnt, n1, n2, all_rot, lst);
@@ -1345,38 +1354,41 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
             __syncthreads();
         }
 
-        // write every stored cell of the tile once (core pieces add into a zeroed region).  GEN
-        // adds onto what the rotation kernel wrote: core pieces with atomics, the other tiles (one
-        // workgroup each) by a plain read and write; without rotations in the call it stores them
-        if (GEN && !touched && (it.core || any_rot)) continue;
-        if (empty && it.core) continue;  // (adds nothing)
+        // write every stored cell of the tile once: a piece of a split tile into its slot of the
+        // workspace (k_finish3 sums them), other tiles into the volume.  GEN adds onto what the
+        // rotation kernel wrote (one workgroup each, so by a plain read and write); without
+        // rotations in the call it stores.
+        const bool onto = GEN && any_rot && (!split || dist2 <= (ts.rho_unit + 1.0f) * (ts.rho_unit + 1.0f));
+        if (GEN && any_rot && !touched && (onto || empty)) continue;
+        if (empty && split) continue;  // (k_finish3 reads no piece of a tile beyond every reach)
         __syncthreads();
         {
             // each lane keeps one (c, r) of the tile and steps along d
             static_assert(NT % (SC * SR) == 0, "write-out lanes keep their column and row");
             const int lc = tid % SC, lr = (tid / SC) % SR;
             const int c = tc + lc, r = tr + lr;
-            if (c < H && r <= half) {
-                const int64_t row = b * g.vol + int64_t(r < 0 ? r + N : r) * H + c, plane = int64_t(N) * H;
-                for (int ld = tid / (SC * SR); ld < SD; ld += NT / (SC * SR)) {
-                    const int d = td + ld;
-                    if (d > half) break;
-                    const int64_t idx = row + (d < 0 ? d + N : d) * plane;
+            if (split || (c < H && r <= half)) {
+                // (a slot: the tile's values, then its weights)
+                char* const slot = ts.part + xcd_item<kRunScatter>(sl.s) * slot_bytes(WEIGHTS);
+                Cx<float>* const out = split ? reinterpret_cast<Cx<float>*>(slot) : dst;
+                float* const wout = split ? reinterpret_cast<float*>(slot + S3 * 8) : wdst;
+                const int64_t row = split ? lr * SC + lc : b * g.vol + int64_t(r < 0 ? r + N : r) * H + c;
+                const int plane = split ? SR * SC : N * H;
+                const int last = split ? SD - 1 : min(SD - 1, half - td);
+                for (int ld = tid / (SC * SR); ld <= last; ld += NT / (SC * SR)) {
+                    const int d = split ? ld : td + ld;
+                    const int64_t idx = row + int64_t(d < 0 ? d + N : d) * plane;
                     const int a = (ld * SR + lr) * SC + ((lc + acc_swizzle(lr, ld)) & (SC - 1));
-                    if (it.core) {
-                        atomic_add(&dst[idx].re, float(acc_re[a]));
-                        atomic_add(&dst[idx].im, float(acc_im[a]));
-                        if (WEIGHTS) atomic_add(&wdst[idx], float(acc_w[a]));
-                    } else if (GEN && any_rot) {
-                        const Cx<float> o = dst[idx];
-                        dst[idx] = Cx<float>{o.re + float(acc_re[a]), o.im + float(acc_im[a])};
-                        if (WEIGHTS) wdst[idx] += float(acc_w[a]);
+                    if (onto) {
+                        const Cx<float> o = out[idx];
+                        out[idx] = Cx<float>{o.re + float(acc_re[a]), o.im + float(acc_im[a])};
+                        if (WEIGHTS) wout[idx] += float(acc_w[a]);
                     } else if (empty) {
-                        dst[idx] = Cx<float>{0.f, 0.f};
-                        if (WEIGHTS) wdst[idx] = 0.f;
+                        out[idx] = Cx<float>{0.f, 0.f};
+                        if (WEIGHTS) wout[idx] = 0.f;
                     } else {
-                        dst[idx] = Cx<float>{float(acc_re[a]), float(acc_im[a])};
-                        if (WEIGHTS) wdst[idx] = float(acc_w[a]);
+                        out[idx] = Cx<float>{float(acc_re[a]), float(acc_im[a])};
+                        if (WEIGHTS) wout[idx] = float(acc_w[a]);
                     }
                 }
             }
@@ -1385,60 +1397,135 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
     }
 }
 
-// Hermitian completion of the x = 0 plane after an unmirrored accumulation:
-// every x = 0 contribution v of the reference is also added, conjugated, at
-// the partner cell (-d, -r) (projection_utils.h:481-492), so the final value
-// of a cell is A(X) + conj(A(mirror X)) (weights: A_w(X) + A_w(mirror X)).
-// One lane per unordered pair {X, mirror X}; self-partnered cells are kept.
-template <bool WEIGHTS>
-__global__ __launch_bounds__(kBlock) void k_mirror_x0(Geom g, Cx<float>* __restrict__ dst,
-                                                      float* __restrict__ wdst) {
-    const int N = g.N, H = g.H;
-    const int64_t plane = int64_t(N) * N;
-    for (int64_t e = int64_t(blockIdx.x) * kBlock + threadIdx.x; e < g.B * plane;
-         e += int64_t(gridDim.x) * kBlock) {
-        const int64_t b = e / plane;
-        const int q = int(e - b * plane);
-        const int de = q / N, re = q - de * N;
-        const int dm = de == 0 ? 0 : N - de, rm = re == 0 ? 0 : N - re;
-        const int qm = dm * N + rm;
-        if (qm <= q) continue;  // self-partnered, or handled by the partner's lane
-        const int64_t i0 = b * g.vol + int64_t(q) * H, i1 = b * g.vol + int64_t(qm) * H;
-        const Cx<float> a = dst[i0], m = dst[i1];
-        dst[i0] = Cx<float>{a.re + m.re, a.im - m.im};
-        dst[i1] = Cx<float>{m.re + a.re, m.im - a.im};
-        if (WEIGHTS) {
-            const float wa = wdst[i0], wm = wdst[i1];
-            wdst[i0] = wa + wm;
-            wdst[i1] = wm + wa;
+// Sum of the pieces of a split tile's cell (their slots of the workspace), fp64; or, for a tile of
+// one piece, the cell as the scatter stored it.
+template <bool CUBIC, bool WEIGHTS>
+__device__ __forceinline__ void cell_sum(const Geom& g, const TileSpec& ts, const PoseSplit& ps, float reach, int64_t b, int d, int r, int c,
+                                         const Cx<float>* dst, const float* wdst, int64_t idx, double& vr, double& vi,
+                                         double& vw) {
+    const int half = g.N / 2;
+    const int kd = (d + half - 1) / SD, kr = (r + half - 1) / SR, kc = c / SC;
+    const int e = ((d + half - 1 - kd * SD) * SR + (r + half - 1 - kr * SR)) * SC + (c - kc * SC);
+    int64_t first = 0, at = 0;
+    int k = 0;
+    if (!ts.ssplit.box.holds(kd, kr, kc)) {
+        vr = double(dst[idx].re);
+        vi = double(dst[idx].im);
+        vw = WEIGHTS ? double(wdst[idx]) : 0.0;
+        return;
+    }
+#pragma unroll
+    for (int l = 0; l < kSplitLevels; ++l) {
+        const PoseSplit::Level& v = ps.lv[l];
+        if (k == 0 && v.holds(kd, kr, kc)) {
+            k = v.k;
+            const int t = ((kd - v.lo[0]) * v.size(1) + (kr - v.lo[1])) * v.size(2) + (kc - v.lo[2]);
+            at = first + b * v.pieces + int64_t(t) * v.k;
         }
+        first += g.B * int64_t(v.pieces);
+    }
+    // a split tile beyond the reach of the call's poses: its pieces stored nothing
+    {
+        const int t3[3] = {kc * SC, kr * SR - half + 1, kd * SD - half + 1}, s3[3] = {SC, SR, SD};
+        constexpr int SL = CUBIC ? 2 : 1, SH = CUBIC ? 1 : 0;
+        float dist2 = 0.f;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float lo = float(t3[a] - SL) - ts.eps, hi = float(t3[a] + s3[a] + SH) + ts.eps;
+            const float q = lo > 0.f ? lo : (hi < 0.f ? -hi : 0.f);
+            dist2 += q * q;
+        }
+        if (!(reach > 0.f) || dist2 > reach * reach) {
+            vr = vi = vw = 0.0;
+            return;
+        }
+    }
+    vr = vi = vw = 0.0;
+    const char* slot = ts.part + at * slot_bytes(WEIGHTS);
+#pragma unroll 4
+    for (int j = 0; j < k; ++j, slot += slot_bytes(WEIGHTS)) {
+        const Cx<float> v = reinterpret_cast<const Cx<float>*>(slot)[e];
+        vr += double(v.re);
+        vi += double(v.im);
+        if (WEIGHTS) vw += double(reinterpret_cast<const float*>(slot + S3 * 8)[e]);
     }
 }
 
-// Zero the stored cells of the scatter core tiles, which their pose-range
-// pieces then accumulate into with atomics: cells e0, e0 + step, ... (wdst may be null).
-__device__ __forceinline__ void zero_core_cells(const Geom& g, const TileSpec& ts, Cx<float>* __restrict__ dst,
-                                                float* __restrict__ wdst, int64_t e0, int64_t step) {
+// Completion of the 3D scatter, after both scatter kernels: the workgroups below `red` sum the pieces
+// of the split tiles' cells into the volume (kFinishParts per batch item and tile of the outermost
+// level's box); with MIRROR the others apply the Hermitian completion of the x = 0 plane (and store its split
+// cells, which the first leave to them):
+// every x = 0 contribution v of the reference is also added, conjugated, at
+// the partner cell (-d, -r) (projection_utils.h:481-492), so the final value
+// of a cell is A(X) + conj(A(mirror X)) (weights: A_w(X) + A_w(mirror X)).
+// One lane per unordered pair {X, mirror X}; self-partnered cells keep their value.
+constexpr int kFinishParts = 6;  // workgroups per split tile (one cell a lane: the sums wait for their loads)
+static_assert(S3 % (kFinishParts * kBlock) == 0, "whole workgroups per part");
+template <bool CUBIC, bool WEIGHTS, bool MIRROR>
+__global__ __launch_bounds__(kBlock) void k_finish3(Geom g, TileSpec ts, PoseSplit ps, int64_t red,
+                                                    Cx<float>* __restrict__ dst, float* __restrict__ wdst,
+                                                    const CallPoses* __restrict__ cp) {
     const int N = g.N, H = g.H, half = N / 2;
-    const int dd = (ts.sd1 - ts.sd0) * SD, rr = (ts.sr1 - ts.sr0) * SR, cc = ts.sc1 * SC;
-    const int64_t cells = int64_t(dd) * rr * cc;
-    for (int64_t e = e0; e < g.B * cells; e += step) {
-        const int64_t b = e / cells;
-        const int64_t q = e - b * cells;
-        const int c = int(q % cc), r = -half + 1 + ts.sr0 * SR + int((q / cc) % rr),
-                  d = -half + 1 + ts.sd0 * SD + int(q / (int64_t(cc) * rr));
-        if (c >= H || r > half || d > half) continue;
-        const int re = r < 0 ? r + N : r, de = d < 0 ? d + N : d;
-        const int64_t idx = b * g.vol + (int64_t(de) * N + re) * H + c;
-        dst[idx] = Cx<float>{0.f, 0.f};
-        if (wdst) wdst[idx] = 0.f;
+    const float reach = fmaxf(cp->any_rot ? ts.rho_unit + 1.0f : 0.f, fminf(ts.rho, cp->gen_reach));
+    if (int64_t(blockIdx.x) < red) {
+        const PoseSplit::Level& v = ts.ssplit.box;
+        const int nc = v.size(2), nr = v.size(1);
+        const int64_t per_b = int64_t(v.size(0)) * nr * nc;
+        const int64_t tile = blockIdx.x / kFinishParts, b = tile / per_b;
+        const int part = int(blockIdx.x - tile * kFinishParts), t = int(tile - b * per_b);
+        const int tc = (v.lo[2] + t % nc) * SC, tr = -half + 1 + (v.lo[1] + (t / nc) % nr) * SR,
+                  td = -half + 1 + (v.lo[0] + t / (nc * nr)) * SD;
+        for (int e = part * (S3 / kFinishParts) + threadIdx.x; e < (part + 1) * (S3 / kFinishParts); e += kBlock) {
+            const int c = tc + e % SC, r = tr + (e / SC) % SR, d = td + e / (SC * SR);
+            if (c >= H || r > half || d > half || (MIRROR && c == 0)) continue;
+            const int64_t idx = b * g.vol + (int64_t(d < 0 ? d + N : d) * N + (r < 0 ? r + N : r)) * H + c;
+            double vr, vi, vw;
+            cell_sum<CUBIC, WEIGHTS>(g, ts, ps, reach, b, d, r, c, dst, wdst, idx, vr, vi, vw);
+            dst[idx] = Cx<float>{float(vr), float(vi)};
+            if (WEIGHTS) wdst[idx] = float(vw);
+        }
+        return;
     }
-}
-template <bool WEIGHTS>
-__global__ __launch_bounds__(kBlock) void k_zero_core(Geom g, TileSpec ts, Cx<float>* __restrict__ dst,
-                                                      float* __restrict__ wdst) {
-    zero_core_cells(g, ts, dst, WEIGHTS ? wdst : nullptr, int64_t(blockIdx.x) * kBlock + threadIdx.x,
-                    int64_t(gridDim.x) * kBlock);
+    if constexpr (MIRROR) {
+        const int64_t plane = int64_t(N) * N;
+        for (int64_t e = (int64_t(blockIdx.x) - red) * kBlock + threadIdx.x; e < g.B * plane;
+             e += (int64_t(gridDim.x) - red) * kBlock) {
+            const int64_t b = e / plane;
+            const int q = int(e - b * plane);
+            const int de = q / N, re = q - de * N;
+            const int dm = de == 0 ? 0 : N - de, rm = re == 0 ? 0 : N - re;
+            const int qm = dm * N + rm;
+            if (qm < q) continue;  // handled by the partner's lane
+            auto sg = [&](int i) { return i <= half ? i : i - N; };
+            const int64_t i0 = b * g.vol + int64_t(q) * H, i1 = b * g.vol + int64_t(qm) * H;
+            auto unsplit = [&](int d, int r) {
+                return !ts.ssplit.box.holds((d + half - 1) / SD, (r + half - 1) / SR, 0);
+            };
+            if (unsplit(sg(de), sg(re)) && unsplit(sg(dm), sg(rm))) {  // most of the plane
+                if (qm == q) continue;
+                const Cx<float> a = dst[i0], m = dst[i1];
+                dst[i0] = Cx<float>{a.re + m.re, a.im - m.im};
+                dst[i1] = Cx<float>{m.re + a.re, m.im - a.im};
+                if (WEIGHTS) {
+                    const float wa = wdst[i0], wm = wdst[i1];
+                    wdst[i0] = wa + wm;
+                    wdst[i1] = wm + wa;
+                }
+                continue;
+            }
+            double ar, ai, aw, mr, mi, mw;
+            cell_sum<CUBIC, WEIGHTS>(g, ts, ps, reach, b, sg(de), sg(re), 0, dst, wdst, i0, ar, ai, aw);
+            if (qm == q) {  // self-partnered
+                dst[i0] = Cx<float>{float(ar), float(ai)};
+                if (WEIGHTS) wdst[i0] = float(aw);
+                continue;
+            }
+            cell_sum<CUBIC, WEIGHTS>(g, ts, ps, reach, b, sg(dm), sg(rm), 0, dst, wdst, i1, mr, mi, mw);
+            dst[i0] = Cx<float>{float(ar + mr), float(ai - mi)};
+            dst[i1] = Cx<float>{float(mr + ar), float(mi - ai)};
+            if (WEIGHTS) wdst[i0] = wdst[i1] = float(aw + mw);
+        }
+    }
 }
 
 // Pose bins (launch_pose_bins): one workgroup per rotation batch item, row of bins along c (bins
@@ -1449,15 +1536,11 @@ __global__ __launch_bounds__(kBlock) void k_zero_core(Geom g, TileSpec ts, Cx<fl
 // per-tile lists that are unordered anyway).  A bin box holds every tile box of its 2 x 2 x 2 tiles
 // with half a voxel to spare on each side, far beyond the rounding of either plane test, so a pose
 // that crosses a tile's box is in its bin.  The counts start at zero (the pose pre-pass clears
-// them).  With dst, the workgroups first zero the scatter's core cells (zero_core_cells).
+// them).
 constexpr int kBinThreads = 256, kBinPer = kBinPoses / kBinThreads;
 static_assert(kBinPer * kBinThreads == kBinPoses, "bin pre-pass shape");
 __global__ __launch_bounds__(kBinThreads) void k_pose_bins(Geom g, const float* __restrict__ rot, BinGrid bg,
-                                                           BinBox bb, const CallPoses* __restrict__ cp, TileSpec ts,
-                                                           Cx<float>* __restrict__ dst, float* __restrict__ wdst) {
-    if (dst)
-        zero_core_cells(g, ts, dst, wdst, int64_t(blockIdx.x) * kBinThreads + threadIdx.x,
-                        int64_t(gridDim.x) * kBinThreads);
+                                                           BinBox bb, const CallPoses* __restrict__ cp) {
     const int lane = threadIdx.x & 63;
     const int nrow = bg.nb[1] * bg.nb[2];
     const int64_t blocks = (g.P + kBinPoses - 1) / kBinPoses;
@@ -1546,8 +1629,7 @@ __global__ __launch_bounds__(kBinThreads) void k_pose_bins(Geom g, const float* 
 
 // Work items of the rotation kernels' forward tile grid (the unit grid).
 int64_t forw_items(const Geom& g, const TileSpec& ts) {
-    const int fc = ts.fc1 - ts.fc0, fd = ts.fd1 - ts.fd0;
-    return g.B * (int64_t(fc) * fc * fd * ts.fksplit + int64_t(ts.nt) * ts.nt * ts.ntfd);
+    return g.B * (ts.fsplit.pieces + int64_t(ts.nt) * ts.nt * ts.ntfd);
 }
 // Workgroups of a launch of `kernel` over `items`: one per item (rotations), or the persistent
 // GEN grid (the scatter's).
@@ -1594,21 +1676,11 @@ hipError_t forw_both(const Geom& g, const TileSpec& ts, const void* rec, const v
 }
 
 template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool OSX>
-hipError_t scatter_launch(const Geom& g, const TileSpec& ts, const void* src, const void* weights, const void* rot,
+hipError_t scatter_launch(const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src, const void* weights, const void* rot,
                           const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
-    const int64_t score = int64_t(ts.sd1 - ts.sd0) * (ts.sr1 - ts.sr0) * ts.sc1 * ts.ksplit;
-    if (score > 0 && !ts.core_zeroed) {
-        const int64_t cells = g.B * int64_t((ts.sd1 - ts.sd0) * SD) * ((ts.sr1 - ts.sr0) * SR) * (ts.sc1 * SC);
-        int64_t blocks = (cells + kBlock - 1) / kBlock;
-        if (blocks > 65536) blocks = 65536;
-        hipLaunchKernelGGL(k_zero_core<WEIGHTS>, dim3(unsigned(blocks)), dim3(kBlock), 0, s, g, ts, (Cx<float>*)dst,
-                           (float*)wdst);
-        const hipError_t ez = hipGetLastError();
-        if (ez != hipSuccess) return ez;
-    }
     // rotations write every tile (none: the other tiled poses store them); the other tiled
     // poses add onto them
-    const int64_t work = g.B * (score + int64_t(ts.ntd) * ts.ntr * ts.ntc);
+    const int64_t work = g.B * (ts.ssplit.pieces + int64_t(ts.ntd) * ts.ntr * ts.ntc);
     const auto kr = k_scatter3_tiled<CUBIC, MODE, WEIGHTS, KP, OSX, false>;
     const auto kg = k_scatter3_tiled<CUBIC, MODE, WEIGHTS, KP, OSX, true>;
     hipLaunchKernelGGL(kr, dim3(grid_of<false, kRunScatter>(work, (const void*)kr, kScatterThreads)),
@@ -1622,36 +1694,38 @@ hipError_t scatter_launch(const Geom& g, const TileSpec& ts, const void* src, co
                        (const Cx<float>*)src, (const float*)weights, (const float*)rot, (const float*)shifts,
                        (Cx<float>*)dst, (float*)wdst, cp, gl);
     e = hipGetLastError();
-    if (e != hipSuccess || MODE != 0) return e;
-    const int64_t pairs = g.B * int64_t(g.N) * g.N;
-    int64_t blocks = (pairs + kBlock - 1) / kBlock;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(k_mirror_x0<WEIGHTS>, dim3(unsigned(blocks)), dim3(kBlock), 0, s, g, (Cx<float>*)dst,
-                       (float*)wdst);
+    if (e != hipSuccess) return e;
+    const PoseSplit::Level& outer = ts.ssplit.box;
+    const int64_t red = kFinishParts * g.B * int64_t(outer.size(0)) * outer.size(1) * outer.size(2);
+    int64_t blocks = 0;
+    if (MODE == 0) blocks = std::min<int64_t>(65536, (g.B * int64_t(g.N) * g.N + kBlock - 1) / kBlock);
+    if (red + blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_finish3<CUBIC, WEIGHTS, MODE == 0>), dim3(unsigned(red + blocks)), dim3(kBlock), 0, s, g, ts, ps, red,
+                       (Cx<float>*)dst, (float*)wdst, cp);
     return hipGetLastError();
 }
 
 template <bool CUBIC, int MODE, bool WEIGHTS, bool OSX>
-hipError_t scatter_kp_osx(const Geom& g, const TileSpec& ts, const void* src, const void* weights, const void* rot,
+hipError_t scatter_kp_osx(const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src, const void* weights, const void* rot,
                           const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
     // (the cubic stencil carries windows across batches and keeps two pose sets: at most 4 poses)
     if constexpr (!CUBIC)
         if (ts.kp_scatter >= 6)
-            return scatter_launch<CUBIC, MODE, WEIGHTS, 6, OSX>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl,
+            return scatter_launch<CUBIC, MODE, WEIGHTS, 6, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl,
                                                                 s);
     if (ts.kp_scatter >= 4)
-        return scatter_launch<CUBIC, MODE, WEIGHTS, 4, OSX>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return scatter_launch<CUBIC, MODE, WEIGHTS, 4, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
     if (ts.kp_scatter >= 3)
-        return scatter_launch<CUBIC, MODE, WEIGHTS, 3, OSX>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
-    return scatter_launch<CUBIC, MODE, WEIGHTS, 1, OSX>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return scatter_launch<CUBIC, MODE, WEIGHTS, 3, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+    return scatter_launch<CUBIC, MODE, WEIGHTS, 1, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
 }
 
 template <bool CUBIC, int MODE, bool WEIGHTS>
-hipError_t scatter_kp(const Geom& g, const TileSpec& ts, const void* src, const void* weights, const void* rot,
+hipError_t scatter_kp(const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src, const void* weights, const void* rot,
                       const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
     if (ts.os_exact)
-        return scatter_kp_osx<CUBIC, MODE, WEIGHTS, true>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
-    return scatter_kp_osx<CUBIC, MODE, WEIGHTS, false>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return scatter_kp_osx<CUBIC, MODE, WEIGHTS, true>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+    return scatter_kp_osx<CUBIC, MODE, WEIGHTS, false>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
 }
 
 template <bool CUBIC, bool OSX>
@@ -1699,7 +1773,23 @@ hipError_t forw_store(bool cubic, const Geom& g, const TileSpec& ts, const void*
 
 }  // namespace
 
-int64_t forw_reach_items(const Geom& g, const TileSpec& ts, std::vector<int>& out) {
+void split_items(const PoseSplit& ps, int64_t B, std::vector<TileItem>& out) {
+    using U = unsigned short;
+    for (int l = 0; l < ps.n; ++l) {
+        const PoseSplit::Level& v = ps.lv[l];
+        for (int64_t b = 0; b < B; ++b)
+            for (int d = v.lo[0]; d < v.lo[0] + v.size(0); ++d)
+                for (int r = v.lo[1]; r < v.lo[1] + v.size(1); ++r)
+                    for (int c = v.lo[2]; c < v.lo[2] + v.size(2); ++c) {
+                        // (the boxes are nested: the next one in holds the others)
+                        const bool held = l > 0 && ps.lv[l - 1].holds(d, r, c);
+                        for (int j = 0; j < v.k; ++j)
+                            out.push_back(TileItem{U(d), U(r), U(c), U(held ? 0 : v.k), int(b), j});
+                    }
+    }
+}
+
+int64_t forw_reach_items(const Geom& g, const TileSpec& ts, const PoseSplit& ps, std::vector<TileItem>& out) {
     const int64_t items = forw_items(g, ts);
     if (items > int64_t(INT32_MAX)) return items;
     // the rotation kernel's test (dist2 > rho2: the tile holds no sample) with a margin, so that
@@ -1710,36 +1800,34 @@ int64_t forw_reach_items(const Geom& g, const TileSpec& ts, std::vector<int>& ou
         const float q = lo > 0.f ? lo : (hi < 0.f ? -hi : 0.f);
         return q * q;
     };
-    // the core pieces (item_of's first items) lie within 40 voxels of the origin: all listed
-    const int cd = ts.fd1 - ts.fd0, cc = ts.fc1 - ts.fc0;
-    const int64_t ncore = g.B * int64_t(cd) * cc * cc * ts.fksplit;
-    for (int64_t w = 0; w < ncore; ++w) out.push_back(int(w));
-    // then every tile of each batch item in item_of's order (kd, kr, kc), the core tiles skipped
-    // when they are split
-    const int nt = ts.nt, nd = ts.ntfd;
+    auto reached = [&](int d, int r, int c) {
+        return axis2(ts.orgd + d * LD, LD) + axis2(ts.org + r * L, L) + axis2(ts.org + c * L, L) <= rho2;
+    };
+    split_items(ps, g.B, out);
+    out.erase(std::remove_if(out.begin(), out.end(),
+                             [&](const TileItem& f) { return f.k == 0 || !reached(f.d, f.r, f.c); }),
+              out.end());
+    // then every unsplit tile of each batch item
+    using U = unsigned short;
     for (int64_t b = 0; b < g.B; ++b)
-        for (int kd = 0; kd < nd; ++kd) {
+        for (int kd = 0; kd < ts.ntfd; ++kd) {
             const float d2 = axis2(ts.orgd + kd * LD, LD);
-            for (int kr = 0; kr < nt; ++kr) {
-                const float r2 = axis2(ts.org + kr * L, L);
-                if (d2 + r2 > rho2) continue;
-                const int64_t row = ncore + b * int64_t(nd) * nt * nt + (int64_t(kd) * nt + kr) * nt;
-                const bool core_row = ts.fksplit > 1 && kd >= ts.fd0 && kd < ts.fd1 && kr >= ts.fc0 && kr < ts.fc1;
-                for (int kc = 0; kc < nt; ++kc) {
-                    if (core_row && kc >= ts.fc0 && kc < ts.fc1) continue;
-                    if (d2 + r2 + axis2(ts.org + kc * L, L) <= rho2) out.push_back(int(row + kc));
-                }
+            for (int kr = 0; kr < ts.nt; ++kr) {
+                const float r2 = d2 + axis2(ts.org + kr * L, L);
+                if (r2 > rho2) continue;
+                for (int kc = 0; kc < ts.nt; ++kc)
+                    if (r2 + axis2(ts.org + kc * L, L) <= rho2 && !(ps.n > 0 && ps.lv[ps.n - 1].holds(kd, kr, kc)))
+                        out.push_back(TileItem{U(kd), U(kr), U(kc), 1, int(b), 0});
             }
         }
     return items;
 }
 
 hipError_t launch_pose_bins(const Geom& g, const void* rot, const BinGrid& bg, const BinBox& bb, const CallPoses* cp,
-                            hipStream_t s, const TileSpec& ts, void* dst, void* wdst) {
+                            hipStream_t s) {
     const int64_t blocks = g.B_rot * int64_t(bg.nb[1]) * bg.nb[2] * ((g.P + kBinPoses - 1) / kBinPoses);
     if (blocks == 0 || blocks > kBinMaxGroups) return hipErrorInvalidValue;  // make_bins keeps calls within
-    hipLaunchKernelGGL(k_pose_bins, dim3(unsigned(blocks)), dim3(kBinThreads), 0, s, g, (const float*)rot, bg, bb, cp,
-                       ts, (Cx<float>*)dst, (float*)wdst);
+    hipLaunchKernelGGL(k_pose_bins, dim3(unsigned(blocks)), dim3(kBinThreads), 0, s, g, (const float*)rot, bg, bb, cp);
     return hipGetLastError();
 }
 
@@ -1780,18 +1868,18 @@ hipError_t launch_bpback3_tiled(bool cubic, const Geom& g, const TileSpec& ts, c
                                                     cp, gl, s);
 }
 
-hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const void* src,
+hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src,
                                  const void* weights, const void* rot, const void* shifts, void* dst, void* wdst,
                                  CallPoses* cp, int gl, hipStream_t s) {
     if (mode == 0) {
         if (weights)
-            return cubic ? scatter_kp<true, 0, true>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s)
-                         : scatter_kp<false, 0, true>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
-        return cubic ? scatter_kp<true, 0, false>(g, ts, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
-                     : scatter_kp<false, 0, false>(g, ts, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
+            return cubic ? scatter_kp<true, 0, true>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s)
+                         : scatter_kp<false, 0, true>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return cubic ? scatter_kp<true, 0, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
+                     : scatter_kp<false, 0, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
     }
-    return cubic ? scatter_kp<true, 1, false>(g, ts, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
-                 : scatter_kp<false, 1, false>(g, ts, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
+    return cubic ? scatter_kp<true, 1, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
+                 : scatter_kp<false, 1, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
 }
 
 }  // namespace tp
