@@ -36,13 +36,54 @@ def _cases():
 CASES = _cases()
 
 
+def _rotations_at(args):
+    return next(i for i, a in enumerate(args) if hasattr(a, "shape") and a.dim() == 4 and a.shape[-2:] in ((2, 2), (3, 3)))
+
+
 @pytest.mark.parametrize("case", CASES, ids=[c["name"] for c in CASES])
 def test_pose_ranges_match_oracle(case, hip, oracle):
     args, tensors = make_inputs(case)
-    rot = args[2].detach().clone()
+    at = _rotations_at(args)
+    rot = args[at].detach().clone()
     rot[:, 2::5] *= 1.1
-    args[2] = rot.requires_grad_(args[2].requires_grad)
+    args[at] = rot.requires_grad_(args[at].requires_grad)
     print(f"[pose ranges] {case['name']}", flush=True)
+    got = getattr(hip, case["op"])(*args)
+    exp = getattr(oracle, case["op"])(*args)
+    check_outputs(case["op"], got, exp, has_shifts=tensors.get("shifts") is not None, label=case["name"],
+                  cells=scatter_cells(case["op"], args, oracle))
+
+
+# Calls just past the size where the tile-owner gathers take over from the per-pixel ones: small boxes
+# with many poses (the other tests' small calls run per pixel).
+def _large_cases():
+    out, seed = [], 772000
+    for op, interp, n, os_, P, B, cut in (
+            ("project_3d_to_2d_forw", "linear", 30, 2.0, 3001, 1, None), ("project_3d_to_2d_forw", "linear", 32, 3.0, 700, 2, 9.5),
+            ("project_3d_to_2d_forw", "cubic", 24, 2.0, 1100, 1, None), ("project_3d_to_2d_forw", "cubic", 34, 1.3, 1500, 1, 15.0),
+            ("project_3d_to_2d_back", "linear", 30, 2.0, 3300, 1, None), ("project_3d_to_2d_back", "cubic", 26, 1.5, 1200, 1, None),
+            ("backproject_2d_to_3d_back", "linear", 30, 2.0, 3300, 1, None), ("backproject_2d_to_3d_back", "cubic", 28, 1.0, 500, 2, 12.0),
+            ("project_2d_forw", "cubic", 48, 3.0, 4000, 1, None), ("project_2d_forw", "linear", 256, 1.0, 1900, 1, None),
+            ("project_2d_back", "linear", 150, 1.5, 21, 2, None), ("project_2d_back", "cubic", 146, 2.0, 18, 1, 60.0),
+            ("backproject_2d_back", "linear", 150, 0.75, 21, 2, 50.0), ("backproject_2d_back", "cubic", 146, 2.0, 18, 1, None)):
+        seed += 1
+        out.append(_case(f"large_{op}_{interp}_n{n}_os{os_:g}_P{P}", op, interp=interp, os=os_, cutoff=cut, B=B, P=P, n=n,
+                         B_rot=B, seed=seed, weights=(seed % 2 == 0)))
+    return out
+
+
+LARGE = _large_cases()
+
+
+@pytest.mark.parametrize("case", LARGE, ids=[c["name"] for c in LARGE])
+def test_tiled_gathers_past_the_per_pixel_sizes(case, hip, oracle):
+    args, tensors = make_inputs(case)
+    at = _rotations_at(args)
+    rot = args[at].detach().clone()
+    rot[:, 1::3] *= 1.1
+    rot[:, 2::7] *= 2.5  # beyond the tiled range
+    args[at] = rot.requires_grad_(args[at].requires_grad)
+    print(f"[large] {case['name']}", flush=True)
     got = getattr(hip, case["op"])(*args)
     exp = getattr(oracle, case["op"])(*args)
     check_outputs(case["op"], got, exp, has_shifts=tensors.get("shifts") is not None, label=case["name"],

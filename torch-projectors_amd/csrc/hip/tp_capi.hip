@@ -175,7 +175,9 @@ tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const 
     double r = one_level ? 40.0 : 16.0, p = 1.0;  // this level's half width; share of the poses that cross its tiles
     double total = 0.0;
     for (int l = 0; l < (one_level ? 1 : tp::kSplitLevels); ++l, r *= 2.0) {
-        const int64_t k = int64_t(std::ceil(double(g.P) * p / target));
+        // (to the nearest: 21 poses in two pieces of a target of 16 cost more than they balanced)
+        const double want = double(g.P) * p / target;
+        const int64_t k = int64_t(one_level ? std::ceil(want) : std::floor(want + 0.5));
         if (k <= 1) break;
         tp::PoseSplit::Level& v = ps.lv[l];
         int64_t tiles = 1;
@@ -352,6 +354,39 @@ tp::TileSpec2 tile_spec2(const tp::Geom& g, bool cubic) {
     const int grows = int(std::ceil(std::sqrt(2.0) * gw / g.os)) + 2;
     ts.kp_gather = grows <= 16 ? 4 : (grows <= 32 ? 2 : 1);
     return ts;
+}
+
+// Calls small enough that the per-pixel gathers beat the tile-owner ones (fp32, complex-half volumes
+// too).  A tiled gather pays for its tiles whatever the call samples (staging, culling, two launches
+// that a call of rotations leaves at once, a zero fill or a completion pass); a per-pixel one is a
+// single launch that reads every tap through the caches.  The lines below were fitted to both sides
+// measured over 64 <= n <= 256, 8 to 4000 poses, in us (tiled / per pixel):
+//   forward, linear: 41 poses of 96 at oversampling 2, 30 / 10; 200 of 64 25 / 14; 200 of 128 56 / 58;
+//     40 of 256 216 / 56, 200 of them 286 / 270; at oversampling 1, whose samples share lines, 200 of 128
+//     44 / 24, 1000 of them 95 / 103; cubic, 40 of 128 at 2 84 / 73, 200 of them 117 / 319;
+//   forward 2D, linear: 256 of 64 24 / 10, 8 x 4000 of 64 489 / 414, 8 x 2000 of 128 706 / 741; cubic, 200
+//     of 128 44 / 26, 2000 of them 179 / 211;
+//   gradient gathers (a projection or backprojection with every gradient): 200 of 64 136 / 99, 1000 of
+//     64 263 / 206, 1000 of 128 595 / 601, at oversampling 1 200 of 256 416 / 534; cubic, 200 of 64
+//     268 / 273.  In 2D a pose of many blocks waits for its own sums' atomics: 50 of 256 133 / 164,
+//     so those boxes stay tiled.
+// Projections of a call's active pixels and the tiles that its samples reach:
+double active_samples(const tp::Geom& g) { return 0.785 * double(g.B) * double(g.P) * double(g.rect); }
+double reached_tiles(const tp::Geom& g) {
+    const double R = std::min(g.os * std::sqrt(std::max(0.0, g.cut2)), g.os * double(g.n));
+    return 4.19 * R * R * R / double(tp::kTileEdge * tp::kTileEdge * tp::kTileEdgeD);
+}
+bool small_forward(int dim, const tp::Geom& g, bool cubic) {
+    const double A = active_samples(g), apart = 2.0 / g.os;
+    if (dim == 2) return A < (cubic ? 4.5e6 * apart : 4.8e7);
+    const double tiles = double(g.B) * reached_tiles(g);
+    return A < (cubic ? 0.15e6 * apart * apart + 55.0 * tiles : 0.9e6 * apart * apart + 180.0 * tiles);
+}
+bool small_gradients(int dim, const tp::Geom& g, bool cubic) {
+    const double A = active_samples(g);
+    if (dim == 2) return A < (cubic ? 1.0e6 : 1.5e6) && g.chunks <= 40;
+    const double tiles = double(g.B) * reached_tiles(g) * std::min(4.0, g.os * g.os / 4.0);
+    return A < (cubic ? 0.25e6 + 40.0 * tiles : 1.0e6 + 300.0 * tiles);
 }
 
 int64_t cx_words(int dtype, int64_t elems) { return elems * (dtype == TP_F32 ? 2 : 4); }
@@ -733,7 +768,12 @@ int project_forw(int dim, int dtype, const void* rec, int64_t B, int64_t D, int6
     TP_TRY(need(out, "projections"));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool cubic = interp == TP_CUBIC;
-    if (use_tiles(dim, dt, os, n)) {
+    const bool tiles = use_tiles(dim, dt, os, n), tiles2 = use_tiles2(dim, dt, os, n);
+    if ((tiles || tiles2) && small_forward(dim, g, cubic)) {
+        TP_TRY(sc.get(s));  // (a stream's first call is refused under capture, whatever its size)
+        return launched(tp::launch_project_forw(dim, kdt, cubic, g, rec, rot, shifts, out, s), "projection launch");
+    }
+    if (tiles) {
         Splits sp{};
         tp::TileSpec ts = tile_spec(g, cubic, TileOp::project, sp);
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s));
@@ -743,7 +783,7 @@ int project_forw(int dim, int dtype, const void* rec, int64_t B, int64_t D, int6
         return launched(tp::launch_project_forw(dim, kdt, cubic, g, rec, rot, shifts, out, s, true),
                         "projection launch");
     }
-    if (use_tiles2(dim, dt, os, n)) {
+    if (tiles2) {
         // zero-fill first: the tiled gather writes the active pixels of tiled poses, the
         // rest kernel the other poses
         TP_TRY(zero(out, cx_words(dt, g.B * g.P * int64_t(g.npix)), s));
@@ -790,19 +830,22 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     TP_TRY(need(rec, "reconstruction"));
     TP_TRY(need(rot, "rotations"));
     CallScratch sc;
+    // (complex-half volumes have no per-pixel gradients without the scatter)
+    const bool per_pixel = (grot || gshift) && !rec_half && small_gradients(dim, g, cubic);
     if (tiles) {
         Splits sp{};
         tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, sp);
         TP_TRY(plan_scatter(g, ts, sp, false, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, &ts));
         TP_TRY(fill_bins(cubic, g, ts, rot, sc, s));
-        TP_TRY(use_forw_lists(g, ts, sp, sc, s));
+        if (!per_pixel) TP_TRY(use_forw_lists(g, ts, sp, sc, s));
         TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 1, g, ts, sp.s[0], gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
                                                   s),
                         "tiled reconstruction-gradient launch"));
-        TP_TRY(launched(tp::launch_grads3_tiled(cubic, g, ts, gproj, rec, rot, shifts, grot, gshift, sc.p, 1, s,
-                                                rec_half),
-                        "tiled rotation/shift-gradient launch"));
+        if (!per_pixel)
+            TP_TRY(launched(tp::launch_grads3_tiled(cubic, g, ts, gproj, rec, rot, shifts, grot, gshift, sc.p, 1, s,
+                                                    rec_half),
+                            "tiled rotation/shift-gradient launch"));
     }
     if (tiles2) {
         const tp::TileSpec2 ts = tile_spec2(g, cubic);
@@ -810,12 +853,13 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
         TP_TRY(launched(tp::launch_scatter2_tiled(cubic, 1, g, ts, gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
                                                   s),
                         "tiled reconstruction-gradient launch"));
-        TP_TRY(launched(tp::launch_gather2_tiled(cubic, 1, g, ts, rec, nullptr, rot, shifts, nullptr, nullptr, gproj,
-                                                 grot, gshift, sc.p, 1, s, rec_half),
-                        "tiled rotation/shift-gradient launch"));
+        if (!per_pixel)
+            TP_TRY(launched(tp::launch_gather2_tiled(cubic, 1, g, ts, rec, nullptr, rot, shifts, nullptr, nullptr,
+                                                     gproj, grot, gshift, sc.p, 1, s, rec_half),
+                            "tiled rotation/shift-gradient launch"));
     }
     return launched(tp::launch_project_back(dim, rec_half ? 2 : dtype, cubic, g, gproj, rec, rot, shifts, grec, grot,
-                                            gshift, s, (tiles || tiles2) ? 1 : 0),
+                                            gshift, s, (tiles || tiles2) ? (per_pixel ? 1 : 2) : 0),
                     "projection backward launch");
 }
 
@@ -888,14 +932,17 @@ int backproject_back(int dim, int dtype, const void* gdata, const void* gw, int6
     TP_TRY(need(rot, "rotations"));
     TP_TRY(need(gproj, "grad_projections"));
     const bool cubic = interp == TP_CUBIC;
-    const bool tiles2 = use_tiles2(dim, dtype, os, n);
-    const bool tiles = use_tiles(dim, dtype, os, n);
+    bool tiles2 = use_tiles2(dim, dtype, os, n), tiles = use_tiles(dim, dtype, os, n);
+    CallScratch sc;
+    if ((tiles || tiles2) && small_gradients(dim, g, cubic)) {
+        TP_TRY(sc.get(s));  // (a stream's first call is refused under capture, whatever its size)
+        tiles = tiles2 = false;
+    }
     if (tiles2 || tiles) {
         // the tiled gathers write the active pixels of tiled poses, the per-pixel kernel the rest
         TP_TRY(zero(gproj, cx_words(dtype, g.B * g.P * int64_t(g.npix)), s));
         TP_TRY(zero(gweights, re_words(dtype, g.B * g.P * int64_t(g.npix)), s));
     }
-    CallScratch sc;
     if (tiles) {
         Splits sp{};
         tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, sp);

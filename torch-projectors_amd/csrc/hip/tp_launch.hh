@@ -213,9 +213,10 @@ hipError_t launch_zero_outside(int dt, const Geom& g, void* out, void* wout, hip
 // do not take (pose_tiled3 / pose_tiled2).
 hipError_t launch_project_forw(int dim, int dt, bool cubic, const Geom& g, const void* rec, const void* rot,
                                const void* shifts, void* out, hipStream_t s, bool rest_only = false);
-// `rest` != 0 (fp32): tiled poses are left to the tiled kernels
+// `rest` 2 (fp32): tiled poses are left to the tiled kernels
 // entirely (the tiled scatter gives their reconstruction gradient,
-// launch_grads3_tiled / launch_gather2_tiled their rotation/shift gradients).
+// launch_grads3_tiled / launch_gather2_tiled their rotation/shift gradients);
+// `rest` 1: only their reconstruction gradient is.
 // `dt` 2: a complex-half volume with fp32 arithmetic, gradients and outputs.
 hipError_t launch_project_back(int dim, int dt, bool cubic, const Geom& g, const void* gproj, const void* rec,
                                const void* rot, const void* shifts, void* grec, void* grot, void* gshift,

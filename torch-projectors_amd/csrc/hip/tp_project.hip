@@ -134,17 +134,17 @@ __global__ __launch_bounds__(kBlock) void k_project_back(Geom g, const Cx<T>* __
     constexpr int K = RS + 2;
     __shared__ T red[kBlock / 64][K];
     const T cut2 = T(g.cut2);
-    // REST: one pose per outer step, checked once
-    const int64_t outer_n = REST != 0 ? g.B * g.P : g.work;
+    // REST 2: one pose per outer step, checked once; otherwise one (pose, chunk)
+    const int64_t outer_n = REST == 2 ? g.B * g.P : g.work;
     for (int64_t outer = blockIdx.x; outer < outer_n; outer += gridDim.x) {
       bool scatter = true;
       if constexpr (REST != 0) {
-        const int64_t b0 = outer / g.P;
-        scatter = !pose_tiled_d<DIM>(rot + ((g.B_rot == 1 ? 0 : b0) * g.P + (outer - b0 * g.P)) * RS);
+        const int64_t bp0 = REST == 2 ? outer : outer / g.chunks, b0 = bp0 / g.P;
+        scatter = !pose_tiled_d<DIM>(rot + ((g.B_rot == 1 ? 0 : b0) * g.P + (bp0 - b0 * g.P)) * RS);
         if (!scatter && (REST == 2 || (!ROT && !SHIFT))) continue;  // block-uniform
       }
-      for (int ch = 0; ch < (REST != 0 ? g.chunks : 1); ++ch) {
-        const int64_t w = REST != 0 ? outer * g.chunks + ch : outer;
+      for (int ch = 0; ch < (REST == 2 ? g.chunks : 1); ++ch) {
+        const int64_t w = REST == 2 ? outer * g.chunks + ch : outer;
         const int64_t bp = w / g.chunks;
         int i = 0, j = 0;
         const bool in_rect = rect_pixel(g, int(w - bp * g.chunks) * kBlock + int(threadIdx.x), i, j);
@@ -228,8 +228,8 @@ hipError_t forw_rest(const Geom& g, const void* rec, const void* rot, const void
 template <int DIM, typename T, bool CUBIC, bool ROT, bool SHIFT, int REST, typename VS>
 hipError_t back4(const Geom& g, const void* gproj, const void* rec, const void* rot, const void* shifts, void* grec,
                  void* grot, void* gshift, hipStream_t s) {
-    // with REST most (pose, chunk) items are skipped at once: fewer, longer-lived blocks
-    const unsigned grid = REST ? grid_for(g.B * g.P) : grid_for(g.work);
+    // with REST 2 most (pose, chunk) items are skipped at once: fewer, longer-lived blocks
+    const unsigned grid = REST == 2 ? grid_for(g.B * g.P) : grid_for(g.work);
     hipLaunchKernelGGL((k_project_back<DIM, T, CUBIC, ROT, SHIFT, REST, VS>), dim3(grid), dim3(kBlock), 0,
                        s, g, (const Cx<T>*)gproj, (const Cx<VS>*)rec, (const T*)rot, (const T*)shifts, (Cx<T>*)grec,
                        (T*)grot, (T*)gshift);
@@ -299,6 +299,13 @@ hipError_t launch_project_back(int dim, int dt, bool cubic, const Geom& g, const
                          : back<2, float, false, 0, __half>(g, gproj, rec, rot, shifts, grec, grot, gshift, s);
         return cubic ? back<3, float, true, 0, __half>(g, gproj, rec, rot, shifts, grec, grot, gshift, s)
                      : back<3, float, false, 0, __half>(g, gproj, rec, rot, shifts, grec, grot, gshift, s);
+    }
+    if (rest == 1 && dt == 0) {
+        if (dim == 2)
+            return cubic ? back<2, float, true, 1>(g, gproj, rec, rot, shifts, grec, grot, gshift, s)
+                         : back<2, float, false, 1>(g, gproj, rec, rot, shifts, grec, grot, gshift, s);
+        return cubic ? back<3, float, true, 1>(g, gproj, rec, rot, shifts, grec, grot, gshift, s)
+                     : back<3, float, false, 1>(g, gproj, rec, rot, shifts, grec, grot, gshift, s);
     }
     if (rest != 0 && dt == 0) {
         if (dim == 2)
