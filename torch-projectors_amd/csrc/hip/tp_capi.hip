@@ -175,9 +175,9 @@ tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const 
     double r = one_level ? 40.0 : 16.0, p = 1.0;  // this level's half width; share of the poses that cross its tiles
     double total = 0.0;
     for (int l = 0; l < (one_level ? 1 : tp::kSplitLevels); ++l, r *= 2.0) {
-        // (to the nearest: 21 poses in two pieces of a target of 16 cost more than they balanced)
+        // (21 poses in two pieces for a target of 16 cost more than they balanced)
         const double want = double(g.P) * p / target;
-        const int64_t k = int64_t(one_level ? std::ceil(want) : std::floor(want + 0.5));
+        const int64_t k = !one_level && want < 1.5 ? 1 : int64_t(std::ceil(want));
         if (k <= 1) break;
         tp::PoseSplit::Level& v = ps.lv[l];
         int64_t tiles = 1;
