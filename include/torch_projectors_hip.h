@@ -243,6 +243,25 @@ int tp_rfftn(int dtype, int dim, int64_t batch, int64_t boxsize, const void* rea
  * their input as scratch). */
 int tp_irfftn(int dtype, int dim, int64_t batch, int64_t boxsize, void* spectrum, void* real, void* stream);
 
+/* The whole preparation of a 3D box in three passes over memory (TP_F32,
+ * dim 3, padded_boxsize even, at most 2048 and with no prime factor above 7):
+ *   tp_to_fourier    tp_fftshift_pad, then tp_rfftn
+ *   tp_from_fourier  tp_normalize_reconstruction (when weights are given: else
+ *                    data is taken as it is), tp_irfftn, then tp_ifftshift_crop
+ *                    to [crop_start, crop_start + boxsize) of each axis
+ * of `batch` boxes, inputs left unchanged, with `work_bytes` >=
+ * tp_fused_fourier_work() bytes of device memory at `work` (256-byte aligned,
+ * free again once the call's work on the stream is done).
+ * tp_fused_fourier_work is 0 for a transform they do not cover (inverse: 0 for
+ * tp_to_fourier, 1 for tp_from_fourier). */
+int64_t tp_fused_fourier_work(int inverse, int dtype, int dim, int64_t batch, int64_t boxsize,
+                              int64_t padded_boxsize);
+int tp_to_fourier(int dtype, int dim, int64_t batch, int64_t boxsize, int64_t padded_boxsize, int64_t pad_before,
+                  const void* real, void* spectrum, void* work, int64_t work_bytes, void* stream);
+int tp_from_fourier(int dtype, int dim, int64_t batch, int64_t boxsize, int64_t padded_boxsize, int64_t crop_start,
+                    const void* data, const void* weights, double reg, void* real, void* work, int64_t work_bytes,
+                    void* stream);
+
 /* out[e] = data[e] / (weights[e] + reg) component-wise where weights[e] + reg > 0,
  * else 0: a Wiener-style normalisation of a backprojected pair (data complex,
  * weights real, both of `dtype`, `elems` elements).  No counterpart in the

@@ -1179,6 +1179,46 @@ int tp_irfftn(int dtype, int dim, int64_t batch, int64_t boxsize, void* spectrum
     return TP_OK;
 }
 
+int64_t tp_fused_fourier_work(int inverse, int dtype, int dim, int64_t batch, int64_t boxsize,
+                              int64_t padded_boxsize) {
+    if (dtype != TP_F32 || dim != 3) return 0;
+    return tp::fused_fft_work(inverse != 0, batch, boxsize, padded_boxsize);
+}
+
+int tp_to_fourier(int dtype, int dim, int64_t batch, int64_t boxsize, int64_t padded_boxsize, int64_t pad_before,
+                  const void* real, void* spectrum, void* work, int64_t work_bytes, void* stream) {
+    g_err.clear();
+    const int64_t need_bytes = tp_fused_fourier_work(0, dtype, dim, batch, boxsize, padded_boxsize);
+    if (need_bytes == 0) return fail("tp_to_fourier does not cover this transform (tp_fused_fourier_work is 0)");
+    if (pad_before < 0 || pad_before > padded_boxsize - boxsize)
+        return fail("pad_before must be in [0, padded_boxsize - boxsize]");
+    TP_TRY(need(real, "real"));
+    TP_TRY(need(spectrum, "spectrum"));
+    TP_TRY(need(work, "work"));
+    if (work_bytes < need_bytes) return fail("work is smaller than tp_fused_fourier_work");
+    return launched(tp::fused_to_fourier(batch, boxsize, padded_boxsize, pad_before, real, spectrum, work,
+                                         static_cast<hipStream_t>(stream)),
+                    "fused forward transform launch");
+}
+
+int tp_from_fourier(int dtype, int dim, int64_t batch, int64_t boxsize, int64_t padded_boxsize, int64_t crop_start,
+                    const void* data, const void* weights, double reg, void* real, void* work, int64_t work_bytes,
+                    void* stream) {
+    g_err.clear();
+    const int64_t need_bytes = tp_fused_fourier_work(1, dtype, dim, batch, boxsize, padded_boxsize);
+    if (need_bytes == 0) return fail("tp_from_fourier does not cover this transform (tp_fused_fourier_work is 0)");
+    if (crop_start < 0 || crop_start > padded_boxsize - boxsize)
+        return fail("crop_start must be in [0, padded_boxsize - boxsize]");
+    if (weights && !std::isfinite(reg)) return fail("reg must be finite");
+    TP_TRY(need(data, "data"));
+    TP_TRY(need(real, "real"));
+    TP_TRY(need(work, "work"));
+    if (work_bytes < need_bytes) return fail("work is smaller than tp_fused_fourier_work");
+    return launched(tp::fused_from_fourier(batch, boxsize, padded_boxsize, crop_start, data, weights, reg, real, work,
+                                           static_cast<hipStream_t>(stream)),
+                    "fused inverse transform launch");
+}
+
 int tp_normalize_reconstruction(int dtype, const void* data, const void* weights, int64_t elems, double reg,
                                 void* out, void* stream) {
     g_err.clear();

@@ -291,6 +291,15 @@ constexpr int kFftNoPlanUnderCapture = -1;
 int fft_forward(int dt, int dim, int64_t batch, int64_t N, const void* real, void* spec, hipStream_t s);
 int fft_inverse(int dt, int dim, int64_t batch, int64_t N, void* spec, void* real, hipStream_t s);
 
+// 3D transforms with their padding / cropping (tp_fft.hip): bytes of workspace they need, 0 when they
+// do not cover the boxes; real [batch, n^3] -> spectrum [batch, N, N, N/2+1], and back from data (divided
+// by weights + reg when weights are given).  The inputs are left unchanged.
+int64_t fused_fft_work(bool inverse, int64_t batch, int64_t n, int64_t N);
+hipError_t fused_to_fourier(int64_t batch, int64_t n, int64_t N, int64_t pad_before, const void* real, void* spectrum,
+                            void* work, hipStream_t s);
+hipError_t fused_from_fourier(int64_t batch, int64_t n, int64_t N, int64_t crop_start, const void* data,
+                              const void* weights, double reg, void* real, void* work, hipStream_t s);
+
 // `rest_only` (fp32): tiled poses were computed by the tiled gathers into
 // zero-filled outputs and are skipped; other poses everything.
 hipError_t launch_backproject_back(int dim, int dt, bool cubic, const Geom& g, const void* gdata, const void* gw,

@@ -37,6 +37,8 @@ SIGNATURES = {
     "tp_ifftshift_crop": [_I, _P, _L, _I, _L, _L, _L, _L, _L, _P, _P],
     "tp_rfftn": [_I, _I, _L, _L, _P, _P, _P],
     "tp_irfftn": [_I, _I, _L, _L, _P, _P, _P],
+    "tp_to_fourier": [_I, _I, _L, _L, _L, _L, _P, _P, _P, _L, _P],
+    "tp_from_fourier": [_I, _I, _L, _L, _L, _L, _P, _P, _D, _P, _P, _L, _P],
     "tp_normalize_reconstruction": [_I, _P, _P, _L, _D, _P, _P],
 }
 # helpers returning a size: name -> argument types
@@ -44,6 +46,7 @@ SIZE_HELPERS = {
     "tp_backproject_rec_boxsize": [_L, _D],
     "tp_padded_boxsize": [_L, _D],
     "tp_cropped_boxsize": [_L, _D],
+    "tp_fused_fourier_work": [_I, _I, _I, _L, _L, _L],
 }
 EXPORTS = ["tp_last_error", "tp_abi_version", *SIZE_HELPERS, *SIGNATURES]
 
@@ -88,3 +91,7 @@ def padded_boxsize(n, oversampling):
 
 def cropped_boxsize(n, oversampling):
     return int(lib().tp_cropped_boxsize(int(n), float(oversampling)))
+
+
+def fused_fourier_work(inverse, dim, batch, n, N):
+    return int(lib().tp_fused_fourier_work(int(inverse), TP_F32, int(dim), int(batch), int(n), int(N)))
