@@ -4,11 +4,13 @@
 // reference (validate_projection_inputs, projection_utils.h:23-48, and the
 // per-op TORCH_CHECKs), derives the launch geometry, zero-fills the outputs
 // that are accumulated, and enqueues the kernels on the caller's stream.
-// Nothing is synchronised.  The only memory besides the caller's is a small
-// scratch area per (device, stream) that the calls of the tiled kernels use
-// (tp::CallPoses: a summary of their poses and work counters), allocated by
-// the first such call on that stream and kept for the life of the process;
-// tp_project_3d_to_2d_forw_noalloc uses a static device array instead.
+// The memory besides the caller's is kept per (device, stream) for the life
+// of the process: a small scratch area that the calls of the tiled kernels use
+// (tp::CallPoses: a summary of their poses and work counters), the last lists
+// of 3D work items, and the 3D scatters' workspace (pose bins, partial sums of
+// split tiles).  Nothing is synchronised except where a call lists a new
+// geometry or outgrows that workspace.  tp_project_3d_to_2d_forw_noalloc uses a
+// static device array and neither list nor workspace.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
