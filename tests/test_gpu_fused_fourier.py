@@ -1,7 +1,7 @@
 """The fused 3D transforms of the reference preparation (to_fourier, from_fourier, reconstruct) against torch.fft
 in double precision: edges whose passes mix every radix, one workgroup tile of columns and ragged ones, both
 tile widths below the widest, an odd number of rows, several boxes, oversampling 1; and boxes with other prime
-factors, which take the hipFFT path.
+factors, which take the hipFFT path.  The boxes of a batch are compared with the same boxes alone.
 
 The bar: each of the log2(N) butterfly levels of each axis rounds to 2^-24 relative, in the 2-norm about
 sqrt(3 log2 N) 2^-24 with the twiddles' rounding as much again: 1e-6 is five times that at N = 2048.
@@ -56,6 +56,56 @@ def test_fused_transforms_match_fft64(B, n, N, gpu):
     v = torch.where(den > 0, data.to(torch.complex128) / den, torch.zeros((), dtype=torch.complex128, device="cuda"))
     assert _rel(FM.reconstruct(data, w, os_, reg=0.25, dim=3), real_of(v)) < 1e-6
     assert torch.equal(data, kept)
+
+
+# (box edge, padded edge, oversampling of the way back): odd and even edges, whose boxes end with a row
+# without and with a partner; 85 is what an oversampling of 1.5 keeps of 128
+BOXES = [(9, 18, 2.0), (8, 16, 2.0), (1, 2, 2.0), (63, 126, 2.0), (85, 128, 1.5), (33, 162, 162 / 33)]
+
+
+@pytest.mark.parametrize("n,N,os_", BOXES, ids=[f"n{n}_N{N}" for n, N, _ in BOXES])
+def test_boxes_of_a_batch_are_independent(n, N, os_, gpu):
+    """Boxes of very different scale, one with a NaN and one with an infinity: every other box must come out
+    bit for bit as it does alone, and within the bar of the double-precision transform."""
+    from torch_projectors import fourier as FM
+    g = torch.Generator(device="cuda").manual_seed(7000 + N)
+    B = 5
+    scale = torch.tensor([1.0, 1e6, 1e-6, 1.0, 1.0], device="cuda").view(B, 1, 1, 1)
+    print(f"[fused fourier] boxes n={n} N={N}", flush=True)
+
+    def check(batch, run, exact, what):
+        out = run(batch)
+        for b in range(B):
+            alone = run(batch[b:b + 1])
+            if b == 3 or b == 1:
+                assert not torch.isfinite(torch.view_as_real(alone) if alone.is_complex() else alone).all()
+                continue
+            assert torch.equal(out[b:b + 1], alone), f"{what}: box {b} differs from the same box alone"
+            assert _rel(alone, exact(batch[b:b + 1])) < 1e-6, f"{what}: box {b}"
+
+    if FM.capi.padded_boxsize(n, os_) == N:
+        x = torch.randn(B, n, n, n, generator=g, device="cuda") * scale
+        x[1, 0, 0, 0] = float("nan")
+        x[3, -1, -1, -1] = float("inf")
+        lo = (N - n) // 2
+
+        def spec64(v):
+            v = torch.nn.functional.pad(v.double(), (lo, N - n - lo) * 3)
+            return torch.fft.rfftn(torch.fft.fftshift(v, dim=(1, 2, 3)), dim=(1, 2, 3), norm="forward")
+        check(x, lambda v: FM.to_fourier(v, os_), spec64, "to_fourier")
+    if FM.capi.cropped_boxsize(N, os_) != n:
+        return
+    at = (N - n) // 2
+
+    def real64(v):
+        y = torch.fft.irfftn(v.to(torch.complex128), s=[N] * 3, dim=(1, 2, 3), norm="forward")
+        return torch.fft.ifftshift(y, dim=(1, 2, 3))[:, at:at + n, at:at + n, at:at + n]
+    d = torch.randn(B, N, N, N // 2 + 1, generator=g, device="cuda", dtype=torch.complex64) * scale
+    d[1, 0, 0, 0] = float("nan")
+    d[3, -1, -1, 0] = float("inf")
+    check(d, lambda v: FM.from_fourier(v, os_, dim=3), real64, "from_fourier")
+    one = torch.ones(1, N, N, N // 2 + 1, device="cuda")
+    check(d, lambda v: FM.reconstruct(v, one.expand(v.shape).contiguous(), os_, dim=3), real64, "reconstruct")
 
 
 def test_strided_inputs_and_grad(gpu):

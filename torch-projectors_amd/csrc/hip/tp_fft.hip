@@ -22,8 +22,10 @@
 // A workgroup transforms W lines at once in LDS: W neighbouring columns of a
 // strided axis (64- or 128-byte rows in memory; workgroups next to each other
 // in x run on one XCD, whose L2 joins the rows' shared cache lines), or W pairs
-// of rows of the real axis (two real rows make one complex line, and their
-// spectra separate by Hermitian symmetry).  Lines stand in LDS as [N][W + 1]
+// of rows of the real axis (two real rows of one box make one complex line, and
+// their spectra separate by Hermitian symmetry; the last row of a box of odd
+// edge has a zero partner, never a row of the next box, whose NaNs or scale it
+// would take on).  Lines stand in LDS as [N][W + 1]
 // (the odd stride keeps both access orders free of bank conflicts) and go
 // through Stockham passes of radix 8, 4, 2, 7, 5 and 3: a thread holds its
 // butterflies' inputs (at most 14 values) in registers between two barriers,
@@ -343,10 +345,25 @@ __global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 
     fft_pass_at<INV, P2>(p.nf - 1, from_lds, st, false, tw, p, Ns);
 }
 
-// The real axis, forward: rows 2l and 2l + 1 of the box (n reals each) as line l; their spectra of
-// H = N / 2 + 1 values to rows 2l, 2l + 1 of `out` (`pitch` values apart).
+// The lines of the real axis: each box's `rows` rows in pairs, 2q and 2q + 1 as line q of its `pairs`.
+struct FftRows {
+    int lines, rows, pairs;
+};
+__device__ __forceinline__ void rows_of_line(const FftRows& r, int l, int64_t& ra, bool& has_a, bool& has_b) {
+    const int b = l / r.pairs, q = l - b * r.pairs;
+    ra = int64_t(b) * r.rows + 2 * q;
+    has_a = l < r.lines;
+    has_b = has_a && 2 * q + 1 < r.rows;
+}
+FftRows rows_in_pairs(int64_t batch, int64_t n) {
+    const int64_t pairs = (n * n + 1) / 2;  // (batch * n * n stays below 2^23: fused_fft_work)
+    return FftRows{int(batch * pairs), int(n * n), int(pairs)};
+}
+
+// The real axis, forward: a pair of rows of a box (n reals each) as one line; their spectra of
+// H = N / 2 + 1 values to the same rows of `out` (`pitch` values apart).
 template <bool P2>
-__global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 ? 6 : 4))) void k_fft_rows_forward(FftPlan p, FftBox box, int64_t rows, int H, int64_t pitch,
+__global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 ? 6 : 4))) void k_fft_rows_forward(FftPlan p, FftBox box, FftRows rows, int H, int64_t pitch,
                                                                   const float* __restrict__ in,
                                                                   const Cx<float>* __restrict__ twg,
                                                                   Cx<float>* __restrict__ out) {
@@ -355,33 +372,39 @@ __global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 
     Cx<float>* tw = buf + p.N * (p.W + 1);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = p.T / 64, WP = p.W + 1;
     for (int k = threadIdx.x; k < p.N; k += p.T) tw[k] = twg[k];
-    const int64_t r0 = int64_t(blockIdx.x) * 2 * p.W;
+    const int l0 = int(blockIdx.x) * p.W;
     for (int w = wave; w < p.W; w += waves) {
-        const int64_t ra = r0 + 2 * w, rb = ra + 1;
+        int64_t ra;
+        bool has_a, has_b;
+        rows_of_line(rows, l0 + w, ra, has_a, has_b);
+        const int64_t rb = ra + 1;
         for (int i = lane; i < p.N; i += 64) {
             const int s = line_to_box(box, p.N, i);
             const bool ok = s >= 0 && s < box.n;
-            buf[i * WP + w] = Cx<float>{ok && ra < rows ? in[ra * box.n + s] : 0.f, ok && rb < rows ? in[rb * box.n + s] : 0.f};
+            buf[i * WP + w] = Cx<float>{ok && has_a ? in[ra * box.n + s] : 0.f, ok && has_b ? in[rb * box.n + s] : 0.f};
         }
     }
     __syncthreads();
     int Ns = 1;
     fft_lines<false, P2>(buf, tw, p, 0, p.nf, Ns);
     for (int w = wave; w < p.W; w += waves) {
-        const int64_t ra = r0 + 2 * w, rb = ra + 1;
+        int64_t ra;
+        bool has_a, has_b;
+        rows_of_line(rows, l0 + w, ra, has_a, has_b);
+        const int64_t rb = ra + 1;
         for (int k = lane; k < H; k += 64) {
             const Cx<float> z = buf[k * WP + w], y = buf[(k == 0 ? 0 : p.N - k) * WP + w];
-            if (ra < rows) out[ra * pitch + k] = Cx<float>{0.5f * (z.re + y.re), 0.5f * (z.im - y.im)};
-            if (rb < rows) out[rb * pitch + k] = Cx<float>{0.5f * (z.im + y.im), 0.5f * (y.re - z.re)};
+            if (has_a) out[ra * pitch + k] = Cx<float>{0.5f * (z.re + y.re), 0.5f * (z.im - y.im)};
+            if (has_b) out[rb * pitch + k] = Cx<float>{0.5f * (z.im + y.im), 0.5f * (y.re - z.re)};
         }
     }
 }
 
-// The real axis, inverse: the half spectra of rows 2l and 2l + 1 as line l, a + i b on the whole axis
+// The real axis, inverse: the half spectra of a pair of rows as one line, a + i b on the whole axis
 // (their Hermitian halves filled in; the imaginary parts at k = 0 and N / 2 are ignored, as complex-to-
 // real transforms do), to the box's n reals of each row.
 template <bool P2>
-__global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 ? 6 : 4))) void k_fft_rows_inverse(FftPlan p, FftBox box, int64_t rows, int H, int64_t pitch,
+__global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 ? 6 : 4))) void k_fft_rows_inverse(FftPlan p, FftBox box, FftRows rows, int H, int64_t pitch,
                                                                   const Cx<float>* __restrict__ in,
                                                                   const Cx<float>* __restrict__ twg,
                                                                   float* __restrict__ out) {
@@ -390,13 +413,16 @@ __global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 
     Cx<float>* tw = buf + p.N * (p.W + 1);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = p.T / 64, WP = p.W + 1;
     for (int k = threadIdx.x; k < p.N; k += p.T) tw[k] = twg[k];
-    const int64_t r0 = int64_t(blockIdx.x) * 2 * p.W;
+    const int l0 = int(blockIdx.x) * p.W;
     for (int w = wave; w < p.W; w += waves) {
-        const int64_t ra = r0 + 2 * w, rb = ra + 1;
+        int64_t ra;
+        bool has_a, has_b;
+        rows_of_line(rows, l0 + w, ra, has_a, has_b);
+        const int64_t rb = ra + 1;
         for (int k = lane; k < H; k += 64) {
             Cx<float> a = {0.f, 0.f}, b = {0.f, 0.f};
-            if (ra < rows) a = in[ra * pitch + k];
-            if (rb < rows) b = in[rb * pitch + k];
+            if (has_a) a = in[ra * pitch + k];
+            if (has_b) b = in[rb * pitch + k];
             if (k == 0 || k == p.N / 2) a.im = b.im = 0.f;
             buf[k * WP + w] = Cx<float>{a.re - b.im, a.im + b.re};
             if (k > 0 && k < p.N / 2) buf[(p.N - k) * WP + w] = Cx<float>{a.re + b.im, b.re - a.im};
@@ -406,11 +432,14 @@ __global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(P2 
     int Ns = 1;
     fft_lines<true, P2>(buf, tw, p, 0, p.nf, Ns);
     for (int w = wave; w < p.W; w += waves) {
-        const int64_t ra = r0 + 2 * w, rb = ra + 1;
+        int64_t ra;
+        bool has_a, has_b;
+        rows_of_line(rows, l0 + w, ra, has_a, has_b);
+        const int64_t rb = ra + 1;
         for (int j = lane; j < box.n; j += 64) {
             const Cx<float> z = buf[box_to_line(box, p.N, j) * WP + w];
-            if (ra < rows) out[ra * box.n + j] = z.re;
-            if (rb < rows) out[rb * box.n + j] = z.im;
+            if (has_a) out[ra * box.n + j] = z.re;
+            if (has_b) out[rb * box.n + j] = z.im;
         }
     }
 }
@@ -455,15 +484,16 @@ hipError_t fused_to_fourier(int64_t batch, int64_t n, int64_t N, int64_t pad_bef
     FftPlan p;
     if (!plan_axis(N, p)) return hipErrorInvalidValue;
     const FftBox box{int(n), int(pad_before)};
-    const int64_t H = N / 2 + 1, rows = batch * n * n;
+    const int64_t H = N / 2 + 1;
+    const FftRows rows = rows_in_pairs(batch, n);
     Cx<float>* tw = static_cast<Cx<float>*>(work);
     char* lines = static_cast<char*>(work) + aligned(size_t(N) * 8);
     hipError_t e = run_twiddles(p, tw, s);
     if (e != hipSuccess) return e;
     // the rows' spectra [batch, n, n, pitch] stand in the output's memory until the last pass overwrites it
     const int64_t pitch = n * n * pitch_of(H) <= N * N * H ? pitch_of(H) : H;
-    const FftPlan pr = for_lines(p, rows / 2);
-    const int64_t groups = (rows + 2 * pr.W - 1) / (2 * pr.W);
+    const FftPlan pr = for_lines(p, rows.lines);
+    const int64_t groups = (rows.lines + pr.W - 1) / pr.W;
     hipLaunchKernelGGL((p.p2 ? k_fft_rows_forward<true> : k_fft_rows_forward<false>), dim3(unsigned(groups)),
                        dim3(pr.T), lds_bytes(pr), s, pr, box, rows, int(H), pitch,
                        (const float*)real, tw, (Cx<float>*)spectrum);
@@ -482,7 +512,8 @@ hipError_t fused_from_fourier(int64_t batch, int64_t n, int64_t N, int64_t crop_
     FftPlan p;
     if (!plan_axis(N, p)) return hipErrorInvalidValue;
     const FftBox box{int(n), int(crop_start)};
-    const int64_t H = N / 2 + 1, rows = batch * n * n;
+    const int64_t H = N / 2 + 1;
+    const FftRows rows = rows_in_pairs(batch, n);
     Cx<float>* tw = static_cast<Cx<float>*>(work);
     char* lines = static_cast<char*>(work) + aligned(size_t(N) * 8);
     char* planes = lines + aligned(size_t(batch) * n * N * H * 8);
@@ -496,8 +527,8 @@ hipError_t fused_from_fourier(int64_t batch, int64_t n, int64_t N, int64_t crop_
     FftCols y{0, N * H, H, n * pitch, pitch, int(H), 0};
     e = run_cols<true, false>(p, box, y, batch * n, lines, nullptr, 0.f, tw, planes, 1.0f, s);
     if (e != hipSuccess) return e;
-    const FftPlan pr = for_lines(p, rows / 2);
-    const int64_t groups = (rows + 2 * pr.W - 1) / (2 * pr.W);
+    const FftPlan pr = for_lines(p, rows.lines);
+    const int64_t groups = (rows.lines + pr.W - 1) / pr.W;
     hipLaunchKernelGGL((p.p2 ? k_fft_rows_inverse<true> : k_fft_rows_inverse<false>), dim3(unsigned(groups)),
                        dim3(pr.T), lds_bytes(pr), s, pr, box, rows, int(H), pitch,
                        (const Cx<float>*)planes, tw, (float*)real);
