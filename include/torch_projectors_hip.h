@@ -68,6 +68,21 @@ const char* tp_last_error(void);
 /* ABI version of this header (bumped on any signature change). */
 int tp_abi_version(void);
 
+/* Which gathers the TP_F32 and TP_F16S forward projections and pose gradients
+ * of the calling thread take, for tests and measurements that compare the two:
+ * by the call's size (the default of every thread), the tile-owner kernels, or
+ * the per-pixel ones (the pose gradients of a TP_F16S reconstruction always
+ * take the tiles).  Calls whose oversampling or size only the per-pixel kernels
+ * take, and TP_F64, are not affected.  Returns the setting it replaces; any
+ * other value changes nothing. */
+#define TP_ROUTE_BY_SIZE 0
+#define TP_ROUTE_TILES 1
+#define TP_ROUTE_PER_PIXEL 2
+int tp_set_gather_route(int route);
+/* The gathers of the calling thread's last call that had the choice
+ * (TP_ROUTE_TILES or TP_ROUTE_PER_PIXEL; TP_ROUTE_BY_SIZE before the first). */
+int tp_last_gather_route(void);
+
 /* Reconstruction box produced by the backprojection ops: ceil(n*os) rounded
  * up to even (cpu/3d/backprojection_2d_to_3d_kernels.cpp:129-132). */
 int64_t tp_backproject_rec_boxsize(int64_t proj_boxsize, double oversampling);

@@ -391,6 +391,15 @@ bool small_gradients(int dim, const tp::Geom& g, bool cubic) {
     return A < (cubic ? 0.25e6 + 40.0 * tiles : 1.0e6 + 300.0 * tiles);
 }
 
+// The calling thread's tp_set_gather_route, and the gathers its last call took.
+thread_local int t_route = TP_ROUTE_BY_SIZE, t_taken = TP_ROUTE_BY_SIZE;
+// Whether a call that the tile-owner gathers could take runs the per-pixel ones.
+bool takes_per_pixel(bool small) {
+    const bool per_pixel = t_route == TP_ROUTE_BY_SIZE ? small : t_route == TP_ROUTE_PER_PIXEL;
+    t_taken = per_pixel ? TP_ROUTE_PER_PIXEL : TP_ROUTE_TILES;
+    return per_pixel;
+}
+
 int64_t cx_words(int dtype, int64_t elems) { return elems * (dtype == TP_F32 ? 2 : 4); }
 int64_t re_words(int dtype, int64_t elems) { return elems * (dtype == TP_F32 ? 1 : 2); }
 
@@ -771,7 +780,7 @@ int project_forw(int dim, int dtype, const void* rec, int64_t B, int64_t D, int6
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool cubic = interp == TP_CUBIC;
     const bool tiles = use_tiles(dim, dt, os, n), tiles2 = use_tiles2(dim, dt, os, n);
-    if ((tiles || tiles2) && small_forward(dim, g, cubic)) {
+    if ((tiles || tiles2) && takes_per_pixel(small_forward(dim, g, cubic))) {
         TP_TRY(sc.get(s));  // (a stream's first call is refused under capture, whatever its size)
         return launched(tp::launch_project_forw(dim, kdt, cubic, g, rec, rot, shifts, out, s), "projection launch");
     }
@@ -833,7 +842,8 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     TP_TRY(need(rot, "rotations"));
     CallScratch sc;
     // (complex-half volumes have no per-pixel gradients without the scatter)
-    const bool per_pixel = (grot || gshift) && !rec_half && small_gradients(dim, g, cubic);
+    const bool per_pixel =
+        (tiles || tiles2) && (grot || gshift) && !rec_half && takes_per_pixel(small_gradients(dim, g, cubic));
     if (tiles) {
         Splits sp{};
         tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, sp);
@@ -936,7 +946,7 @@ int backproject_back(int dim, int dtype, const void* gdata, const void* gw, int6
     const bool cubic = interp == TP_CUBIC;
     bool tiles2 = use_tiles2(dim, dtype, os, n), tiles = use_tiles(dim, dtype, os, n);
     CallScratch sc;
-    if ((tiles || tiles2) && small_gradients(dim, g, cubic)) {
+    if ((tiles || tiles2) && takes_per_pixel(small_gradients(dim, g, cubic))) {
         TP_TRY(sc.get(s));  // (a stream's first call is refused under capture, whatever its size)
         tiles = tiles2 = false;
     }
@@ -973,6 +983,14 @@ extern "C" {
 const char* tp_last_error(void) { return g_err.c_str(); }
 
 int tp_abi_version(void) { return 1; }
+
+int tp_set_gather_route(int route) {
+    const int was = t_route;
+    if (route >= TP_ROUTE_BY_SIZE && route <= TP_ROUTE_PER_PIXEL) t_route = route;
+    return was;
+}
+
+int tp_last_gather_route(void) { return t_taken; }
 
 int64_t tp_backproject_rec_boxsize(int64_t proj_boxsize, double oversampling) {
     return rec_box(proj_boxsize, oversampling);

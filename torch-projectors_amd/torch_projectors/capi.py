@@ -48,7 +48,10 @@ SIZE_HELPERS = {
     "tp_cropped_boxsize": [_L, _D],
     "tp_fused_fourier_work": [_I, _I, _I, _L, _L, _L],
 }
-EXPORTS = ["tp_last_error", "tp_abi_version", *SIZE_HELPERS, *SIGNATURES]
+# which gathers this thread's calls take (for tests and measurements): name -> argument types
+ROUTE_BY_SIZE, ROUTE_TILES, ROUTE_PER_PIXEL = range(3)
+ROUTE_HELPERS = {"tp_set_gather_route": [_I], "tp_last_gather_route": []}
+EXPORTS = ["tp_last_error", "tp_abi_version", *SIZE_HELPERS, *ROUTE_HELPERS, *SIGNATURES]
 
 _lib = None
 
@@ -67,7 +70,7 @@ def lib():
             f = getattr(L, name)
             f.restype = ctypes.c_int64
             f.argtypes = argtypes
-        for name, argtypes in SIGNATURES.items():
+        for name, argtypes in (*ROUTE_HELPERS.items(), *SIGNATURES.items()):
             f = getattr(L, name)
             f.restype = ctypes.c_int
             f.argtypes = argtypes
