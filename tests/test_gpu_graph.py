@@ -11,14 +11,16 @@ The second test captures calls that do use the stream's pose bins (the warm-up h
 then grows that workspace with an eager call of twice the poses on the same stream: the replays
 must still read the workspace the capture recorded, which stays allocated.
 
-The third captures a forward that uses the stream's list of the rotation kernels' work items in
-reach (made by the warm-up of the same geometry), then runs forwards of five other geometries on
-the capture stream, which replace every list the stream keeps (four): the replays must still read
-the list the capture recorded, and the other geometries' forwards must equal the same calls on
-another stream.
+The third captures a forward on the tile-owner kernels that uses the stream's list of the tiles in
+the rotations' reach (made by the warm-up of the same geometry), then runs forwards of fourteen
+other geometries on the capture stream, which replace every list the stream keeps (twelve): the
+replays must still read the list the capture recorded, and the other geometries' forwards must equal
+the same calls on another stream.
 """
 import pytest
 import torch
+
+from torch_projectors import capi
 
 pytestmark = pytest.mark.gpu
 
@@ -157,7 +159,14 @@ def test_fourier_transforms_replayed_after_plan_eviction(gpu):
         assert _rel(back_g, back_e) <= 1e-6, f"replay {replay}: inverse {_rel(back_g, back_e):.3e}"
 
 
-def test_replay_after_the_forward_lists_turned_over(gpu):
+@pytest.fixture
+def tiles(gpu):
+    was = capi.lib().tp_set_gather_route(capi.ROUTE_TILES)
+    yield
+    capi.lib().tp_set_gather_route(was)
+
+
+def test_replay_after_the_forward_lists_turned_over(gpu, tiles):
     T = torch.ops.torch_projectors
     gen = torch.Generator().manual_seed(8100)
     P, n, os_, N = 24, 32, 2.0, 64
@@ -180,7 +189,9 @@ def test_replay_after_the_forward_lists_turned_over(gpu):
         proj_g = fwd(vol, rot, sh, n)
     torch.cuda.synchronize()
 
-    others = [(16, 64), (24, 64), (40, 64), (48, 64), (16, 32)]  # (projection size, volume size)
+    # (projection size, volume size): the list depends on the projection size
+    others = [(m, 64) for m in range(12, 64, 4) if m != n] + [(16, 32), (70, 32)]
+    assert len({m for m, _ in others}) > 12
     vols = {m: torch.randn(1, m, m, m // 2 + 1, generator=gen, dtype=torch.complex64).to(gpu) for m in (32, 64)}
     for replay in range(3):
         with torch.cuda.stream(stream):

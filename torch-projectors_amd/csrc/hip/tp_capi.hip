@@ -6,8 +6,8 @@
 // that are accumulated, and enqueues the kernels on the caller's stream.
 // The memory besides the caller's is kept per (device, stream) for the life
 // of the process: a small scratch area that the calls of the tiled kernels use
-// (tp::CallPoses: a summary of their poses and work counters), the last lists
-// of 3D work items, and the 3D scatters' workspace (pose bins, partial sums of
+// (tp::CallPoses: a summary of their poses and work counters), the
+// last lists of 3D forward tiles, and the 3D scatters' workspace (pose bins, partial sums of
 // split tiles).  Nothing is synchronised except where a call lists a new
 // geometry or outgrows that workspace.  tp_project_3d_to_2d_forw_noalloc uses a
 // static device array and neither list nor workspace.
@@ -159,19 +159,18 @@ constexpr double kMaxScatterPieces = double(1 << 17), kMaxGatherPieces = double(
 //     poses of 90 x 90 at oversampling 1.5, cubic forward and backward 1.59 -> 0.84 ms; 1000 poses of
 //     64 x 64 at 2, linear: backprojection 0.211 -> 0.124, projection with all gradients 0.549 -> 0.279 ms;
 //     1000 of 64 x 64 at 1, cubic backprojection 3.34 -> 0.65 ms.
-//   - in calls where that is 512 poses or more (and without `levels`: when the call can have no list
-//     of its pieces), one level of 40 voxels with `range` poses per piece: there the levels measured
+//   - in calls where that is 512 poses or more, one level of 40 voxels with `range` poses per piece: there the levels measured
 //     slower (the headline backprojection 1.33 -> 1.39 ms: less of the projections' rows is shared
 //     by the pieces that run together).
 tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const int org[3], const int edge[3],
-                         double stencil, double per_slot, double least, int64_t range, double most, bool levels) {
+                         double stencil, double per_slot, double least, int64_t range, double most) {
     constexpr double kSlots = 1024.0, kLongRange = 512.0;
     const double h = 0.25 * (edge[0] + edge[1] + edge[2] + 3.0 * stencil);
     const double vt = double(edge[0]) * edge[1] * edge[2], R = std::max(reach, h);
     const double cross =
         double(g.B) * double(g.P) * 2.0 * M_PI / vt * (h * h * h / 3.0 + h * (R * R - h * h) / 2.0);
     double target = std::max(least, cross / (kSlots * per_slot));
-    const bool one_level = !levels || target >= kLongRange;
+    const bool one_level = target >= kLongRange;
     if (one_level) target = double(range);
     tp::PoseSplit ps{};
     double r = one_level ? 40.0 : 16.0, p = 1.0;  // this level's half width; share of the poses that cross its tiles
@@ -185,19 +184,23 @@ tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const 
         int64_t tiles = 1;
         for (int a = 0; a < 3; ++a) {
             const double rc = std::min(r, reach);
-            v.lo[a] = std::max(0, int(std::floor((-rc - org[a]) / edge[a])));
-            const int hi = std::max(v.lo[a], std::min(n[a], int(std::floor((rc - org[a]) / edge[a])) + 1));
-            v.ext |= unsigned(hi - v.lo[a]) << (10 * a);
-            tiles *= hi - v.lo[a];
+            v.box.lo[a] = std::max(0, int(std::floor((-rc - org[a]) / edge[a])));
+            const int hi = std::max(v.box.lo[a], std::min(n[a], int(std::floor((rc - org[a]) / edge[a])) + 1));
+            v.box.ext |= unsigned(hi - v.box.lo[a]) << (10 * a);
+            tiles *= hi - v.box.lo[a];
         }
         total += double(g.B) * double(tiles) * double(k);
         if (total > most || k > tp::kMaxTilePieces || double(ps.pieces) + double(tiles) * double(k) > double(INT32_MAX))  // (twice as long until they fit)
-            return pose_split(g, reach, n, org, edge, stencil, per_slot / 2.0, 2.0 * target, 2 * int64_t(target), most,
-                              levels);
+            return pose_split(g, reach, n, org, edge, stencil, per_slot / 2.0, 2.0 * target, 2 * int64_t(target), most);
         v.k = int(k);
         v.pieces = int(tiles * k);
+        v.by_pieces = tp::divisor(unsigned(v.pieces));
+        v.by_k = tp::divisor(unsigned(k));
+        v.by_r = tp::divisor(unsigned(v.box.size(1)));
+        v.by_c = tp::divisor(unsigned(v.box.size(2)));
         ps.n = l + 1;
         ps.pieces += v.pieces;
+        ps.box = v.box;
         if (r >= reach) break;
         p = std::min(1.0, h / (r + 6.0));
     }
@@ -206,12 +209,7 @@ tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const 
 
 // The op a TileSpec is for: its pose ranges differ.
 enum class TileOp { project, gradients, backproject };
-// The pose ranges of a call's tile grids (forward, the other poses' wider forward grid, scatter): in
-// levels, and in the one level of a call without a list of its pieces.
-struct Splits {
-    tp::PoseSplit f[2], f2[2], s[2];
-};
-tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, Splits& sp) {
+tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, tp::ForwWorks& fw, tp::ScatterWork& sw) {
     constexpr int L = tp::kTileEdge;
     tp::TileSpec ts{};
     // radius bound of the active pixels: the cutoff disc, within the pixel grid
@@ -251,15 +249,14 @@ tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, Splits& sp) {
     const int nsc[3] = {ts.ntd, ts.ntr, ts.ntc}, osc[3] = {1 - half, 1 - half, 0},
               esc[3] = {tp::kScTD, tp::kScTR, tp::kScTC};
     const double flo = op == TileOp::project ? 64.0 : 32.0;
-    for (int i = 0; i < 2; ++i) {
-        const bool lv = i == 0;
-        sp.f[i] = pose_split(g, rho_unit, nf, of, ef, 0.0, 0.5, flo,
-                             op == TileOp::project ? forw_poses_per_range(g.os) : 512, kMaxGatherPieces, lv);
-        sp.f2[i] = pose_split(g, rho_unit, nf2, of2, ef, 0.0, 0.5, flo, 512, kMaxGatherPieces, lv);
-        sp.s[i] = pose_split(g, rho_unit, nsc, osc, esc, cubic ? 3.0 : 1.0, cubic ? 1.5 : 1.0, cubic ? 16.0 : 48.0,
-                             op == TileOp::backproject ? std::min<int64_t>(2048, std::max<int64_t>(512, g.P / 4)) : 512,
-                             kMaxScatterPieces, lv);
-    }
+    fw.rot.split =
+        pose_split(g, rho_unit, nf, of, ef, 0.0, 0.5, flo, op == TileOp::project ? forw_poses_per_range(g.os) : 512,
+                   kMaxGatherPieces);
+    fw.gen.split = pose_split(g, rho_unit, nf2, of2, ef, 0.0, 0.5, flo, 512, kMaxGatherPieces);
+    sw.split =
+        pose_split(g, rho_unit, nsc, osc, esc, cubic ? 3.0 : 1.0, cubic ? 1.5 : 1.0, cubic ? 16.0 : 48.0,
+                   op == TileOp::backproject ? std::min<int64_t>(2048, std::max<int64_t>(512, g.P / 4)) : 512,
+                   kMaxScatterPieces);
     ts.rho = float(rho);
     ts.rho_unit = float(rho_unit);
     ts.os = float(g.os);
@@ -436,17 +433,17 @@ struct StreamScratch {
     // until the process ends; growth is geometric, so these stay a small multiple of the last).
     bool bins_captured = false;
     std::vector<void*> bins_retired;
-    // Lists of work items (tp::TileSpec::flist, tp::SplitView::list) of the last few geometries; a
-    // list that a capture has used is retired in the same way.
+    // Lists of the forward tiles in reach (tp::ForwWork::list) of the last few geometries; a list
+    // that a capture has used is retired in the same way.
     struct ForwList {
         std::vector<int64_t> key;
-        tp::TileItem* p = nullptr;
+        tp::TileAt* p = nullptr;
         size_t cap = 0;
-        int64_t count = 0;
+        int n[tp::kSplitLevels + 1] = {};
         bool captured = false;
         uint64_t used = 0;
     };
-    ForwList flists[12];  // (a projection with gradients uses four)
+    ForwList flists[12];  // (the pose count of a call decides between at most five per geometry)
     uint64_t flist_tick = 0;
     std::vector<void*> flist_retired;
 };
@@ -542,13 +539,13 @@ struct CallScratch {
         if (capturing) area->bins_captured = true;
         return area->bins;
     }
-    // The list of work items with this key (everything it depends on), or nullptr (the kernels then
-    // take every work item of their grid, split in one level).  The area keeps the last twelve; another
-    // one is listed on the host (`build` appends it) and copied in on the call's stream, which is then
-    // synchronised (once per new key).  A stream under graph capture takes a list that the area holds,
-    // else none, and a list that a capture has used is retired, never rewritten or freed.
+    // The list of tiles with this key (everything it depends on), or nullptr (the kernels then take
+    // every work item of their grid).  The area keeps the last twelve; another one is made on the host
+    // (`build`) and copied in on the call's stream, which is then synchronised (once per new key).  A
+    // stream under graph capture takes a list that the area holds, else none, and a list that a capture
+    // has used is retired, never rewritten or freed.
     template <typename F>
-    const tp::TileItem* item_list(const std::vector<int64_t>& key, hipStream_t st, int64_t& count, F&& build) {
+    const StreamScratch::ForwList* tile_list(const std::vector<int64_t>& key, hipStream_t st, F&& build) {
         if (static_area || !area) return nullptr;
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
@@ -561,15 +558,16 @@ struct CallScratch {
             if (f.p && f.key == key) {
                 f.used = ++area->flist_tick;
                 if (capturing) f.captured = true;
-                count = f.count;
-                return f.p;
+                return &f;
             }
             if (!victim || (victim->p && (!f.p || f.used < victim->used))) victim = &f;
         }
         if (capturing) return nullptr;
-        std::vector<tp::TileItem> host;
-        if (!build(host) || host.empty()) return nullptr;
-        const size_t need = host.size() * sizeof(tp::TileItem);
+        std::vector<tp::TileAt> host;
+        int n[tp::kSplitLevels + 1];
+        build(host, n);
+        if (host.empty()) return nullptr;
+        const size_t need = host.size() * sizeof(tp::TileAt);
         // queued work may still read the list that is replaced
         if (hipStreamSynchronize(st) != hipSuccess) {
             (void)hipGetLastError();
@@ -599,10 +597,9 @@ struct CallScratch {
             return nullptr;
         }
         f.key = key;
-        f.count = int64_t(host.size());
+        std::copy(n, n + tp::kSplitLevels + 1, f.n);
         f.used = ++area->flist_tick;
-        count = f.count;
-        return f.p;
+        return &f;
     }
     int get(hipStream_t st) {
         if (p) return TP_OK;
@@ -645,42 +642,18 @@ struct CallScratch {
 };
 
 // Summary of the call's poses for its tiled kernels (tp::launch_call_poses), which also clears the
-// counts of the pose bins that plan_scatter laid out in ts (if any).
+// counts of the pose bins `bins` (if any).
 int call_poses(int dim, const tp::Geom& g, const void* rot, float rho_unit, CallScratch& sc, hipStream_t s,
-               const tp::TileSpec* ts = nullptr) {
+               const tp::BinGrid& bins = {}) {
     TP_TRY(sc.get(s));
-    int* zero = ts && ts->sbins.list ? ts->sbins.count : nullptr;
-    const int64_t nzero = zero ? g.B_rot * int64_t(ts->sbins.n) : 0;
+    int* zero = bins.list ? bins.count : nullptr;
+    const int64_t nzero = zero ? g.B_rot * int64_t(bins.n) : 0;
     return launched(tp::launch_call_poses(dim, g.B_rot * g.P, rot, rho_unit, sc.p, s, zero, nzero),
                     "pose summary launch");
 }
 
-// A split as the kernels take it: its pieces listed when it has several levels, or the one-level
-// split (`ps` then becomes that) when the call's (device, stream) area can hold no list.
-tp::SplitView split_view(tp::PoseSplit& ps, const tp::PoseSplit& one, int64_t B, CallScratch& sc, hipStream_t s) {
-    const tp::TileItem* list = nullptr;
-    if (ps.n > 1) {
-        std::vector<int64_t> key{1, B};
-        for (int l = 0; l < ps.n; ++l) {
-            const tp::PoseSplit::Level& v = ps.lv[l];
-            key.insert(key.end(), {v.lo[0], v.lo[1], v.lo[2], int64_t(v.ext), v.k});
-        }
-        int64_t count = 0;
-        list = sc.item_list(key, s, count, [&](std::vector<tp::TileItem>& out) {
-            tp::split_items(ps, B, out);
-            return true;
-        });
-        if (!list) ps = one;
-    }
-    tp::SplitView v{};
-    if (ps.n > 0) v.box = ps.lv[ps.n - 1];
-    v.pieces = ps.pieces;
-    v.list = list;
-    return v;
-}
-
 // Workspace of the tiled 3D scatter for this call: the slots of the split tiles' pieces
-// (tp::TileSpec::part), and the pose bins of its tile grid (tp::BinGrid) in 2 x 2 x 2 tiles, which
+// (tp::ScatterWork::part), and the pose bins of its tile grid (tp::BinGrid) in 2 x 2 x 2 tiles, which
 // plan_scatter lays out (the pose summary then clears their counts) and fill_bins fills after the
 // summary.  No bins below kBinsMinPoses poses, from 65536 poses (list entries are 16-bit), beyond
 // kBinsMaxBytes or tp::kBinMaxGroups workgroups of the pre-pass; without a workspace (a failed
@@ -688,12 +661,10 @@ tp::SplitView split_view(tp::PoseSplit& ps, const tp::PoseSplit& one, int64_t B,
 // of the call's poses itself.
 constexpr int64_t kBinsMinPoses = 16;
 constexpr size_t kBinsMaxBytes = size_t(1) << 30;
-int plan_scatter(const tp::Geom& g, tp::TileSpec& ts, Splits& sp, bool weights, CallScratch& sc, hipStream_t s) {
-    ts.sbins = tp::BinGrid{};
+int plan_scatter(const tp::Geom& g, const tp::TileSpec& ts, tp::ScatterWork& sw, bool weights, CallScratch& sc, hipStream_t s) {
     TP_TRY(sc.get(s));
-    ts.ssplit = split_view(sp.s[0], sp.s[1], g.B, sc, s);
     auto align = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t slots = align(size_t(g.B) * size_t(ts.ssplit.pieces) * size_t(tp::slot_bytes(weights)));
+    const size_t slots = align(size_t(g.B) * size_t(sw.split.pieces) * size_t(tp::slot_bytes(weights)));
     tp::BinGrid sb{};
     sb.nb[0] = (ts.ntc + 1) / 2;
     sb.nb[1] = (ts.ntr + 1) / 2;
@@ -707,21 +678,20 @@ int plan_scatter(const tp::Geom& g, tp::TileSpec& ts, Splits& sp, bool weights, 
     const size_t need = slots + counts + lists;
     char* w = need ? static_cast<char*>(sc.bins(need, s)) : nullptr;
     if (!w) {
-        ts.ssplit = tp::SplitView{};
-        sp.s[0] = tp::PoseSplit{};
+        sw.split = tp::PoseSplit{};
         return TP_OK;
     }
-    ts.part = w;
+    sw.part = w;
     if (counts) {
         sb.count = reinterpret_cast<int*>(w + slots);
         sb.list = reinterpret_cast<unsigned short*>(w + slots + counts);
-        ts.sbins = sb;
+        sw.bins = sb;
     }
     return TP_OK;
 }
-int fill_bins(bool cubic, const tp::Geom& g, const tp::TileSpec& ts, const void* rot, CallScratch& sc,
+int fill_bins(bool cubic, const tp::Geom& g, const tp::TileSpec& ts, const tp::ScatterWork& sw, const void* rot, CallScratch& sc,
               hipStream_t s) {
-    if (!ts.sbins.list) return TP_OK;
+    if (!sw.bins.list) return TP_OK;
     // a bin's box holds its tiles' box-1 boxes (the tile dilated by the stencil and the slack) with
     // half a voxel to spare
     const float half = float(g.N / 2), pad = 0.5f;
@@ -729,29 +699,39 @@ int fill_bins(bool cubic, const tp::Geom& g, const tp::TileSpec& ts, const void*
     const tp::BinBox bb{{0.f, -half + 1.f, -half + 1.f},
                         {2.f * tp::kScTC, 2.f * tp::kScTR, 2.f * tp::kScTD},
                         sl + ts.eps + pad, sh + ts.eps + pad, ts.rho_unit + 1.0f};
-    return launched(tp::launch_pose_bins(g, rot, ts.sbins, bb, sc.p, s), "pose-bin launch");
+    return launched(tp::launch_pose_bins(g, rot, sw.bins, bb, sc.p, s), "pose-bin launch");
 }
 
-// The forward kernels' splits, and the rotation kernels' work items in reach (tp::TileSpec::flist)
-// when the call's (device, stream) area can hold them.
-int use_forw_lists(const tp::Geom& g, tp::TileSpec& ts, Splits& sp, CallScratch& sc, hipStream_t s) {
+// The work items of the forward kernels for rotations, with the list of the tiles in reach
+// (tp::ForwWork::list) when the call's (device, stream) area can hold it.
+int use_forw_tiles(const tp::Geom& g, const tp::TileSpec& ts, tp::ForwWorks& fw, CallScratch& sc, hipStream_t s) {
     TP_TRY(sc.get(s));
+    const tp::PoseSplit ps = fw.rot.split;
+    fw.rot.list = nullptr;
+    fw.rot.count = fw.gen.count = g.B * (ps.pieces + int64_t(ts.nt) * ts.nt * ts.ntfd);
+    if (fw.rot.count > int64_t(INT32_MAX)) return TP_OK;
     uint32_t rho_bits = 0, eps_bits = 0;
     std::memcpy(&rho_bits, &ts.rho_unit, 4);
     std::memcpy(&eps_bits, &ts.eps, 4);
-    std::vector<int64_t> key{0, g.B, ts.nt, ts.org, ts.ntfd, ts.orgd, int64_t(rho_bits), int64_t(eps_bits)};
-    for (int l = 0; l < sp.f[0].n; ++l) {
-        const tp::PoseSplit::Level& v = sp.f[0].lv[l];
-        key.insert(key.end(), {v.lo[0], v.lo[1], v.lo[2], int64_t(v.ext), v.k});
+    std::vector<int64_t> key{ts.nt, ts.org, ts.ntfd, ts.orgd, int64_t(rho_bits), int64_t(eps_bits)};
+    for (int l = 0; l < ps.n; ++l) {
+        const tp::PoseSplit::Box& v = ps.lv[l].box;
+        key.insert(key.end(), {v.lo[0], v.lo[1], v.lo[2], int64_t(v.ext)});
     }
-    ts.fsplit2 = split_view(sp.f2[0], sp.f2[1], g.B, sc, s);
-    ts.fsplit.pieces = sp.f[0].pieces;  // (the grid's item count, should the list have it)
-    int64_t count = 0;
-    ts.flist = sc.item_list(key, s, count, [&](std::vector<tp::TileItem>& out) {
-        return tp::forw_reach_items(g, ts, sp.f[0], out) <= int64_t(INT32_MAX);
+    const StreamScratch::ForwList* f = sc.tile_list(key, s, [&](std::vector<tp::TileAt>& out, int* n) {
+        tp::forw_reach_tiles(ts, ps, out, n);
     });
-    ts.fcount = ts.flist ? count : 0;
-    if (!ts.flist) ts.fsplit = split_view(sp.f[1], sp.f[1], g.B, sc, s);
+    if (!f) return TP_OK;
+    fw.rot.list = f->p;
+    fw.rot.count = 0;
+    unsigned first = 0;
+    for (int l = 0; l <= tp::kSplitLevels; ++l) {
+        const unsigned k = l < ps.n ? unsigned(ps.lv[l].k) : 1u, tiles = unsigned(f->n[l]);
+        fw.rot.reach[l] = tp::ReachLevel{unsigned(fw.rot.count), first, tiles * k, k, tp::divisor(tiles * k),
+                                         tp::divisor(k)};
+        fw.rot.count += g.B * int64_t(tiles) * k;
+        first += tiles;
+    }
     return TP_OK;
 }
 
@@ -785,11 +765,12 @@ int project_forw(int dim, int dtype, const void* rec, int64_t B, int64_t D, int6
         return launched(tp::launch_project_forw(dim, kdt, cubic, g, rec, rot, shifts, out, s), "projection launch");
     }
     if (tiles) {
-        Splits sp{};
-        tp::TileSpec ts = tile_spec(g, cubic, TileOp::project, sp);
+        tp::ForwWorks fw{};
+        tp::ScatterWork sw{};
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::project, fw, sw);
+        TP_TRY(use_forw_tiles(g, ts, fw, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s));
-        TP_TRY(use_forw_lists(g, ts, sp, sc, s));
-        TP_TRY(launched(tp::launch_project3_forw_tiled(cubic, g, ts, rec, rot, shifts, out, sc.p, 0, s, rec_half),
+        TP_TRY(launched(tp::launch_project3_forw_tiled(cubic, g, ts, fw, rec, rot, shifts, out, sc.p, 0, s, rec_half),
                         "tiled projection launch"));
         return launched(tp::launch_project_forw(dim, kdt, cubic, g, rec, rot, shifts, out, s, true),
                         "projection launch");
@@ -844,18 +825,20 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     // (complex-half volumes have no per-pixel gradients without the scatter)
     const bool per_pixel =
         (tiles || tiles2) && (grot || gshift) && !rec_half && takes_per_pixel(small_gradients(dim, g, cubic));
+    const bool tiled_gradients = (grot || gshift) && !per_pixel;
     if (tiles) {
-        Splits sp{};
-        tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, sp);
-        TP_TRY(plan_scatter(g, ts, sp, false, sc, s));
-        TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, &ts));
-        TP_TRY(fill_bins(cubic, g, ts, rot, sc, s));
-        if (!per_pixel) TP_TRY(use_forw_lists(g, ts, sp, sc, s));
-        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 1, g, ts, sp.s[0], gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
+        tp::ForwWorks fw{};
+        tp::ScatterWork sw{};
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, fw, sw);
+        TP_TRY(plan_scatter(g, ts, sw, false, sc, s));
+        if (tiled_gradients) TP_TRY(use_forw_tiles(g, ts, fw, sc, s));
+        TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, sw.bins));
+        TP_TRY(fill_bins(cubic, g, ts, sw, rot, sc, s));
+        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 1, g, ts, sw, gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
                                                   s),
                         "tiled reconstruction-gradient launch"));
-        if (!per_pixel)
-            TP_TRY(launched(tp::launch_grads3_tiled(cubic, g, ts, gproj, rec, rot, shifts, grot, gshift, sc.p, 1, s,
+        if (tiled_gradients)
+            TP_TRY(launched(tp::launch_grads3_tiled(cubic, g, ts, fw, gproj, rec, rot, shifts, grot, gshift, sc.p, 1, s,
                                                     rec_half),
                             "tiled rotation/shift-gradient launch"));
     }
@@ -865,7 +848,7 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
         TP_TRY(launched(tp::launch_scatter2_tiled(cubic, 1, g, ts, gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
                                                   s),
                         "tiled reconstruction-gradient launch"));
-        if (!per_pixel)
+        if (tiled_gradients)
             TP_TRY(launched(tp::launch_gather2_tiled(cubic, 1, g, ts, rec, nullptr, rot, shifts, nullptr, nullptr,
                                                      gproj, grot, gshift, sc.p, 1, s, rec_half),
                             "tiled rotation/shift-gradient launch"));
@@ -903,12 +886,13 @@ int backproject_forw(int dim, int dtype, const void* proj, int64_t B, int64_t P,
     TP_TRY(need(rot, "rotations"));
     CallScratch sc;
     if (tiles) {
-        Splits sp{};
-        tp::TileSpec ts = tile_spec(g, cubic, TileOp::backproject, sp);
-        TP_TRY(plan_scatter(g, ts, sp, weights != nullptr, sc, s));
-        TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, &ts));
-        TP_TRY(fill_bins(cubic, g, ts, rot, sc, s));
-        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 0, g, ts, sp.s[0], proj, weights, rot, shifts, data, wrec, sc.p, 0, s),
+        tp::ForwWorks fw{};
+        tp::ScatterWork sw{};
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::backproject, fw, sw);
+        TP_TRY(plan_scatter(g, ts, sw, weights != nullptr, sc, s));
+        TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, sw.bins));
+        TP_TRY(fill_bins(cubic, g, ts, sw, rot, sc, s));
+        TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 0, g, ts, sw, proj, weights, rot, shifts, data, wrec, sc.p, 0, s),
                         "tiled backprojection launch"));
     }
     if (tiles2) {
@@ -956,11 +940,12 @@ int backproject_back(int dim, int dtype, const void* gdata, const void* gw, int6
         TP_TRY(zero(gweights, re_words(dtype, g.B * g.P * int64_t(g.npix)), s));
     }
     if (tiles) {
-        Splits sp{};
-        tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, sp);
+        tp::ForwWorks fw{};
+        tp::ScatterWork sw{};
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, fw, sw);
+        TP_TRY(use_forw_tiles(g, ts, fw, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s));
-        TP_TRY(use_forw_lists(g, ts, sp, sc, s));
-        TP_TRY(launched(tp::launch_bpback3_tiled(cubic, g, ts, gdata, gw, proj, rot, shifts, gproj, gweights, grot,
+        TP_TRY(launched(tp::launch_bpback3_tiled(cubic, g, ts, fw, gdata, gw, proj, rot, shifts, gproj, gweights, grot,
                                                  gshift, sc.p, 0, s),
                         "tiled backprojection backward launch"));
     }

@@ -66,40 +66,59 @@ struct BinBox {
 
 // Pose ranges of a 3D tile grid.  Tiles near the origin are crossed by every pose, tiles at distance
 // x by about h / x of them (h a tile's half width), so the tiles within nested boxes around the origin
-// are split into pieces, more of them further in: level l (0 innermost) holds the tiles [lo, hi) along
-// d, r, c that no inner level holds, k pieces each.  Tiles outside every level are one piece.
+// are split into pieces, more of them further in: level l (0 innermost) holds the tiles of its box
+// along d, r, c that no inner level holds, k pieces each.  Tiles outside every level are one piece.
+// Work items 0 .. B * pieces - 1 are the levels' pieces (level by level, batch item by batch item, tile
+// by tile; the tiles that an inner level holds are skipped), then come the tiles of the whole grid,
+// where those of `box`, the outermost level, are skipped.  The kernels index the levels in the kernel
+// arguments' memory (held in registers, all three cost 60 of the scalar ones; a device list of the
+// pieces, which depends on the pose count, had to be made anew for nearly every other count).
 constexpr int kSplitLevels = 3;
+// Division of n < 2^31 by d through a product (exact: m = floor(2^(31 + s) / d) + 1 with 2^s >= d is
+// off by at most d <= 2^s from 2^(31 + s) / d times d).  The kernels decode a work item per workgroup
+// in scalar registers with it, where the compiler's vector division waits for itself several times.
+struct Divisor {
+    unsigned m, s;  // m = 0: d is 1
+    __host__ __device__ unsigned of(unsigned n) const {
+        return m ? unsigned((uint64_t(n) * m) >> 32) >> (s - 1) : n;
+    }
+};
+inline Divisor divisor(unsigned d) {
+    if (d <= 1) return Divisor{0, 0};
+    unsigned s = 1;
+    while ((uint64_t(1) << s) < d) ++s;
+    return Divisor{unsigned((uint64_t(1) << (31 + s)) / d + 1), s};
+}
 struct PoseSplit {
-    int n;  // levels in use
-    struct Level {
+    struct Box {
         int lo[3];       // tile box along d, r, c: first tile
         unsigned ext;    // and its extents, 10 bits each
-        int k;           // pieces per tile
-        int pieces;      // k times the box's tiles: work items of one batch item
         __host__ __device__ int size(int a) const { return int(ext >> (10 * a)) & 1023; }
         __host__ __device__ bool holds(int d, int r, int c) const {
             return unsigned(d - lo[0]) < unsigned(size(0)) && unsigned(r - lo[1]) < unsigned(size(1)) &&
                    unsigned(c - lo[2]) < unsigned(size(2));
         }
+    };
+    struct Level {
+        Box box;
+        int k;       // pieces per tile
+        int pieces;  // k times the box's tiles: work items of one batch item
+        Divisor by_pieces, by_k, by_r, by_c;  // by the pieces, k, and the box's extents along r and c
     } lv[kSplitLevels];  // (pieces 0 past the levels in use)
+    int n;               // levels in use
     int pieces;          // of every level, for one batch item
+    Box box;             // of the outermost level
 };
-// A work item of the rotation kernels' forward tile grid, decoded: piece j of k of tile (d, r, c) of
-// batch item b.
-struct alignas(16) TileItem {
-    unsigned short d, r, c, k;
-    int b, j;
-};
-static_assert(sizeof(TileItem) == 16, "one 16-byte load per workgroup");
 constexpr int kMaxTilePieces = 65535;
-// A split as the tile kernels see it: work items 0 .. B * pieces - 1 are the levels' pieces, listed in
-// device memory (level by level, batch item by batch item; the levels themselves in kernel arguments
-// cost the kernels 60 scalar registers), or without a list the pieces of one level, `box`.  Then come
-// the tiles of the whole grid, where those of `box`, the outermost level, are skipped.
-struct SplitView {
-    PoseSplit::Level box;
-    int pieces;
-    const TileItem* list;
+// A tile of the forward grid (ForwWork::list).
+struct alignas(8) TileAt {
+    unsigned short d, r, c, pad;
+};
+// The listed tiles of one level, or the whole ones: their first work item, first list entry, work items
+// per batch item and pieces per tile.
+struct ReachLevel {
+    unsigned begin, first, per, k;
+    Divisor by_per, by_k;
 };
 
 // Bytes of one split tile's piece in the scatter's workspace.
@@ -107,14 +126,37 @@ __host__ __device__ constexpr int64_t slot_bytes(bool weights) {
     return int64_t(kScTC) * kScTR * kScTD * (weights ? 12 : 8);
 }
 
+// The `count` work items of the 3D gather kernel for rotations: those of its grid and `split`, or, with
+// a list of the grid's tiles that the rotations' samples can reach (forw_reach_tiles), the pieces of its
+// tiles (about half of the headline's tiles lie outside that sphere).  For the kernel of the other tiled
+// poses, `split` of their grid (it finds its items itself) and the rotation grid's number of items.
+struct ForwWork {
+    const TileAt* list;
+    int64_t count;
+    union {
+        PoseSplit split;                       // without a list
+        ReachLevel reach[kSplitLevels + 1];    // with one: by level, the whole tiles last
+    };
+};
+struct ForwWorks {
+    ForwWork rot, gen;
+};
+// The split of a scatter's grid, its pose bins (list null: none), and the workspace of its split tiles: a slot
+// of slot_bytes per piece (B * split.pieces: the tile's values, then its weights), which k_finish3 sums
+// into the volume.
+struct ScatterWork {
+    PoseSplit split;
+    BinGrid bins;
+    char* part;
+};
+// (a kernel's arguments carry little more than it reads: 512 bytes more in each of a forward's cost 4096
+// poses of 128 x 128 1.3 of 290 us)
 struct TileSpec {
     int nt, org;              // forward: tiles along c and r, and the signed origin of the grid there,
                               // laid out for unit-scale poses (|x| <= rho_unit + 1)
     int ntfd, orgd;           // forward: the same along d (tiles of kTileEdgeD)
     int nt2, org2, ntfd2, orgd2;  // forward: the grid that the other tiled poses reach (|x| <= rho)
-    SplitView fsplit, fsplit2;    // forward: pose ranges on the two grids
     int ntd, ntr, ntc;        // scatter: tiles along d, r, c of the stored half volume
-    SplitView ssplit;         // scatter: pose ranges
     float rho;                // bound on |x| of every active sample of a tiled pose (singular values <= kScaleMax)
     float rho_unit;           // the same for singular values <= 1, less the +1 voxel margin
     float eps;                // slack (voxels) added to every enumeration box
@@ -126,23 +168,12 @@ struct TileSpec {
     // at most 4)
     int kp_forw, kp_scatter;
     bool os_exact;            // float(os) == os: c * os can be formed in float exactly as in double
-    BinGrid sbins;            // pose bins of the scatter tile grid (list null: none)
-    // forward: the rotation kernels' work items whose tiles the rotations' samples can reach, in
-    // work-item order (forw_reach_items), fcount of them; flist null: every work item of the grid
-    // (about half of the headline's tiles lie outside that sphere)
-    const TileItem* flist;
-    int64_t fcount;
-    // scatter: a slot of slot_bytes per piece of the split tiles (B * ssplit.pieces: the tile's values, then
-    // its weights), which k_finish3 sums into the volume
-    char* part;
 };
 
-// The pieces of split ps in work-item order, appended to `out` (k = 0: a tile that an inner level
-// holds, which the kernels skip).  Host code, for SplitView::list.
-void split_items(const PoseSplit& ps, int64_t B, std::vector<TileItem>& out);
-// The work items of the rotation kernels' forward tile grid (ts's nt, ntfd and split ps) whose tiles lie within rho_unit + 1 (and a margin) of the origin, in increasing order,
-// appended to `out`; returns the grid's item count.  Host code, for TileSpec::flist.
-int64_t forw_reach_items(const Geom& g, const TileSpec& ts, const PoseSplit& ps, std::vector<TileItem>& out);
+// The tiles of the forward grid (ts's nt, ntfd) that lie within rho_unit + 1 (and a margin) of the
+// origin, appended to `out`: those of ps's levels, innermost first, then the others (n: their counts).
+// Their order depends on the levels' boxes but not on the pose count.  Host code, for ForwWork::list.
+void forw_reach_tiles(const TileSpec& ts, const PoseSplit& ps, std::vector<TileAt>& out, int n[kSplitLevels + 1]);
 
 // Tile-owner kernels of the fp32 2D operators (tp_tiled2d.hip).
 constexpr int kTile2C = 32, kTile2R = 16;  // scatter tile edges (c, r): fp64 accumulators
@@ -231,24 +262,23 @@ hipError_t launch_backproject_forw(int dim, int dt, bool cubic, const Geom& g, c
 // launch_call_poses has filled *cp; `gl` (< kTiledPairs) picks their
 // counters, distinct for the kernel pairs of one call.
 // `rec_half`: the volume is stored as complex half and widened to fp32 on load.
-hipError_t launch_project3_forw_tiled(bool cubic, const Geom& g, const TileSpec& ts, const void* rec,
+hipError_t launch_project3_forw_tiled(bool cubic, const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* rec,
                                       const void* rot, const void* shifts, void* out, CallPoses* cp, int gl,
                                       hipStream_t s, bool rec_half = false);
 // Rotation/shift gradients of project_3d_to_2d_back for tiled poses, added
 // into zero-filled grot / gshift (either may be null); `rec_half` as for the forward.
-hipError_t launch_grads3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const void* gproj, const void* rec,
+hipError_t launch_grads3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* gproj, const void* rec,
                                const void* rot, const void* shifts, void* grot, void* gshift, CallPoses* cp, int gl,
                                hipStream_t s, bool rec_half = false);
 // backproject_2d_to_3d_back for tiled poses into zero-filled outputs:
 // grad_projections from grad_data_rec, grad_weights from grad_weight_rec (when
 // both gw and gweights are given), rotation/shift gradients (either may be null).
-hipError_t launch_bpback3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const void* gdata, const void* gw,
+hipError_t launch_bpback3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* gdata, const void* gw,
                                 const void* proj, const void* rot, const void* shifts, void* gproj, void* gweights,
                                 void* grot, void* gshift, CallPoses* cp, int gl, hipStream_t s);
 // mode 0: backprojection into data (+ weights), with the x = 0 Hermitian completion;
 // mode 1: reconstruction gradient of the projection.
-// `ps`: the split of ts.ssplit.
-hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src,
+hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const ScatterWork& sw, const void* src,
                                  const void* weights, const void* rot, const void* shifts, void* dst, void* wdst,
                                  CallPoses* cp, int gl, hipStream_t s);
 

@@ -39,7 +39,7 @@
 // comes in two instantiations:
 //   GEN = false  rotations (columns orthonormal to kRotationTol), one
 //                workgroup per work item over the grid their samples reach
-//                (the forward family's: per work item of TileSpec::flist,
+//                (the forward family's: per work item of ForwWork::list,
 //                the tiles within that reach, when the C ABI has the list);
 //   GEN = true   the other tiled poses (scaled, anisotropically magnified or
 //                sheared matrices), launched after the first on a smaller
@@ -266,25 +266,64 @@ struct Item {
     int j, k;   // piece j of k of the tile's poses
     bool skip;  // a split tile
 };
-__device__ __forceinline__ Item listed_item(const TileItem* __restrict__ list, int64_t w) {
-    const TileItem f = list[w];
-    return Item{f.b, f.d, f.r, f.c, f.j, f.k, f.k == 0};
+// The decoding of a work item into its tile and poses is scalar arithmetic on tables that are constant
+// during the kernel, loaded where it needs them.
+template <typename T> using Constant = const __attribute__((address_space(4))) T;
+template <typename T, typename S> __device__ __forceinline__ T scalar_load(S* p) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    T v;
+    Constant<unsigned>* q = (Constant<unsigned>*)p;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) reinterpret_cast<unsigned*>(&v)[i] = q[i];
+    return v;
+}
+// The kernel's first argument, of type T, where it stands in memory.  As an ordinary argument, its fields
+// and what the decoding makes of them are loaded at the kernel's start and kept in scalar registers
+// (spilled, most of them) throughout its loop over work items: a forward of 4096 poses of 128 x 128 took
+// 1.3 % longer.
+template <typename T> __device__ __forceinline__ Constant<T>* first_argument() {
+    Constant<T>* p = (Constant<T>*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));  // (not the same pointer as before: nothing read from it is)
+    return p;
+}
+// Work item w of the rotation kernels' list of tiles in reach (ForwWork::list).
+__device__ __forceinline__ Item reach_item(Constant<ForwWork>* fw, int64_t w) {
+    const unsigned u = unsigned(w);
+    int l = 0;
+#pragma unroll
+    for (int i = 1; i <= kSplitLevels; ++i) l += u >= fw->reach[i].begin;
+    const ReachLevel v = scalar_load<ReachLevel>(&fw->reach[l]);
+    const unsigned n = u - v.begin, b = v.by_per.of(n), q = n - b * v.per, t = v.by_k.of(q);
+    const TileAt f = scalar_load<TileAt>(fw->list + (v.first + t));
+    return Item{int64_t(b), f.d, f.r, f.c, int(q - t * v.k), int(v.k), false};
 }
 __device__ __forceinline__ Item item_of(int64_t w, int64_t B, int nd, int nr, int nc, int offd, int off,
-                                        const SplitView& sp) {
+                                        Constant<PoseSplit>* sp) {
     Item it;
-    const int64_t split = B * sp.pieces;
-    const PoseSplit::Level& v = sp.box;
+    const int64_t split = B * sp->pieces;
     if (w < split) {
-        if (sp.list) return listed_item(sp.list, w);
-        it.b = w / sp.pieces;
-        const int q = int(w - it.b * sp.pieces), t = q / v.k, nc_ = v.size(2), nr_ = v.size(1);
-        it.j = q - t * v.k;
+        unsigned u = unsigned(w);  // (split < 2^31: pose_split)
+        int l = 0;
+#pragma unroll
+        for (int i = 0; i + 1 < kSplitLevels; ++i) {
+            const unsigned span = unsigned(B) * unsigned(sp->lv[i].pieces);
+            if (l == i && u >= span) {
+                u -= span;
+                ++l;
+            }
+        }
+        const PoseSplit::Level v = scalar_load<PoseSplit::Level>(&sp->lv[l]);
+        PoseSplit::Box in{};
+        if (l > 0) in = scalar_load<PoseSplit::Box>(&sp->lv[l - 1].box);  // (the boxes are nested: the next one in holds the others)
+        const unsigned b = v.by_pieces.of(u), q = u - b * unsigned(v.pieces), t = v.by_k.of(q), tr = v.by_c.of(t),
+                       td = v.by_r.of(tr);
+        it.b = b;
+        it.j = int(q - t * unsigned(v.k));
         it.k = v.k;
-        it.kc = v.lo[2] + t % nc_;
-        it.kr = v.lo[1] + (t / nc_) % nr_;
-        it.kd = v.lo[0] + t / (nc_ * nr_);
-        it.skip = false;
+        it.kc = v.box.lo[2] + int(t - tr * unsigned(v.box.size(2)));
+        it.kr = v.box.lo[1] + int(tr - td * unsigned(v.box.size(1)));
+        it.kd = v.box.lo[0] + int(td);
+        it.skip = in.holds(it.kd, it.kr, it.kc);
     } else {
         const int64_t per_b = int64_t(nd) * nr * nc;
         w -= split;
@@ -295,11 +334,11 @@ __device__ __forceinline__ Item item_of(int64_t w, int64_t B, int nd, int nr, in
         it.kd = offd + t / (nc * nr);
         it.j = 0;
         it.k = 1;
-        it.skip = v.holds(it.kd, it.kr, it.kc);
+        it.skip = scalar_load<PoseSplit::Box>(&sp->box).holds(it.kd, it.kr, it.kc);
     }
     return it;
 }
-// The same in scalar registers (every lane holds the same item; a listed one comes by a vector load).
+// The same in scalar registers (every lane holds the same item).
 __device__ __forceinline__ Item uniform(Item it) {
     it.kd = __builtin_amdgcn_readfirstlane(it.kd);
     it.kr = __builtin_amdgcn_readfirstlane(it.kr);
@@ -307,6 +346,7 @@ __device__ __forceinline__ Item uniform(Item it) {
     it.j = __builtin_amdgcn_readfirstlane(it.j);
     it.k = __builtin_amdgcn_readfirstlane(it.k);
     it.b = __builtin_amdgcn_readfirstlane(int(it.b));
+    it.skip = __builtin_amdgcn_readfirstlane(int(it.skip));
     return it;
 }
 // Start of piece j of k of n poses.
@@ -566,7 +606,7 @@ constexpr int forw_waves_per_eu() {
 template <bool CUBIC, int KP, bool OSX, int GMODE = 0, bool RS = true, bool WG = false, typename VS = float,
           bool GEN = false>
 __global__ __launch_bounds__(kForwThreads)
-__attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>()))) void k_forw3_tiled(Geom g, TileSpec ts, const Cx<VS>* __restrict__ rec,
+__attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>()))) void k_forw3_tiled(ForwWork fw, Geom g, TileSpec ts, const Cx<VS>* __restrict__ rec,
                                                         const float* __restrict__ rot,
                                                         const float* __restrict__ shifts,
                                                         Cx<float>* __restrict__ out, CallPoses* __restrict__ cp,
@@ -626,7 +666,6 @@ __attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>())))
     const bool all_rot = !GEN && call_flag(&cp->all_rot);
     float rho_k = ts.rho_unit + 1.0f;
     int nt = ts.nt, ntd = ts.ntfd, org = ts.org, orgd = ts.orgd;
-    const SplitView& ps = GEN ? ts.fsplit2 : ts.fsplit;
     int off = 0, offd = 0;  // first tile of the part of the wide grid that the reach needs
     if constexpr (GEN) {
         rho_k = fminf(ts.rho, cp->gen_reach);
@@ -640,11 +679,7 @@ __attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>())))
         orgd = ts.orgd2;
     }
     const float rho2 = rho_k * rho_k;
-    int64_t items = g.B * (ps.pieces + int64_t(nt) * nt * ntd);
-    // rotations: the slots may index the list of the work items in reach (the others' workgroups
-    // would only start and leave)
-    const TileItem* __restrict__ flist = GEN ? nullptr : ts.flist;
-    if (flist) items = ts.fcount;
+    const int64_t items = GEN ? g.B * (fw.split.pieces + int64_t(nt) * nt * ntd) : fw.count;
     const float cut2 = float(g.cut2);
     const int N = g.N, H = g.H;
     // (GEN: the grid holds a quarter of the rotation kernel's slots and steps over the rest)
@@ -653,7 +688,9 @@ __attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>())))
         const int64_t slot_i = sl.s;
         const int64_t wi = xcd_item<kRunForw>(slot_i);
         if (wi >= items) continue;
-        const Item it = uniform(flist ? listed_item(flist, wi) : item_of(wi, g.B, ntd, nt, nt, offd, off, ps));
+        Constant<ForwWork>* const work = first_argument<ForwWork>();
+        const Item it = uniform(!GEN && work->list ? reach_item(work, wi)
+                                                   : item_of(wi, g.B, ntd, nt, nt, offd, off, &work->split));
         if (it.skip) continue;
         const int64_t b = it.b;
         const int tc = org + it.kc * L, tr = org + it.kr * L, td = orgd + it.kd * LD;
@@ -1059,7 +1096,7 @@ __device__ __forceinline__ void scatter_sample(const Geom& g, const Slot& sd, in
 // MODE 0: backprojection, v = proj * conj(phase(r, c)), optional weights.
 // MODE 1: reconstruction gradient of the projection, v = g * phase(-r, -c).
 template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool OSX, bool GEN>
-__global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_scatter3_tiled(Geom g, TileSpec ts, const Cx<float>* __restrict__ src,
+__global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_scatter3_tiled(ScatterWork sw, Geom g, TileSpec ts, const Cx<float>* __restrict__ src,
                                                            const float* __restrict__ weights,
                                                            const float* __restrict__ rot,
                                                            const float* __restrict__ shifts,
@@ -1087,7 +1124,7 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool pose_lane = lane < KP;  // lane k holds pose k of the wave's batch
     const int N = g.N, H = g.H, half = N / 2;
-    const int64_t items = g.B * (ts.ssplit.pieces + int64_t(ts.ntd) * ts.ntr * ts.ntc);
+    const int64_t items = g.B * (sw.split.pieces + int64_t(ts.ntd) * ts.ntr * ts.ntc);
     const float cut2 = float(g.cut2);
     // samples lie within |x| <= rho_k: rotations reach rho_unit + 1, GEN poses the call's own
     // reach (up to kScaleMax times farther).  Without rotations in the call the rotation kernel
@@ -1104,9 +1141,9 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
         const int64_t slot_i = sl.s;
         const int64_t w = xcd_item<kRunScatter>(slot_i);
         if (w >= items) continue;
-        const Item it = uniform(item_of(w, g.B, ts.ntd, ts.ntr, ts.ntc, 0, 0, ts.ssplit));
+        const Item it = uniform(item_of(w, g.B, ts.ntd, ts.ntr, ts.ntc, 0, 0, &first_argument<ScatterWork>()->split));
         if (it.skip) continue;
-        const bool split = w < g.B * ts.ssplit.pieces;  // a piece, whose slot of the workspace is w
+        const bool split = w < g.B * sw.split.pieces;  // a piece, whose slot of the workspace is w
         const int64_t b = it.b;
         // stored cells of this tile, signed coordinates: d, r in [-N/2+1, N/2], c in [0, N/2]
         const int tc = it.kc * SC, tr = -half + 1 + it.kr * SR, td = -half + 1 + it.kd * SD;
@@ -1147,7 +1184,7 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
         // same poses' projections), or the poses of the tile's bin
         const unsigned short* lst = nullptr;
         int lcnt = int(g.P);
-        if (!empty && !split) tile_bin(ts.sbins, rb, g.P, it.kc, it.kr, it.kd, lst, lcnt);
+        if (!empty && !split) tile_bin(sw.bins, rb, g.P, it.kc, it.kr, it.kd, lst, lcnt);
         const int c_begin = empty ? 0 : piece_at(lcnt, it.j, it.k), c_end = empty ? 0 : piece_at(lcnt, it.j + 1, it.k);
         for (int pbase = c_begin; pbase < c_end; pbase += kChunkSc) {
             int n1, n2;
@@ -1369,7 +1406,7 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
             const int c = tc + lc, r = tr + lr;
             if (split || (c < H && r <= half)) {
                 // (a slot: the tile's values, then its weights)
-                char* const slot = ts.part + xcd_item<kRunScatter>(sl.s) * slot_bytes(WEIGHTS);
+                char* const slot = sw.part + xcd_item<kRunScatter>(sl.s) * slot_bytes(WEIGHTS);
                 Cx<float>* const out = split ? reinterpret_cast<Cx<float>*>(slot) : dst;
                 float* const wout = split ? reinterpret_cast<float*>(slot + S3 * 8) : wdst;
                 const int64_t row = split ? lr * SC + lc : b * g.vol + int64_t(r < 0 ? r + N : r) * H + c;
@@ -1400,7 +1437,7 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
 // Sum of the pieces of a split tile's cell (their slots of the workspace), fp64; or, for a tile of
 // one piece, the cell as the scatter stored it.
 template <bool CUBIC, bool WEIGHTS>
-__device__ __forceinline__ void cell_sum(const Geom& g, const TileSpec& ts, const PoseSplit& ps, float reach, int64_t b, int d, int r, int c,
+__device__ __forceinline__ void cell_sum(const Geom& g, const TileSpec& ts, const ScatterWork& sw, float reach, int64_t b, int d, int r, int c,
                                          const Cx<float>* dst, const float* wdst, int64_t idx, double& vr, double& vi,
                                          double& vw) {
     const int half = g.N / 2;
@@ -1408,7 +1445,7 @@ __device__ __forceinline__ void cell_sum(const Geom& g, const TileSpec& ts, cons
     const int e = ((d + half - 1 - kd * SD) * SR + (r + half - 1 - kr * SR)) * SC + (c - kc * SC);
     int64_t first = 0, at = 0;
     int k = 0;
-    if (!ts.ssplit.box.holds(kd, kr, kc)) {
+    if (!sw.split.box.holds(kd, kr, kc)) {
         vr = double(dst[idx].re);
         vi = double(dst[idx].im);
         vw = WEIGHTS ? double(wdst[idx]) : 0.0;
@@ -1416,10 +1453,10 @@ __device__ __forceinline__ void cell_sum(const Geom& g, const TileSpec& ts, cons
     }
 #pragma unroll
     for (int l = 0; l < kSplitLevels; ++l) {
-        const PoseSplit::Level& v = ps.lv[l];
-        if (k == 0 && v.holds(kd, kr, kc)) {
+        const PoseSplit::Level& v = sw.split.lv[l];
+        if (k == 0 && v.box.holds(kd, kr, kc)) {
             k = v.k;
-            const int t = ((kd - v.lo[0]) * v.size(1) + (kr - v.lo[1])) * v.size(2) + (kc - v.lo[2]);
+            const int t = ((kd - v.box.lo[0]) * v.box.size(1) + (kr - v.box.lo[1])) * v.box.size(2) + (kc - v.box.lo[2]);
             at = first + b * v.pieces + int64_t(t) * v.k;
         }
         first += g.B * int64_t(v.pieces);
@@ -1441,7 +1478,7 @@ __device__ __forceinline__ void cell_sum(const Geom& g, const TileSpec& ts, cons
         }
     }
     vr = vi = vw = 0.0;
-    const char* slot = ts.part + at * slot_bytes(WEIGHTS);
+    const char* slot = sw.part + at * slot_bytes(WEIGHTS);
 #pragma unroll 4
     for (int j = 0; j < k; ++j, slot += slot_bytes(WEIGHTS)) {
         const Cx<float> v = reinterpret_cast<const Cx<float>*>(slot)[e];
@@ -1462,13 +1499,13 @@ __device__ __forceinline__ void cell_sum(const Geom& g, const TileSpec& ts, cons
 constexpr int kFinishParts = 6;  // workgroups per split tile (one cell a lane: the sums wait for their loads)
 static_assert(S3 % (kFinishParts * kBlock) == 0, "whole workgroups per part");
 template <bool CUBIC, bool WEIGHTS, bool MIRROR>
-__global__ __launch_bounds__(kBlock) void k_finish3(Geom g, TileSpec ts, PoseSplit ps, int64_t red,
+__global__ __launch_bounds__(kBlock) void k_finish3(Geom g, TileSpec ts, ScatterWork sw, int64_t red,
                                                     Cx<float>* __restrict__ dst, float* __restrict__ wdst,
                                                     const CallPoses* __restrict__ cp) {
     const int N = g.N, H = g.H, half = N / 2;
     const float reach = fmaxf(cp->any_rot ? ts.rho_unit + 1.0f : 0.f, fminf(ts.rho, cp->gen_reach));
     if (int64_t(blockIdx.x) < red) {
-        const PoseSplit::Level& v = ts.ssplit.box;
+        const PoseSplit::Box& v = sw.split.box;
         const int nc = v.size(2), nr = v.size(1);
         const int64_t per_b = int64_t(v.size(0)) * nr * nc;
         const int64_t tile = blockIdx.x / kFinishParts, b = tile / per_b;
@@ -1480,7 +1517,7 @@ __global__ __launch_bounds__(kBlock) void k_finish3(Geom g, TileSpec ts, PoseSpl
             if (c >= H || r > half || d > half || (MIRROR && c == 0)) continue;
             const int64_t idx = b * g.vol + (int64_t(d < 0 ? d + N : d) * N + (r < 0 ? r + N : r)) * H + c;
             double vr, vi, vw;
-            cell_sum<CUBIC, WEIGHTS>(g, ts, ps, reach, b, d, r, c, dst, wdst, idx, vr, vi, vw);
+            cell_sum<CUBIC, WEIGHTS>(g, ts, sw, reach, b, d, r, c, dst, wdst, idx, vr, vi, vw);
             dst[idx] = Cx<float>{float(vr), float(vi)};
             if (WEIGHTS) wdst[idx] = float(vw);
         }
@@ -1499,7 +1536,7 @@ __global__ __launch_bounds__(kBlock) void k_finish3(Geom g, TileSpec ts, PoseSpl
             auto sg = [&](int i) { return i <= half ? i : i - N; };
             const int64_t i0 = b * g.vol + int64_t(q) * H, i1 = b * g.vol + int64_t(qm) * H;
             auto unsplit = [&](int d, int r) {
-                return !ts.ssplit.box.holds((d + half - 1) / SD, (r + half - 1) / SR, 0);
+                return !sw.split.box.holds((d + half - 1) / SD, (r + half - 1) / SR, 0);
             };
             if (unsplit(sg(de), sg(re)) && unsplit(sg(dm), sg(rm))) {  // most of the plane
                 if (qm == q) continue;
@@ -1514,13 +1551,13 @@ __global__ __launch_bounds__(kBlock) void k_finish3(Geom g, TileSpec ts, PoseSpl
                 continue;
             }
             double ar, ai, aw, mr, mi, mw;
-            cell_sum<CUBIC, WEIGHTS>(g, ts, ps, reach, b, sg(de), sg(re), 0, dst, wdst, i0, ar, ai, aw);
+            cell_sum<CUBIC, WEIGHTS>(g, ts, sw, reach, b, sg(de), sg(re), 0, dst, wdst, i0, ar, ai, aw);
             if (qm == q) {  // self-partnered
                 dst[i0] = Cx<float>{float(ar), float(ai)};
                 if (WEIGHTS) wdst[i0] = float(aw);
                 continue;
             }
-            cell_sum<CUBIC, WEIGHTS>(g, ts, ps, reach, b, sg(dm), sg(rm), 0, dst, wdst, i1, mr, mi, mw);
+            cell_sum<CUBIC, WEIGHTS>(g, ts, sw, reach, b, sg(dm), sg(rm), 0, dst, wdst, i1, mr, mi, mw);
             dst[i0] = Cx<float>{float(ar + mr), float(ai - mi)};
             dst[i1] = Cx<float>{float(mr + ar), float(mi - ai)};
             if (WEIGHTS) wdst[i0] = wdst[i1] = float(aw + mw);
@@ -1627,10 +1664,6 @@ __global__ __launch_bounds__(kBinThreads) void k_pose_bins(Geom g, const float* 
     }
 }
 
-// Work items of the rotation kernels' forward tile grid (the unit grid).
-int64_t forw_items(const Geom& g, const TileSpec& ts) {
-    return g.B * (ts.fsplit.pieces + int64_t(ts.nt) * ts.nt * ts.ntfd);
-}
 // Workgroups of a launch of `kernel` over `items`: one per item (rotations), or the persistent
 // GEN grid (the scatter's).
 template <bool GEN, int RUN>
@@ -1649,94 +1682,93 @@ unsigned grid_of(int64_t items, const void* kernel, int threads) {
 // and per-XCD counters, 0.77 / 0.74 / 0.74 ms with an eighth / a quarter / half of the rotation
 // slots, 0.83 ms with a sixteenth (and 1.29 against 1.69 ms with poses scaled by 1.4).
 constexpr int kGenForwShare = 4;
-inline unsigned gen_forw_grid(const Geom& g, const TileSpec& ts) {
-    const int64_t w = kXcds * xcd_per<kRunForw>(forw_items(g, ts)) / kGenForwShare;
+inline unsigned gen_forw_grid(int64_t rot_grid_items) {
+    const int64_t w = kXcds * xcd_per<kRunForw>(rot_grid_items) / kGenForwShare;
     return grid_for(std::max<int64_t>(kXcds, (w + kXcds - 1) / kXcds * kXcds));
 }
 
 // One forward-family kernel (GMODE 0, 1, 2) for rotations, then for the other tiled poses.
 template <bool CUBIC, int KP, bool OSX, int GMODE, bool RS, bool WG, typename VS>
-hipError_t forw_both(const Geom& g, const TileSpec& ts, const void* rec, const void* rot, const void* shifts,
+hipError_t forw_both(const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* rec, const void* rot, const void* shifts,
                      void* out, CallPoses* cp, int gl, const void* gsrc, void* grot, void* gshift, const void* gw,
                      void* wout, hipStream_t s) {
     const auto kr = k_forw3_tiled<CUBIC, KP, OSX, GMODE, RS, WG, VS, false>;
     const auto kg = k_forw3_tiled<CUBIC, KP, OSX, GMODE, RS, WG, VS, true>;
-    const int64_t rot_items = ts.flist ? ts.fcount : forw_items(g, ts);
-    hipLaunchKernelGGL(kr, dim3(grid_of<false, kRunForw>(rot_items, (const void*)kr, kForwThreads)),
-                       dim3(kForwThreads), 0, s, g, ts,
+    hipLaunchKernelGGL(kr, dim3(grid_of<false, kRunForw>(fw.rot.count, (const void*)kr, kForwThreads)),
+                       dim3(kForwThreads), 0, s, fw.rot, g, ts,
                        (const Cx<VS>*)rec, (const float*)rot, (const float*)shifts, (Cx<float>*)out, cp, gl,
                        (const Cx<float>*)gsrc, (float*)grot, (float*)gshift, (const float*)gw, (float*)wout);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kg, dim3(gen_forw_grid(g, ts)),
-                       dim3(kForwThreads), 0, s, g, ts,
+    hipLaunchKernelGGL(kg, dim3(gen_forw_grid(fw.gen.count)),
+                       dim3(kForwThreads), 0, s, fw.gen, g, ts,
                        (const Cx<VS>*)rec, (const float*)rot, (const float*)shifts, (Cx<float>*)out, cp, gl,
                        (const Cx<float>*)gsrc, (float*)grot, (float*)gshift, (const float*)gw, (float*)wout);
     return hipGetLastError();
 }
 
 template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool OSX>
-hipError_t scatter_launch(const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src, const void* weights, const void* rot,
+hipError_t scatter_launch(const Geom& g, const TileSpec& ts, const ScatterWork& sw, const void* src, const void* weights, const void* rot,
                           const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
     // rotations write every tile (none: the other tiled poses store them); the other tiled
     // poses add onto them
-    const int64_t work = g.B * (ts.ssplit.pieces + int64_t(ts.ntd) * ts.ntr * ts.ntc);
+    const int64_t work = g.B * (sw.split.pieces + int64_t(ts.ntd) * ts.ntr * ts.ntc);
     const auto kr = k_scatter3_tiled<CUBIC, MODE, WEIGHTS, KP, OSX, false>;
     const auto kg = k_scatter3_tiled<CUBIC, MODE, WEIGHTS, KP, OSX, true>;
     hipLaunchKernelGGL(kr, dim3(grid_of<false, kRunScatter>(work, (const void*)kr, kScatterThreads)),
-                       dim3(kScatterThreads), 0, s, g, ts,
+                       dim3(kScatterThreads), 0, s, sw, g, ts,
                        (const Cx<float>*)src, (const float*)weights, (const float*)rot, (const float*)shifts,
                        (Cx<float>*)dst, (float*)wdst, cp, gl);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kg, dim3(grid_of<true, kRunScatter>(work, (const void*)kg, kScatterThreads)),
-                       dim3(kScatterThreads), 0, s, g, ts,
+                       dim3(kScatterThreads), 0, s, sw, g, ts,
                        (const Cx<float>*)src, (const float*)weights, (const float*)rot, (const float*)shifts,
                        (Cx<float>*)dst, (float*)wdst, cp, gl);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const PoseSplit::Level& outer = ts.ssplit.box;
+    const PoseSplit::Box& outer = sw.split.box;
     const int64_t red = kFinishParts * g.B * int64_t(outer.size(0)) * outer.size(1) * outer.size(2);
     int64_t blocks = 0;
     if (MODE == 0) blocks = std::min<int64_t>(65536, (g.B * int64_t(g.N) * g.N + kBlock - 1) / kBlock);
     if (red + blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_finish3<CUBIC, WEIGHTS, MODE == 0>), dim3(unsigned(red + blocks)), dim3(kBlock), 0, s, g, ts, ps, red,
+    hipLaunchKernelGGL((k_finish3<CUBIC, WEIGHTS, MODE == 0>), dim3(unsigned(red + blocks)), dim3(kBlock), 0, s, g, ts, sw, red,
                        (Cx<float>*)dst, (float*)wdst, cp);
     return hipGetLastError();
 }
 
 template <bool CUBIC, int MODE, bool WEIGHTS, bool OSX>
-hipError_t scatter_kp_osx(const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src, const void* weights, const void* rot,
+hipError_t scatter_kp_osx(const Geom& g, const TileSpec& ts, const ScatterWork& sw, const void* src, const void* weights, const void* rot,
                           const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
     // (the cubic stencil carries windows across batches and keeps two pose sets: at most 4 poses)
     if constexpr (!CUBIC)
         if (ts.kp_scatter >= 6)
-            return scatter_launch<CUBIC, MODE, WEIGHTS, 6, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl,
+            return scatter_launch<CUBIC, MODE, WEIGHTS, 6, OSX>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl,
                                                                 s);
     if (ts.kp_scatter >= 4)
-        return scatter_launch<CUBIC, MODE, WEIGHTS, 4, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return scatter_launch<CUBIC, MODE, WEIGHTS, 4, OSX>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl, s);
     if (ts.kp_scatter >= 3)
-        return scatter_launch<CUBIC, MODE, WEIGHTS, 3, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
-    return scatter_launch<CUBIC, MODE, WEIGHTS, 1, OSX>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return scatter_launch<CUBIC, MODE, WEIGHTS, 3, OSX>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+    return scatter_launch<CUBIC, MODE, WEIGHTS, 1, OSX>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl, s);
 }
 
 template <bool CUBIC, int MODE, bool WEIGHTS>
-hipError_t scatter_kp(const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src, const void* weights, const void* rot,
+hipError_t scatter_kp(const Geom& g, const TileSpec& ts, const ScatterWork& sw, const void* src, const void* weights, const void* rot,
                       const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
     if (ts.os_exact)
-        return scatter_kp_osx<CUBIC, MODE, WEIGHTS, true>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
-    return scatter_kp_osx<CUBIC, MODE, WEIGHTS, false>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return scatter_kp_osx<CUBIC, MODE, WEIGHTS, true>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+    return scatter_kp_osx<CUBIC, MODE, WEIGHTS, false>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl, s);
 }
 
 template <bool CUBIC, bool OSX>
-hipError_t bpback_flags(const Geom& g, const TileSpec& ts, const void* gdata, const void* gw, const void* proj,
+hipError_t bpback_flags(const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* gdata, const void* gw, const void* proj,
                         const void* rot, const void* shifts, void* gproj, void* gweights, void* grot, void* gshift,
                         CallPoses* cp, int gl, hipStream_t s) {
     // poses per wave batch: the forward's count, at most two with gradient sums (a set per pose)
     const bool rs = grot || gshift, wg = gw && gweights;
     const int kp = ts.kp_forw >= 4 ? 4 : (ts.kp_forw == 2 ? 2 : 1);
 #define TP_BPB(KPV, RSV, WGV)                                                                                   \
-    forw_both<CUBIC, KPV, OSX, 2, RSV, WGV, float>(g, ts, gdata, rot, shifts, gproj, cp, gl, proj, grot, gshift, gw, \
+    forw_both<CUBIC, KPV, OSX, 2, RSV, WGV, float>(g, ts, fw, gdata, rot, shifts, gproj, cp, gl, proj, grot, gshift, gw, \
                                                    WGV ? gweights : nullptr, s)
     if (rs) {
         if (kp >= 2) return wg ? TP_BPB(2, true, true) : TP_BPB(2, true, false);
@@ -1749,10 +1781,10 @@ hipError_t bpback_flags(const Geom& g, const TileSpec& ts, const void* gdata, co
 }
 
 template <bool CUBIC, bool OSX, typename VS>
-hipError_t forw_kp(const Geom& g, const TileSpec& ts, const void* rec, const void* rot, const void* shifts, void* out,
+hipError_t forw_kp(const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* rec, const void* rot, const void* shifts, void* out,
                    CallPoses* cp, int gl, hipStream_t s) {
 #define TP_FORW(KPV) \
-    forw_both<CUBIC, KPV, OSX, 0, true, false, VS>(g, ts, rec, rot, shifts, out, cp, gl, nullptr, nullptr, nullptr, \
+    forw_both<CUBIC, KPV, OSX, 0, true, false, VS>(g, ts, fw, rec, rot, shifts, out, cp, gl, nullptr, nullptr, nullptr, \
                                                    nullptr, nullptr, s)
     // the forward's batches spread their rows over the lanes: about 64 / (rows of a pose) poses
     if (ts.kp_forw >= 4) return TP_FORW(kForwFlatKP);
@@ -1762,65 +1794,48 @@ hipError_t forw_kp(const Geom& g, const TileSpec& ts, const void* rec, const voi
 }
 
 template <typename VS>
-hipError_t forw_store(bool cubic, const Geom& g, const TileSpec& ts, const void* rec, const void* rot,
+hipError_t forw_store(bool cubic, const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* rec, const void* rot,
                       const void* shifts, void* out, CallPoses* cp, int gl, hipStream_t s) {
     if (cubic)
-        return ts.os_exact ? forw_kp<true, true, VS>(g, ts, rec, rot, shifts, out, cp, gl, s)
-                           : forw_kp<true, false, VS>(g, ts, rec, rot, shifts, out, cp, gl, s);
-    return ts.os_exact ? forw_kp<false, true, VS>(g, ts, rec, rot, shifts, out, cp, gl, s)
-                       : forw_kp<false, false, VS>(g, ts, rec, rot, shifts, out, cp, gl, s);
+        return ts.os_exact ? forw_kp<true, true, VS>(g, ts, fw, rec, rot, shifts, out, cp, gl, s)
+                           : forw_kp<true, false, VS>(g, ts, fw, rec, rot, shifts, out, cp, gl, s);
+    return ts.os_exact ? forw_kp<false, true, VS>(g, ts, fw, rec, rot, shifts, out, cp, gl, s)
+                       : forw_kp<false, false, VS>(g, ts, fw, rec, rot, shifts, out, cp, gl, s);
 }
 
 }  // namespace
 
-void split_items(const PoseSplit& ps, int64_t B, std::vector<TileItem>& out) {
-    using U = unsigned short;
-    for (int l = 0; l < ps.n; ++l) {
-        const PoseSplit::Level& v = ps.lv[l];
-        for (int64_t b = 0; b < B; ++b)
-            for (int d = v.lo[0]; d < v.lo[0] + v.size(0); ++d)
-                for (int r = v.lo[1]; r < v.lo[1] + v.size(1); ++r)
-                    for (int c = v.lo[2]; c < v.lo[2] + v.size(2); ++c) {
-                        // (the boxes are nested: the next one in holds the others)
-                        const bool held = l > 0 && ps.lv[l - 1].holds(d, r, c);
-                        for (int j = 0; j < v.k; ++j)
-                            out.push_back(TileItem{U(d), U(r), U(c), U(held ? 0 : v.k), int(b), j});
-                    }
-    }
-}
-
-int64_t forw_reach_items(const Geom& g, const TileSpec& ts, const PoseSplit& ps, std::vector<TileItem>& out) {
-    const int64_t items = forw_items(g, ts);
-    if (items > int64_t(INT32_MAX)) return items;
+void forw_reach_tiles(const TileSpec& ts, const PoseSplit& ps, std::vector<TileAt>& out, int n[kSplitLevels + 1]) {
     // the rotation kernel's test (dist2 > rho2: the tile holds no sample) with a margin, so that
-    // every tile the kernel would take is listed whatever the rounding
-    const float rho = ts.rho_unit + 1.0f, rho2 = rho * rho * 1.001f + 4.0f;
-    auto axis2 = [&](int t, int edge) {  // squared distance of [t, t + edge] (+ slack) from 0
+    // its own arithmetic drops no tile that the list leaves out
+    const float rho2 = (ts.rho_unit + 1.5f) * (ts.rho_unit + 1.5f);
+    auto axis2 = [&](int t, int edge) {
         const float lo = float(t) - ts.eps, hi = float(t + edge) + ts.eps;
         const float q = lo > 0.f ? lo : (hi < 0.f ? -hi : 0.f);
         return q * q;
     };
-    auto reached = [&](int d, int r, int c) {
-        return axis2(ts.orgd + d * LD, LD) + axis2(ts.org + r * L, L) + axis2(ts.org + c * L, L) <= rho2;
-    };
-    split_items(ps, g.B, out);
-    out.erase(std::remove_if(out.begin(), out.end(),
-                             [&](const TileItem& f) { return f.k == 0 || !reached(f.d, f.r, f.c); }),
-              out.end());
-    // then every unsplit tile of each batch item
     using U = unsigned short;
-    for (int64_t b = 0; b < g.B; ++b)
-        for (int kd = 0; kd < ts.ntfd; ++kd) {
-            const float d2 = axis2(ts.orgd + kd * LD, LD);
-            for (int kr = 0; kr < ts.nt; ++kr) {
-                const float r2 = d2 + axis2(ts.org + kr * L, L);
+    for (int l = 0; l <= kSplitLevels; ++l) {
+        n[l] = 0;
+        const bool whole = l == kSplitLevels;
+        if (!whole && l >= ps.n) continue;
+        const PoseSplit::Box all{}, &v = whole ? all : ps.lv[l].box;
+        const int hd = whole ? ts.ntfd : v.lo[0] + v.size(0), hr = whole ? ts.nt : v.lo[1] + v.size(1),
+                  hc = whole ? ts.nt : v.lo[2] + v.size(2), held = whole ? ps.n - 1 : l - 1;
+        const size_t before = out.size();
+        for (int d = v.lo[0]; d < hd; ++d) {
+            const float d2 = axis2(ts.orgd + d * LD, LD);
+            for (int r = v.lo[1]; r < hr; ++r) {
+                const float r2 = d2 + axis2(ts.org + r * L, L);
                 if (r2 > rho2) continue;
-                for (int kc = 0; kc < ts.nt; ++kc)
-                    if (r2 + axis2(ts.org + kc * L, L) <= rho2 && !(ps.n > 0 && ps.lv[ps.n - 1].holds(kd, kr, kc)))
-                        out.push_back(TileItem{U(kd), U(kr), U(kc), 1, int(b), 0});
+                for (int c = v.lo[2]; c < hc; ++c)
+                    // (the boxes are nested: the next one in holds the others)
+                    if (r2 + axis2(ts.org + c * L, L) <= rho2 && !(held >= 0 && ps.lv[held].box.holds(d, r, c)))
+                        out.push_back(TileAt{U(d), U(r), U(c), 0});
             }
         }
-    return items;
+        n[l] = int(out.size() - before);
+    }
 }
 
 hipError_t launch_pose_bins(const Geom& g, const void* rot, const BinGrid& bg, const BinBox& bb, const CallPoses* cp,
@@ -1831,19 +1846,19 @@ hipError_t launch_pose_bins(const Geom& g, const void* rot, const BinGrid& bg, c
     return hipGetLastError();
 }
 
-hipError_t launch_project3_forw_tiled(bool cubic, const Geom& g, const TileSpec& ts, const void* rec,
+hipError_t launch_project3_forw_tiled(bool cubic, const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* rec,
                                       const void* rot, const void* shifts, void* out, CallPoses* cp, int gl,
                                       hipStream_t s, bool rec_half) {
-    if (rec_half) return forw_store<__half>(cubic, g, ts, rec, rot, shifts, out, cp, gl, s);
-    return forw_store<float>(cubic, g, ts, rec, rot, shifts, out, cp, gl, s);
+    if (rec_half) return forw_store<__half>(cubic, g, ts, fw, rec, rot, shifts, out, cp, gl, s);
+    return forw_store<float>(cubic, g, ts, fw, rec, rot, shifts, out, cp, gl, s);
 }
 
-hipError_t launch_grads3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const void* gproj, const void* rec,
+hipError_t launch_grads3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* gproj, const void* rec,
                                const void* rot, const void* shifts, void* grot, void* gshift, CallPoses* cp, int gl,
                                hipStream_t s, bool rec_half) {
     if (!grot && !gshift) return hipSuccess;
 #define TP_GRADS(C, O, V) \
-    forw_both<C, 2, O, 1, true, false, V>(g, ts, rec, rot, shifts, nullptr, cp, gl, gproj, grot, gshift, nullptr, \
+    forw_both<C, 2, O, 1, true, false, V>(g, ts, fw, rec, rot, shifts, nullptr, cp, gl, gproj, grot, gshift, nullptr, \
                                           nullptr, s)
     if (rec_half) {
         if (cubic) return ts.os_exact ? TP_GRADS(true, true, __half) : TP_GRADS(true, false, __half);
@@ -1854,32 +1869,32 @@ hipError_t launch_grads3_tiled(bool cubic, const Geom& g, const TileSpec& ts, co
 #undef TP_GRADS
 }
 
-hipError_t launch_bpback3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const void* gdata, const void* gw,
+hipError_t launch_bpback3_tiled(bool cubic, const Geom& g, const TileSpec& ts, const ForwWorks& fw, const void* gdata, const void* gw,
                                 const void* proj, const void* rot, const void* shifts, void* gproj, void* gweights,
                                 void* grot, void* gshift, CallPoses* cp, int gl, hipStream_t s) {
     if (cubic)
-        return ts.os_exact ? bpback_flags<true, true>(g, ts, gdata, gw, proj, rot, shifts, gproj, gweights, grot, gshift,
+        return ts.os_exact ? bpback_flags<true, true>(g, ts, fw, gdata, gw, proj, rot, shifts, gproj, gweights, grot, gshift,
                                                       cp, gl, s)
-                           : bpback_flags<true, false>(g, ts, gdata, gw, proj, rot, shifts, gproj, gweights, grot,
+                           : bpback_flags<true, false>(g, ts, fw, gdata, gw, proj, rot, shifts, gproj, gweights, grot,
                                                        gshift, cp, gl, s);
-    return ts.os_exact ? bpback_flags<false, true>(g, ts, gdata, gw, proj, rot, shifts, gproj, gweights, grot, gshift,
+    return ts.os_exact ? bpback_flags<false, true>(g, ts, fw, gdata, gw, proj, rot, shifts, gproj, gweights, grot, gshift,
                                                    cp, gl, s)
-                       : bpback_flags<false, false>(g, ts, gdata, gw, proj, rot, shifts, gproj, gweights, grot, gshift,
+                       : bpback_flags<false, false>(g, ts, fw, gdata, gw, proj, rot, shifts, gproj, gweights, grot, gshift,
                                                     cp, gl, s);
 }
 
-hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const PoseSplit& ps, const void* src,
+hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const TileSpec& ts, const ScatterWork& sw, const void* src,
                                  const void* weights, const void* rot, const void* shifts, void* dst, void* wdst,
                                  CallPoses* cp, int gl, hipStream_t s) {
     if (mode == 0) {
         if (weights)
-            return cubic ? scatter_kp<true, 0, true>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s)
-                         : scatter_kp<false, 0, true>(g, ts, ps, src, weights, rot, shifts, dst, wdst, cp, gl, s);
-        return cubic ? scatter_kp<true, 0, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
-                     : scatter_kp<false, 0, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
+            return cubic ? scatter_kp<true, 0, true>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl, s)
+                         : scatter_kp<false, 0, true>(g, ts, sw, src, weights, rot, shifts, dst, wdst, cp, gl, s);
+        return cubic ? scatter_kp<true, 0, false>(g, ts, sw, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
+                     : scatter_kp<false, 0, false>(g, ts, sw, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
     }
-    return cubic ? scatter_kp<true, 1, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
-                 : scatter_kp<false, 1, false>(g, ts, ps, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
+    return cubic ? scatter_kp<true, 1, false>(g, ts, sw, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s)
+                 : scatter_kp<false, 1, false>(g, ts, sw, src, nullptr, rot, shifts, dst, nullptr, cp, gl, s);
 }
 
 }  // namespace tp
