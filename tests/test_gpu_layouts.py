@@ -104,3 +104,21 @@ def test_volume_at_an_8_byte_boundary(gpu, oracle, interp, odd_box):
     assert torch.equal(got, aligned)
     ref = oracle.project_3d_to_2d_forw(rec.cpu(), rot, None, (n, n), interp, 2.0, None)
     assert torch.equal(got.cpu(), ref)
+
+
+@pytest.mark.parametrize("interp", ["linear", "cubic"])
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("N", [2, 3, 9, 21, 33])
+def test_reconstruction_gradient_of_odd_boxes(hip, oracle, dim, interp, N):
+    """A reconstruction of odd edge has cells that no sample's tap can reach (beyond N / 2 on an axis): their
+    gradient is zero, not what the output's memory held."""
+    g = torch.Generator().manual_seed(600 + N)
+    n, P = 16, 9
+    rec = torch.randn((1,) + (N,) * (dim - 1) + (N // 2 + 1,), generator=g, dtype=torch.complex64)
+    gp = torch.randn(1, P, n, n // 2 + 1, generator=g, dtype=torch.complex64)
+    rot = torch.linalg.qr(torch.randn(1, P, dim, dim, generator=g, dtype=torch.float64))[0].float()
+    op = "project_2d_back" if dim == 2 else "project_3d_to_2d_back"
+    print(f"[layouts] odd box dim={dim} {interp} N={N}", flush=True)
+    got = getattr(hip, op)(gp, rec, rot, None, interp, 1.5, None)[0]
+    exp = getattr(oracle, op)(gp, rec, rot, None, interp, 1.5, None)[0]
+    assert rel_l2(got, exp) <= 1e-5

@@ -814,7 +814,8 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     const bool tiles = use_tiles(dim, dtype, os, n) && g.work > 0;
     const bool tiles2 = use_tiles2(dim, dtype, os, n) && g.work > 0;
     if (g.B > 0) TP_TRY(need(grec, "grad_reconstruction"));
-    if (!tiles) TP_TRY(zero(grec, cx_words(dtype, g.B * g.vol), s));
+    // (the 3D tiles write every cell of an even box; an odd one has a plane and rows more, beyond any tap)
+    if (!tiles || N % 2) TP_TRY(zero(grec, cx_words(dtype, g.B * g.vol), s));
     TP_TRY(zero(grot, re_words(dtype, g.B_rot * g.P * dim * dim), s));
     TP_TRY(zero(gshift, re_words(dtype, g.B_shift * g.P * 2), s));
     if (g.work == 0) return TP_OK;
