@@ -124,6 +124,47 @@ def test_replay_after_the_bin_workspace_grew(gpu):
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("warm", [48, 600])
+def test_2d_backprojection_replayed(gpu, warm):
+    """A 2D backprojection of 600 poses captured after an eager call of few poses (the stream's workspace is
+    too small for the pose ranges' slots: the captured call adds its ranges into the image) and of as many
+    (it uses the slots), and, after the latter, an eager call that grows the workspace."""
+    T = torch.ops.torch_projectors
+    gen = torch.Generator().manual_seed(8085)
+    P, n = 600, 40
+    proj = torch.randn(2, 3 * P, n, n // 2 + 1, generator=gen, dtype=torch.complex64).to(gpu)
+    w = torch.rand(2, 3 * P, n, n // 2 + 1, generator=gen).to(gpu)
+    a = torch.rand(3 * P, generator=gen) * 6.283
+    rot = torch.stack([a.cos(), -a.sin(), a.sin(), a.cos()], 1).reshape(1, 3 * P, 2, 2)
+    rot[:, ::4] *= 1.2
+    rot = rot.to(gpu)
+
+    def bp(count):
+        return T.backproject_2d_forw(proj[:, :count].contiguous(), w[:, :count].contiguous(),
+                                     rot[:, :count].contiguous(), None, "linear", 1.0, None)
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        bp(warm)
+    torch.cuda.synchronize()
+    pg, wg, rg = proj[:, :P].contiguous(), w[:, :P].contiguous(), rot[:, :P].contiguous()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        data_g, wrec_g = T.backproject_2d_forw(pg, wg, rg, None, "linear", 1.0, None)
+    torch.cuda.synchronize()
+    data_e, wrec_e = bp(P)
+    torch.cuda.synchronize()
+    for replay in range(3):
+        with torch.cuda.stream(stream):
+            bp(3 * P)  # eager work on the capture stream, with its own slots
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        print(f"[graph] 2D replay {replay} warm {warm}", flush=True)
+        assert _rel(data_g, data_e) <= 1e-5 and _rel(wrec_g, wrec_e) <= 1e-5
+
+
 def test_fourier_transforms_replayed_after_plan_eviction(gpu):
     """hipFFT transforms captured after one eager call of their shape on the capture stream, then
     replayed after more distinct shapes on that stream than the plan cache holds (32): the plans a

@@ -88,3 +88,50 @@ def test_tiled_gathers_past_the_per_pixel_sizes(case, hip, oracle):
     exp = getattr(oracle, case["op"])(*args)
     check_outputs(case["op"], got, exp, has_shifts=tensors.get("shifts") is not None, label=case["name"],
                   cells=scatter_cells(case["op"], args, oracle))
+
+
+# 2D scatters of many short pose ranges on small images: rotations alone, with scaled poses among them
+# (their kernel adds onto the rotations' tiles), and scaled poses alone; tiles beyond the cutoff's reach.
+MANY = [(op, interp, n, os_, P, B, cut, scale)
+        for op in ("backproject_2d_forw", "project_2d_back")
+        for interp, n, os_, P, B, cut, scale in (
+            ("linear", 32, 1.0, 4099, 1, None, None), ("linear", 40, 1.0, 517, 3, 9.0, "some"),
+            ("cubic", 24, 1.0, 1031, 2, None, "all"), ("cubic", 36, 2.0, 700, 1, 7.5, "some"),
+            ("linear", 48, 1.75, 333, 2, None, "some"), ("linear", 33, 2.0, 97, 1, None, "all"))]
+
+
+@pytest.mark.parametrize("op,interp,n,os_,P,B,cut,scale", MANY)
+def test_many_ranges_match_oracle(op, interp, n, os_, P, B, cut, scale, hip, oracle):
+    case = _case("many", op, interp=interp, os=os_, cutoff=cut, B=B, P=P, n=n, B_rot=B, seed=773000 + P + n,
+                 weights=True)
+    args, tensors = make_inputs(case)
+    at = _rotations_at(args)
+    rot = args[at].detach().clone()
+    if scale:
+        rot[:, ::(3 if scale == "some" else 1)] *= 1.3
+    args[at] = rot.requires_grad_(args[at].requires_grad)
+    print(f"[many ranges] {op} {interp} n={n} os={os_} P={P} {scale}", flush=True)
+    got = getattr(hip, op)(*args)
+    exp = getattr(oracle, op)(*args)
+    check_outputs(op, got, exp, has_shifts=tensors.get("shifts") is not None, label=f"{op} {P}",
+                  cells=scatter_cells(op, args, oracle))
+
+
+@pytest.mark.parametrize("scale", [1.0, 1.1])
+def test_precision_does_not_fall_with_the_pose_count(gpu, scale):
+    """The weight image of 4096 poses of a small image, against the complex128 path: a range's sum rounds
+    to fp32 once and the ranges' sum once (2^-24 each, relative), the taps' weight products round
+    independently over the poses: together below 2^-23.  (256 ranges added in fp32 gave 2.1e-7.)"""
+    import torch
+    n, P = 64, 4096
+    g = torch.Generator(device="cuda").manual_seed(774000)
+    pr = torch.randn(1, P, n, n // 2 + 1, generator=g, device="cuda", dtype=torch.complex64)
+    w = torch.rand(1, P, n, n // 2 + 1, generator=g, device="cuda")
+    a = torch.rand(P, generator=g, device="cuda", dtype=torch.float64) * 6.283
+    rot = (scale * torch.stack([a.cos(), -a.sin(), a.sin(), a.cos()], 1)).reshape(1, P, 2, 2).float()
+    f = torch.ops.torch_projectors.backproject_2d_forw
+    data, wrec = f(pr, w, rot, None, "linear", 1.0, None)
+    data64, wrec64 = f(pr.to(torch.complex128), w.double(), rot.double(), None, "linear", 1.0, None)
+    print(f"[precision] scale {scale}", flush=True)
+    assert ((wrec.double() - wrec64).norm() / wrec64.norm()).item() < 2.0 ** -23
+    assert ((data.to(torch.complex128) - data64).norm() / data64.norm()).item() < 2e-6

@@ -303,19 +303,7 @@ tp::TileSpec2 tile_spec2(const tp::Geom& g, bool cubic) {
     };
     tiles_within(rho_unit + 1.0, ts.kr0, ts.nr, ts.nc);
     tiles_within(rho, ts.kr0_2, ts.nr_2, ts.nc_2);
-    // Every pose reaches every tile of the disc: split the poses into ranges until there are about
-    // 32768 work items, keeping >= 32 poses a range.  A workgroup's item is long (all of its range's
-    // poses cross its tile), so many short items balance the CUs far better than the partial tiles'
-    // extra float atomics cost: 8 images of 100 x 100 with 500 poses each (112 tiles) took 1.11 ms
-    // in ranges of 167 poses (336 items), 0.43 ms of 64, 0.36 of 32 and 0.33 of 16; 16 x 512 poses of
-    // 256 x 256 (1440 tiles, a cubic step) 2.84 / 2.81 / 2.83 ms with ranges of 64 / 32 / 16, and
-    // 16 x 4096 of them 10.18 ms at 16384 items, 9.7 at 32768 and 65536.  Ranges of 16 pay only while
-    // the items are few (below about 4096); past that they cost up to 3 % by their fixed work.
-    const int64_t tiles = g.B * int64_t(ts.nr) * ts.nc;
-    const int64_t want = tiles > 0 ? (32768 + tiles - 1) / tiles : 1;
-    const int64_t most = std::max<int64_t>(1, g.P / (tiles * (g.P / 32) < 4096 ? 16 : 32));
-    ts.ksplit = int(std::max<int64_t>(1, std::min(want, most)));
-    ts.prange = int((g.P + ts.ksplit - 1) / ts.ksplit);
+    // (the pose ranges: plan_scatter2)
     ts.rho = float(rho);
     ts.rho_unit = float(rho_unit);
     ts.os = float(g.os);
@@ -353,6 +341,13 @@ tp::TileSpec2 tile_spec2(const tp::Geom& g, bool cubic) {
     const int grows = int(std::ceil(std::sqrt(2.0) * gw / g.os)) + 2;
     ts.kp_gather = grows <= 16 ? 4 : (grows <= 32 ? 2 : 1);
     return ts;
+}
+
+// The 2D scatters' pose ranges, `ksplit` of them, none empty.
+void pose_ranges2(const tp::Geom& g, tp::TileSpec2& ts, int64_t ksplit) {
+    ksplit = std::max<int64_t>(1, ksplit);
+    ts.prange = int((g.P + ksplit - 1) / ksplit);
+    ts.ksplit = int((g.P + ts.prange - 1) / ts.prange);
 }
 
 // Calls small enough that the per-pixel gathers beat the tile-owner ones (fp32, complex-half volumes
@@ -689,6 +684,32 @@ int plan_scatter(const tp::Geom& g, const tp::TileSpec& ts, tp::ScatterWork& sw,
     }
     return TP_OK;
 }
+// The 2D scatter's pose ranges and their slots (tp::TileSpec2::part).  Every pose reaches every tile of the
+// disc: split the poses into ranges until there are about 32768 work items, keeping >= 32 poses a range.
+// A workgroup's item is long (all of its range's poses cross its tile), so many short items balance the
+// CUs far better than the partial tiles' extra traffic costs: 8 images of 100 x 100 with 500 poses each
+// (112 tiles) took 1.11 ms in ranges of 167 poses (336 items), 0.43 ms of 64, 0.36 of 32 and 0.33 of 16;
+// 16 x 512 poses of 256 x 256 (1440 tiles, a cubic step) 2.84 / 2.81 / 2.83 ms with ranges of 64 / 32 / 16,
+// and 16 x 4096 of them 10.18 ms at 16384 items, 9.7 at 32768 and 65536.  Ranges of 16 pay only while
+// the items are few (below about 4096); past that they cost up to 3 % by their fixed work.  At most
+// kMaxSlots2 bytes of slots (longer ranges then).  Without a workspace (one range, a failed allocation,
+// growth under graph capture) every range is added in fp32 into the zeroed image: ranges of >= 128 poses,
+// about 65536 items at most, keep that sum short.
+constexpr double kMaxSlots2 = double(size_t(1) << 29);
+int plan_scatter2(const tp::Geom& g, tp::TileSpec2& ts, bool weights, CallScratch& sc, hipStream_t s) {
+    TP_TRY(sc.get(s));
+    const int64_t tiles = std::max<int64_t>(1, g.B * int64_t(ts.nr) * ts.nc);
+    const int64_t most = g.P / (tiles * (g.P / 32) < 4096 ? 16 : 32);
+    int64_t k = std::min((32768 + tiles - 1) / tiles, most);
+    const double range = double(g.B) * (double(ts.nr) * ts.nc + double(ts.nr_2) * ts.nc_2) *
+                         double(tp::slot_bytes2(weights));
+    k = std::min(k, int64_t(kMaxSlots2 / std::max(1.0, range)));
+    pose_ranges2(g, ts, k);
+    ts.part = nullptr;
+    if (ts.ksplit > 1) ts.part = static_cast<char*>(sc.bins(size_t(range) * size_t(ts.ksplit), s));
+    if (!ts.part) pose_ranges2(g, ts, std::min((65536 + tiles - 1) / tiles, g.P / 128));
+    return TP_OK;
+}
 int fill_bins(bool cubic, const tp::Geom& g, const tp::TileSpec& ts, const tp::ScatterWork& sw, const void* rot, CallScratch& sc,
               hipStream_t s) {
     if (!sw.bins.list) return TP_OK;
@@ -815,7 +836,7 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     const bool tiles2 = use_tiles2(dim, dtype, os, n) && g.work > 0;
     if (g.B > 0) TP_TRY(need(grec, "grad_reconstruction"));
     // (the 3D tiles write every cell of an even box; an odd one has a plane and rows more, beyond any tap)
-    if (!tiles || N % 2) TP_TRY(zero(grec, cx_words(dtype, g.B * g.vol), s));
+    if (!(tiles || tiles2) || (tiles && N % 2)) TP_TRY(zero(grec, cx_words(dtype, g.B * g.vol), s));
     TP_TRY(zero(grot, re_words(dtype, g.B_rot * g.P * dim * dim), s));
     TP_TRY(zero(gshift, re_words(dtype, g.B_shift * g.P * 2), s));
     if (g.work == 0) return TP_OK;
@@ -844,7 +865,9 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
                             "tiled rotation/shift-gradient launch"));
     }
     if (tiles2) {
-        const tp::TileSpec2 ts = tile_spec2(g, cubic);
+        tp::TileSpec2 ts = tile_spec2(g, cubic);
+        TP_TRY(plan_scatter2(g, ts, false, sc, s));
+        if (!ts.part) TP_TRY(zero(grec, cx_words(dtype, g.B * g.vol), s));
         TP_TRY(call_poses(2, g, rot, ts.rho_unit, sc, s));
         TP_TRY(launched(tp::launch_scatter2_tiled(cubic, 1, g, ts, gproj, nullptr, rot, shifts, grec, nullptr, sc.p, 0,
                                                   s),
@@ -878,7 +901,7 @@ int backproject_forw(int dim, int dtype, const void* proj, int64_t B, int64_t P,
     const bool tiles = use_tiles(dim, dtype, os, n) && g.work > 0;
     const bool tiles2 = use_tiles2(dim, dtype, os, n) && g.work > 0;
     if (g.B > 0) TP_TRY(need(data, "data_reconstruction"));
-    if (!tiles) {
+    if (!tiles && !tiles2) {
         TP_TRY(zero(data, cx_words(dtype, g.B * g.vol), s));
         TP_TRY(zero(wrec, re_words(dtype, g.B * g.vol), s));
     }
@@ -897,7 +920,12 @@ int backproject_forw(int dim, int dtype, const void* proj, int64_t B, int64_t P,
                         "tiled backprojection launch"));
     }
     if (tiles2) {
-        const tp::TileSpec2 ts = tile_spec2(g, cubic);
+        tp::TileSpec2 ts = tile_spec2(g, cubic);
+        TP_TRY(plan_scatter2(g, ts, weights != nullptr, sc, s));
+        if (!ts.part) {
+            TP_TRY(zero(data, cx_words(dtype, g.B * g.vol), s));
+            TP_TRY(zero(wrec, re_words(dtype, g.B * g.vol), s));
+        }
         TP_TRY(call_poses(2, g, rot, ts.rho_unit, sc, s));
         TP_TRY(launched(tp::launch_scatter2_tiled(cubic, 0, g, ts, proj, weights, rot, shifts, data, wrec, sc.p, 0, s),
                         "tiled backprojection launch"));

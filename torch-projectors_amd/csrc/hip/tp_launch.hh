@@ -193,7 +193,16 @@ struct TileSpec2 {
     int gnt2, gorg2;        // gather: the same for the other tiled poses
     int gksplit, gprange;   // gather: pose ranges per tile, poses per range
     int kp_gather;          // gather (forward): poses per wavefront batch
+    // scatter: a slot of slot_bytes2 per work item of the rotations (B * ksplit * nr * nc), then per work
+    // item of the other poses (at most B * ksplit * nr_2 * nc_2; where the rotations have the same tile
+    // and range, that slot takes both), which k_finish2 sums into the image; null: the items are added
+    // into a zeroed image
+    char* part;
 };
+// Bytes of one range's tile in the 2D scatter's workspace: its values, then its weights.
+__host__ __device__ constexpr int64_t slot_bytes2(bool weights) {
+    return int64_t(kTile2C) * kTile2R * (weights ? 12 : 8);
+}
 
 // Per-call summary of the poses, written into a device scratch area by
 // launch_call_poses before the tiled kernels of the call (stream order) and
@@ -282,7 +291,8 @@ hipError_t launch_scatter3_tiled(bool cubic, int mode, const Geom& g, const Tile
                                  const void* weights, const void* rot, const void* shifts, void* dst, void* wdst,
                                  CallPoses* cp, int gl, hipStream_t s);
 
-// fp32 2D tile-owner scatter (tiled poses only), into zero-filled dst / wdst.
+// fp32 2D tile-owner scatter (tiled poses only): with ts.part it writes every cell of dst / wdst, else it
+// adds into them, zero-filled.
 // mode 0: backprojection with the x = 0 Hermitian completion; mode 1:
 // reconstruction gradient of the projection.
 hipError_t launch_scatter2_tiled(bool cubic, int mode, const Geom& g, const TileSpec2& ts, const void* src,

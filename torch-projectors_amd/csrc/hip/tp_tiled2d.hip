@@ -29,6 +29,7 @@
 // has sc = as . x and sr = bs . x with the dual basis (the rows of R^-1),
 // which bounds the rows and the half plane sc >= 0 that reach a box; their
 // tiles reach up to kScaleMax times farther out.
+#include <algorithm>
 #include <type_traits>
 
 #include "tp_device.hh"
@@ -313,13 +314,26 @@ __device__ __forceinline__ void scatter_sample2_priv(const Geom& g, const Slot2&
     }
 }
 
+// The tiles that the call's other tiled poses reach (|x| <= rho_k): rows [kr0, kr0 + nr), columns [0, nc).
+__device__ __forceinline__ void gen_tiles2(const Geom& g, const TileSpec2& ts, float rho_k, int& kr0, int& nr, int& nc) {
+    const int half = g.N / 2;
+    const float reach = fminf(rho_k + 3.0f, float(g.N));
+    kr0 = max(ts.kr0_2, int(floorf((-reach + float(half - 1)) / float(TR))));
+    const int kr1 = min(ts.kr0_2 + ts.nr_2, int(floorf((reach + float(half - 1)) / float(TR))) + 1);
+    nr = max(0, kr1 - kr0);
+    nc = min(ts.nc_2, int(floorf(reach / float(TC))) + 1);
+}
+
 // MODE 0: backprojection, v = proj * conj(phase(r, c)), optional weights.
 // MODE 1: reconstruction gradient of the projection, v = g * phase(-r, -c).
-// dst (and wdst) must be zero-filled: every item adds its partial tile.
+// Every item stores its partial tile in its slot of the workspace ts.part, which k_finish2 sums in fp64
+// (the fp32 sum of a cell over the short pose ranges of a small call, up to 31 of them with 500 poses,
+// took its weights' error against 64 bits from 0.9e-7 to 1.1e-7, over 256 ranges from 0.8e-7 to 2.1e-7); or,
+// without a workspace, adds it into dst (and wdst), zero-filled.
 // PRIV (one pose per window, KP = 1, os > sqrt(2) with margin): wave-private
 // fp32 accumulators without atomics, summed over the waves at write-out;
 // otherwise one fp64 accumulator per tile with LDS atomics.
-template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool PRIV, bool GEN>
+template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool PRIV, bool GEN, bool SLOTS>
 __global__ __launch_bounds__(kThreads) void k_scatter2_tiled(Geom g, TileSpec2 ts, const Cx<float>* __restrict__ src,
                                                              const float* __restrict__ weights,
                                                              const float* __restrict__ rot,
@@ -353,11 +367,7 @@ __global__ __launch_bounds__(kThreads) void k_scatter2_tiled(Geom g, TileSpec2 t
     if constexpr (GEN) {
         rho_k = fminf(ts.rho, cp->gen_reach);
         if (!(rho_k > 0.f)) return;  // no such pose in this call
-        const float reach = fminf(rho_k + 3.0f, float(N));
-        tkr0 = max(ts.kr0_2, int(floorf((-reach + float(half - 1)) / float(TR))));
-        const int kr1 = min(ts.kr0_2 + ts.nr_2, int(floorf((reach + float(half - 1)) / float(TR))) + 1);
-        tnr = max(0, kr1 - tkr0);
-        tnc = min(ts.nc_2, int(floorf(reach / float(TC))) + 1);
+        gen_tiles2(g, ts, rho_k, tkr0, tnr, tnc);
     }
     const int64_t items = g.B * ts.ksplit * int64_t(tnr) * tnc;
     const float cut2 = float(g.cut2);
@@ -520,37 +530,140 @@ __global__ __launch_bounds__(kThreads) void k_scatter2_tiled(Geom g, TileSpec2 t
             }
         }
 
-        // add the partial tile into the image (cells past the stored range are dropped taps)
         __syncthreads();
-        if (pend > p0) {
-            for (int e = tid; e < T2; e += kThreads) {
-                const int lc = e % TC, lr = e / TC;
-                const int c = tc + lc, r = tr + lr;
-                if (c >= H || r > half) continue;
-                const int re = r < 0 ? r + N : r;
-                const int64_t idx = b * g.vol + int64_t(re) * H + c;
-                const int a = (e - lc) + ((lc + swizzle2(lr)) & (TC - 1));
-                double vr, vi, vw = 0.0;
-                if constexpr (PRIV) {
-                    const int pa = lr * PS + lc;
-                    vr = vi = 0.0;
+        auto cell = [&](int e, double& vr, double& vi, double& vw) {  // of the accumulators
+            const int lc = e % TC, lr = e / TC;
+            vw = 0.0;
+            if constexpr (PRIV) {
+                const int pa = lr * PS + lc;
+                vr = vi = 0.0;
 #pragma unroll
-                    for (int k = 0; k < NW; ++k) {
-                        vr += double(pacc[k][pa].x);
-                        vi += double(pacc[k][pa].y);
-                        if (WEIGHTS) vw += double(pwacc[k][pa]);
-                    }
-                } else {
-                    vr = acc_re[a];
-                    vi = acc_im[a];
-                    if (WEIGHTS) vw = acc_w[a];
+                for (int k = 0; k < NW; ++k) {
+                    vr += double(pacc[k][pa].x);
+                    vi += double(pacc[k][pa].y);
+                    if (WEIGHTS) vw += double(pwacc[k][pa]);
                 }
+            } else {
+                const int a = (e - lc) + ((lc + swizzle2(lr)) & (TC - 1));
+                vr = acc_re[a];
+                vi = acc_im[a];
+                if (WEIGHTS) vw = acc_w[a];
+            }
+        };
+        if constexpr (SLOTS) {
+            // every cell of the partial tile to the item's slot (zeros where no pose reaches it: the
+            // accumulators are clear); GEN onto the rotations' slot where they have the tile
+            int64_t at = xcd_item<kRun>(sl.s);
+            bool onto = false;
+            if constexpr (GEN) {
+                onto = call_flag(&cp->any_rot) && unsigned(kr - ts.kr0) < unsigned(ts.nr) && kc < ts.nc;
+                const int64_t rows = b * ts.ksplit + jr;
+                at = onto ? (rows * ts.nr + (kr - ts.kr0)) * ts.nc + kc : g.B * ts.ksplit * int64_t(ts.nr) * ts.nc + at;
+            }
+            if (!(onto && pend <= p0)) {
+                char* const slot = ts.part + at * slot_bytes2(WEIGHTS);
+                for (int e = tid; e < T2; e += kThreads) {
+                    double vr, vi, vw;
+                    cell(e, vr, vi, vw);
+                    Cx<float>* const sv = reinterpret_cast<Cx<float>*>(slot) + e;
+                    float* const sw = reinterpret_cast<float*>(slot + T2 * 8) + e;
+                    if (GEN && onto) {
+                        vr += double(sv->re);
+                        vi += double(sv->im);
+                        if (WEIGHTS) vw += double(*sw);
+                    }
+                    *sv = Cx<float>{float(vr), float(vi)};
+                    if (WEIGHTS) *sw = float(vw);
+                }
+            }
+        } else if (pend > p0) {
+            // add the partial tile into the image (cells past the stored range are dropped taps)
+            for (int e = tid; e < T2; e += kThreads) {
+                const int c = tc + e % TC, r = tr + e / TC;
+                if (c >= H || r > half) continue;
+                const int64_t idx = b * g.vol + int64_t(r < 0 ? r + N : r) * H + c;
+                double vr, vi, vw;
+                cell(e, vr, vi, vw);
                 if (vr != 0.0) atomic_add(&dst[idx].re, float(vr));
                 if (vi != 0.0) atomic_add(&dst[idx].im, float(vi));
                 if (WEIGHTS && vw != 0.0) atomic_add(&wdst[idx], float(vw));
             }
         }
         __syncthreads();
+    }
+}
+
+// Completion of a scatter into slots: LANES lanes per stored cell sum its ranges' slots in fp64 and write
+// the cell (zero where no tile reaches); with MIRROR the cells of the x = 0 column also take their
+// partner's sum, as in k_mirror2_x0.  Bound by reading the slots: neighbouring cells are neighbouring
+// lanes, and a small image's cells take several lanes each, so that enough loads are in flight (8 images
+// of 100 x 100, 31 ranges: 36 us with one lane per cell, 8 with eight; 16 x 512 poses of 256 x 256, cutoff
+// 64, 94 MB of slots: 20 us).
+template <bool WEIGHTS, bool MIRROR, int LANES>
+__global__ __launch_bounds__(kBlock) void k_finish2(Geom g, TileSpec2 ts, Cx<float>* __restrict__ dst,
+                                                    float* __restrict__ wdst, const CallPoses* __restrict__ cp) {
+    constexpr int CELLS = kBlock / LANES;  // per workgroup: lane = part * CELLS + cell
+    __shared__ double red[LANES > 1 ? LANES : 1][LANES > 1 ? CELLS : 1][3];
+    const int N = g.N, H = g.H, half = N / 2;
+    const bool rot = cp->any_rot;
+    int gkr0 = 0, gnr = 0, gnc = 0;
+    const float rho_k = fminf(ts.rho, cp->gen_reach);
+    if (rho_k > 0.f) gen_tiles2(g, ts, rho_k, gkr0, gnr, gnc);
+    const int cell = threadIdx.x % CELLS, part = threadIdx.x / CELLS;
+    double vr, vi, vw;
+    auto add = [&](int64_t b, int r, int c, double conj) {
+        const int t = r + half - 1, kr = t / TR, kc = c / TC;
+        if (t < 0) return;  // (the row of an odd box that no tap reaches)
+        int64_t tiles, at;  // of a range, and the tile's place among them
+        if (rot && unsigned(kr - ts.kr0) < unsigned(ts.nr) && kc < ts.nc) {
+            tiles = int64_t(ts.nr) * ts.nc;
+            at = b * ts.ksplit * tiles + (kr - ts.kr0) * int64_t(ts.nc) + kc;
+        } else if (unsigned(kr - gkr0) < unsigned(gnr) && kc < gnc) {
+            tiles = int64_t(gnr) * gnc;
+            at = g.B * ts.ksplit * int64_t(ts.nr) * ts.nc + b * ts.ksplit * tiles + (kr - gkr0) * int64_t(gnc) + kc;
+        } else {
+            return;
+        }
+        const int e = (t - kr * TR) * TC + (c - kc * TC);
+        const char* slot = ts.part + (at + part * tiles) * slot_bytes2(WEIGHTS);
+        const int64_t step = LANES * tiles * slot_bytes2(WEIGHTS);
+#pragma unroll 4
+        for (int j = part; j < ts.ksplit; j += LANES, slot += step) {
+            const Cx<float> v = reinterpret_cast<const Cx<float>*>(slot)[e];
+            vr += double(v.re);
+            vi += conj * double(v.im);
+            if (WEIGHTS) vw += double(reinterpret_cast<const float*>(slot + T2 * 8)[e]);
+        }
+    };
+    const int64_t cells = g.B * g.vol;
+    for (int64_t i0 = int64_t(blockIdx.x) * CELLS; i0 < cells; i0 += int64_t(gridDim.x) * CELLS) {
+        const int64_t i = i0 + cell;
+        vr = vi = vw = 0.0;
+        if (i < cells) {
+            const int64_t b = g.B == 1 ? 0 : i / g.vol;
+            const int q = int(i - b * g.vol), re = q / H, c = q - re * H;
+            auto sg = [&](int k) { return k <= half ? k : k - N; };
+            add(b, sg(re), c, 1.0);
+            if (MIRROR && c == 0 && re != 0 && 2 * re != N) add(b, sg(N - re), 0, -1.0);
+        }
+        if constexpr (LANES > 1) {
+            red[part][cell][0] = vr;
+            red[part][cell][1] = vi;
+            if (WEIGHTS) red[part][cell][2] = vw;
+            __syncthreads();
+            if (part == 0)
+#pragma unroll
+                for (int k = 1; k < LANES; ++k) {
+                    vr += red[k][cell][0];
+                    vi += red[k][cell][1];
+                    if (WEIGHTS) vw += red[k][cell][2];
+                }
+            __syncthreads();
+        }
+        if (part == 0 && i < cells) {
+            dst[i] = Cx<float>{float(vr), float(vi)};
+            if (WEIGHTS) wdst[i] = float(vw);
+        }
     }
 }
 
@@ -590,15 +703,24 @@ unsigned grid2_of(int64_t items, const void* kernel) {
     return grid_for(slots > most ? most : slots);
 }
 
-template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool PRIV, bool GEN>
-hipError_t scatter2_one(const Geom& g, const TileSpec2& ts, const void* src, const void* weights, const void* rot,
+template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool PRIV, bool GEN, bool SLOTS>
+hipError_t scatter2_with(const Geom& g, const TileSpec2& ts, const void* src, const void* weights, const void* rot,
                         const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
     const int64_t work = g.B * ts.ksplit * (GEN ? int64_t(ts.nr_2) * ts.nc_2 : int64_t(ts.nr) * ts.nc);
     if (work == 0) return hipSuccess;
-    const auto k = k_scatter2_tiled<CUBIC, MODE, WEIGHTS, KP, PRIV, GEN>;
+    const auto k = k_scatter2_tiled<CUBIC, MODE, WEIGHTS, KP, PRIV, GEN, SLOTS>;
     hipLaunchKernelGGL(k, dim3(grid2_of<GEN>(work, (const void*)k)), dim3(kThreads), 0, s, g, ts, (const Cx<float>*)src, (const float*)weights, (const float*)rot,
                        (const float*)shifts, (Cx<float>*)dst, (float*)wdst, cp, gl);
     return hipGetLastError();
+}
+
+template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool PRIV, bool GEN>
+hipError_t scatter2_one(const Geom& g, const TileSpec2& ts, const void* src, const void* weights, const void* rot,
+                        const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
+    return ts.part ? scatter2_with<CUBIC, MODE, WEIGHTS, KP, PRIV, GEN, true>(g, ts, src, weights, rot, shifts, dst,
+                                                                             wdst, cp, gl, s)
+                   : scatter2_with<CUBIC, MODE, WEIGHTS, KP, PRIV, GEN, false>(g, ts, src, weights, rot, shifts, dst,
+                                                                              wdst, cp, gl, s);
 }
 
 // Poses per wave batch, and wave-private accumulation: one pose per window keeps a window's
@@ -614,15 +736,27 @@ hipError_t scatter2_kp(const Geom& g, const TileSpec2& ts, const void* src, cons
     return scatter2_one<CUBIC, MODE, WEIGHTS, 1, false, GEN>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
 }
 
-// Rotations, then the other tiled poses (both add into the zero-filled image), then the
-// x = 0 completion of the backprojection.
+// Rotations, then the other tiled poses (both into the slots, or added into the zero-filled image), then
+// the slots' sum and the x = 0 completion of the backprojection.
 template <bool CUBIC, int MODE, bool WEIGHTS>
 hipError_t scatter2_all(const Geom& g, const TileSpec2& ts, const void* src, const void* weights, const void* rot,
                         const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
     hipError_t e = scatter2_kp<CUBIC, MODE, WEIGHTS, false>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
     if (e != hipSuccess) return e;
     e = scatter2_kp<CUBIC, MODE, WEIGHTS, true>(g, ts, src, weights, rot, shifts, dst, wdst, cp, gl, s);
-    if (e != hipSuccess || MODE != 0) return e;
+    if (e != hipSuccess) return e;
+    if (ts.part) {
+        // (about 1024 workgroups of 256 cells fill the GPU)
+        const int64_t cells = g.B * g.vol;
+        auto finish = [&](auto k, int per) {
+            hipLaunchKernelGGL(k, dim3(unsigned(std::min<int64_t>(65536, (cells + per - 1) / per))), dim3(kBlock), 0,
+                               s, g, ts, (Cx<float>*)dst, (float*)wdst, cp);
+            return hipGetLastError();
+        };
+        return cells >= 1024 * kBlock ? finish(k_finish2<WEIGHTS, MODE == 0, 1>, kBlock)
+                                      : finish(k_finish2<WEIGHTS, MODE == 0, 8>, kBlock / 8);
+    }
+    if (MODE != 0) return hipSuccess;
     int64_t blocks = (g.B * g.N + kBlock - 1) / kBlock;
     if (blocks > 65536) blocks = 65536;
     if (blocks < 1) return hipSuccess;
