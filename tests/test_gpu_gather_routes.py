@@ -23,7 +23,8 @@ MODULES = (test_gpu_carried_windows, test_gpu_golden, test_gpu_graph, test_gpu_h
            test_gpu_oversampling, test_gpu_parity, test_gpu_pose_classes, test_gpu_pose_ranges, test_gpu_random,
            test_gpu_streams, test_gpu_tiled2d, test_zz_no_alloc)
 # no gathers, or no small calls
-LEFT_OUT = ("test_pose_class_predicate_bounds", "test_fourier_transforms_replayed_after_plan_eviction", "test_2d_backprojection_replayed",
+LEFT_OUT = ("test_pose_class_predicate_bounds", "test_fourier_transforms_replayed_after_plan_eviction",
+            "test_2d_backprojection_replayed", "test_3d_scatters_replayed_without_a_workspace",
             "test_many_ranges_match_oracle", "test_precision_does_not_fall_with_the_pose_count",
             "test_strided_inputs_backprojection", "test_half_volume_through_autograd",
             "test_tiled_gathers_past_the_per_pixel_sizes")

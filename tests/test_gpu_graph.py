@@ -165,6 +165,52 @@ def test_2d_backprojection_replayed(gpu, warm):
         assert _rel(data_g, data_e) <= 1e-5 and _rel(wrec_g, wrec_e) <= 1e-5
 
 
+@pytest.mark.parametrize("interp", ["linear", "cubic"])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_3d_scatters_replayed_without_a_workspace(gpu, interp, scaled):
+    """Scatters of 1300 poses captured after an eager call of ten: the stream's workspace has no room for the
+    split tiles' slots, whose pieces are added into the zeroed tiles of the volume instead, by the kernels
+    of the rotations and of the scaled poses."""
+    T = torch.ops.torch_projectors
+    gen = torch.Generator().manual_seed(8087)
+    P, n, os_, N, B = 1300, 24, 2.0, 48, 2
+    vol = torch.randn(B, N, N, N // 2 + 1, generator=gen, dtype=torch.complex64).to(gpu)
+    proj = torch.randn(B, P, n, n // 2 + 1, generator=gen, dtype=torch.complex64).to(gpu)
+    w = torch.rand(B, P, n, n // 2 + 1, generator=gen).to(gpu)
+    rot = _rotations(P, gen)
+    if scaled:
+        rot[:, ::3] *= 1.2
+    rot = rot.to(gpu)
+
+    def both(count):
+        p, r = proj[:, :count].contiguous(), rot[:, :count].contiguous()
+        data, wrec = T.backproject_2d_to_3d_forw(p, w[:, :count].contiguous(), r, None, interp, os_, None)
+        return data, wrec, T.project_3d_to_2d_back(p, vol, r, None, interp, os_, None)[0]
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        both(10)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = both(P)
+    torch.cuda.synchronize()
+    exp = both(P)
+    torch.cuda.synchronize()
+    for replay in range(3):
+        with torch.cuda.stream(stream):
+            both(10)
+        for t in got:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        print(f"[graph] 3D replay {replay} {interp} scaled {scaled}", flush=True)
+        for a, b in zip(got, exp):
+            assert _rel(a, b) <= 1e-5, f"replay {replay}: {_rel(a, b):.3e}"
+
+
 def test_fourier_transforms_replayed_after_plan_eviction(gpu):
     """hipFFT transforms captured after one eager call of their shape on the capture stream, then
     replayed after more distinct shapes on that stream than the plan cache holds (32): the plans a

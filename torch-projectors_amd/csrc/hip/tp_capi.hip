@@ -143,9 +143,10 @@ int64_t forw_poses_per_range(double os) {
     return r >= 2048.0 ? 2048 : (r <= 512.0 || !(r == r) ? 512 : int64_t(r));
 }
 
-// Most pieces of split tiles of one scatter call (12-18 KB of workspace each: up to 2.4 GB) and of one
-// gather call (which needs none); a call of more takes longer pieces.
-constexpr double kMaxScatterPieces = double(1 << 17), kMaxGatherPieces = double(1 << 30);
+// Most pieces of split tiles of one scatter call (12-18 KB of workspace each: up to 604 MB; 32 for each
+// workgroup that runs at once) and of one gather call (which needs none); a call of more takes longer
+// pieces.
+constexpr double kMaxScatterPieces = double(1 << 15), kMaxGatherPieces = double(1 << 30);
 
 // Pose ranges of a 3D tile grid (tp::PoseSplit): n tiles per axis (d, r, c) of `edge` voxels from the
 // signed coordinate `org`, for samples within `reach` of the origin; `stencil` voxels more per axis
@@ -159,18 +160,18 @@ constexpr double kMaxScatterPieces = double(1 << 17), kMaxGatherPieces = double(
 //     poses of 90 x 90 at oversampling 1.5, cubic forward and backward 1.59 -> 0.84 ms; 1000 poses of
 //     64 x 64 at 2, linear: backprojection 0.211 -> 0.124, projection with all gradients 0.549 -> 0.279 ms;
 //     1000 of 64 x 64 at 1, cubic backprojection 3.34 -> 0.65 ms.
-//   - in calls where that is 512 poses or more, one level of 40 voxels with `range` poses per piece: there the levels measured
-//     slower (the headline backprojection 1.33 -> 1.39 ms: less of the projections' rows is shared
-//     by the pieces that run together).
+//   - in calls where that is 512 poses or more (and without `levels`), one level of 40 voxels with `range`
+//     poses per piece: there the levels measured slower (the headline backprojection 1.33 -> 1.39 ms:
+//     less of the projections' rows is shared by the pieces that run together).
 tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const int org[3], const int edge[3],
-                         double stencil, double per_slot, double least, int64_t range, double most) {
+                         double stencil, double per_slot, double least, int64_t range, double most, bool levels = true) {
     constexpr double kSlots = 1024.0, kLongRange = 512.0;
     const double h = 0.25 * (edge[0] + edge[1] + edge[2] + 3.0 * stencil);
     const double vt = double(edge[0]) * edge[1] * edge[2], R = std::max(reach, h);
     const double cross =
         double(g.B) * double(g.P) * 2.0 * M_PI / vt * (h * h * h / 3.0 + h * (R * R - h * h) / 2.0);
     double target = std::max(least, cross / (kSlots * per_slot));
-    const bool one_level = target >= kLongRange;
+    const bool one_level = !levels || target >= kLongRange;
     if (one_level) target = double(range);
     tp::PoseSplit ps{};
     double r = one_level ? 40.0 : 16.0, p = 1.0;  // this level's half width; share of the poses that cross its tiles
@@ -191,7 +192,8 @@ tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const 
         }
         total += double(g.B) * double(tiles) * double(k);
         if (total > most || k > tp::kMaxTilePieces || double(ps.pieces) + double(tiles) * double(k) > double(INT32_MAX))  // (twice as long until they fit)
-            return pose_split(g, reach, n, org, edge, stencil, per_slot / 2.0, 2.0 * target, 2 * int64_t(target), most);
+            return pose_split(g, reach, n, org, edge, stencil, per_slot / 2.0, 2.0 * target, 2 * int64_t(target), most,
+                              levels);
         v.k = int(k);
         v.pieces = int(tiles * k);
         v.by_pieces = tp::divisor(unsigned(v.pieces));
@@ -209,7 +211,18 @@ tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const 
 
 // The op a TileSpec is for: its pose ranges differ.
 enum class TileOp { project, gradients, backproject };
-tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, tp::ForwWorks& fw, tp::ScatterWork& sw) {
+// The scatter's pose ranges.  In large calls its core tiles carry the most work of its grid and take 512
+// poses per piece (at 1024 the headline backprojection took 1.41 ms against 1.34), the backprojection of
+// more than 2048 poses about four pieces of up to 2048 (8192 poses of 128 x 128: 1.369 ms at 512, 1.347 at
+// 2048).  Its pieces, above all the cubic ones, hold more work per pose than the gathers'.
+tp::PoseSplit scatter_split(const tp::Geom& g, const tp::TileSpec& ts, bool cubic, TileOp op, bool levels) {
+    const int half = g.N / 2, n[3] = {ts.ntd, ts.ntr, ts.ntc}, org[3] = {1 - half, 1 - half, 0},
+              edge[3] = {tp::kScTD, tp::kScTR, tp::kScTC};
+    return pose_split(g, double(ts.rho_unit), n, org, edge, cubic ? 3.0 : 1.0, cubic ? 1.5 : 1.0, cubic ? 16.0 : 48.0,
+                      op == TileOp::backproject ? std::min<int64_t>(2048, std::max<int64_t>(512, g.P / 4)) : 512,
+                      kMaxScatterPieces, levels);
+}
+tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, tp::ForwWorks& fw) {
     constexpr int L = tp::kTileEdge;
     tp::TileSpec ts{};
     // radius bound of the active pixels: the cutoff disc, within the pixel grid
@@ -231,32 +244,21 @@ tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, tp::ForwWorks& 
     ts.org2 = -half2 * L;
     ts.ntfd2 = 2 * half2_d;
     ts.orgd2 = -half2_d * tp::kTileEdgeD;
-    const int half = g.N / 2;
     ts.ntd = (g.N + tp::kScTD - 1) / tp::kScTD;
     ts.ntr = (g.N + tp::kScTR - 1) / tp::kScTR;
     ts.ntc = (g.H + tp::kScTC - 1) / tp::kScTC;
-    // Pieces of the tiles' poses.  Measured targets (calls in pose_split's comment): the gathers stage
-    // their tile once per piece and do best with half as many pieces as slots would take; the
-    // scatters' pieces, above all the cubic ones, hold more work per pose.  In large calls the
-    // scatter's core tiles carry the most work of its grid and take 512 poses per piece (at 1024 the
-    // headline backprojection took 1.41 ms against 1.34), the backprojection of more than 2048 poses
-    // about four pieces of up to 2048 (8192 poses of 128 x 128: 1.369 ms at 512, 1.347 at 2048); the
-    // gradient modes and the kernels of the other tiled poses 512 (1-4 % slower at 2048); the forward
+    // Pieces of the gathers' poses (calls in pose_split's comment): they stage their tile once per piece
+    // and do best with half as many pieces as slots would take.  In large calls the gradient modes and the
+    // kernels of the other tiled poses take 512 poses per piece (1-4 % slower at 2048); the forward
     // projection's rotation kernel forw_poses_per_range (at oversampling 2, 4096 poses of 128 x 128 take
     // 0.317 ms at 512 against 0.299 at 2048, the headline the same).
     const int nf[3] = {ts.ntfd, ts.nt, ts.nt}, of[3] = {ts.orgd, ts.org, ts.org}, ef[3] = {tp::kTileEdgeD, L, L};
     const int nf2[3] = {ts.ntfd2, ts.nt2, ts.nt2}, of2[3] = {ts.orgd2, ts.org2, ts.org2};
-    const int nsc[3] = {ts.ntd, ts.ntr, ts.ntc}, osc[3] = {1 - half, 1 - half, 0},
-              esc[3] = {tp::kScTD, tp::kScTR, tp::kScTC};
     const double flo = op == TileOp::project ? 64.0 : 32.0;
     fw.rot.split =
         pose_split(g, rho_unit, nf, of, ef, 0.0, 0.5, flo, op == TileOp::project ? forw_poses_per_range(g.os) : 512,
                    kMaxGatherPieces);
     fw.gen.split = pose_split(g, rho_unit, nf2, of2, ef, 0.0, 0.5, flo, 512, kMaxGatherPieces);
-    sw.split =
-        pose_split(g, rho_unit, nsc, osc, esc, cubic ? 3.0 : 1.0, cubic ? 1.5 : 1.0, cubic ? 16.0 : 48.0,
-                   op == TileOp::backproject ? std::min<int64_t>(2048, std::max<int64_t>(512, g.P / 4)) : 512,
-                   kMaxScatterPieces);
     ts.rho = float(rho);
     ts.rho_unit = float(rho_unit);
     ts.os = float(g.os);
@@ -423,6 +425,8 @@ struct StreamScratch {
     std::mutex busy;
     void* bins = nullptr;  // pose-bin workspace of the tiled 3D kernels, grown on demand
     size_t bins_cap = 0;
+    size_t bins_failed = 0;  // the size that could not be allocated last (0: none), and the calls since
+    int bins_refused = 0;
     // A graph captured on the stream keeps the address of the workspace its calls used, so a
     // workspace that a capture has used is never freed: growing it retires it instead (kept
     // until the process ends; growth is geometric, so these stay a small multiple of the last).
@@ -495,16 +499,17 @@ int noalloc_device(NoAllocDevice*& out) {
 // held until the call returns, with the `busy` lock of its area.  `static_area`:
 // the current GPU's static array (no allocation); otherwise the area of the
 // (device, stream), allocated by the first call on that stream.
+constexpr int kBinsRetry = 256;
 struct CallScratch {
     tp::CallPoses* p = nullptr;
     std::unique_lock<std::mutex> hold;
     bool static_area = false;
     StreamScratch* area = nullptr;  // the (device, stream) area, when not static_area
-    // A pose-bin workspace of `need` bytes on the call's stream, or nullptr: the static area has
-    // none, and a failed allocation leaves the call without bins (the kernels then cull every pose).
+    // A workspace of `need` bytes on the call's stream, or nullptr: the static area has none, and a
+    // failed allocation leaves the call without (plan_scatter, plan_scatter2).
     // Growing waits for the stream's queued work, which may still read the old workspace; a stream
-    // under graph capture can neither wait nor allocate, so there the call goes without bins, and
-    // a workspace that a captured call uses is retired rather than freed when it grows later.
+    // under graph capture can neither wait nor allocate, so there the call goes without what does not
+    // fit, and a workspace that a captured call uses is retired rather than freed when it grows later.
     void* bins(size_t need, hipStream_t st) {
         if (static_area || !area) return nullptr;
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -515,6 +520,10 @@ struct CallScratch {
         const bool capturing = cs != hipStreamCaptureStatusNone;
         if (need > area->bins_cap) {
             if (capturing) return nullptr;
+            // (a size that the last attempt could not get is tried again after kBinsRetry calls: freeing
+            // the workspace and waiting for the stream on each of them would cost more than it can give)
+            if (area->bins_failed && need >= area->bins_failed && area->bins_refused++ < kBinsRetry) return nullptr;
+            area->bins_failed = 0;
             if (hipStreamSynchronize(st) != hipSuccess) return nullptr;
             if (area->bins) {
                 if (area->bins_captured) area->bins_retired.push_back(area->bins);
@@ -526,6 +535,8 @@ struct CallScratch {
             const size_t cap = need + need / 4;
             if (hipMalloc(&area->bins, cap) != hipSuccess) {
                 area->bins = nullptr;
+                area->bins_failed = need;
+                area->bins_refused = 0;
                 (void)hipGetLastError();  // clear the allocation error
                 return nullptr;
             }
@@ -647,19 +658,22 @@ int call_poses(int dim, const tp::Geom& g, const void* rot, float rho_unit, Call
                     "pose summary launch");
 }
 
-// Workspace of the tiled 3D scatter for this call: the slots of the split tiles' pieces
-// (tp::ScatterWork::part), and the pose bins of its tile grid (tp::BinGrid) in 2 x 2 x 2 tiles, which
-// plan_scatter lays out (the pose summary then clears their counts) and fill_bins fills after the
+// The tiled 3D scatter's pose ranges, and its workspace for this call: the slots of the split tiles'
+// pieces (tp::ScatterWork::part), and the pose bins of its tile grid (tp::BinGrid) in 2 x 2 x 2 tiles,
+// which plan_scatter lays out (the pose summary then clears their counts) and fill_bins fills after the
 // summary.  No bins below kBinsMinPoses poses, from 65536 poses (list entries are 16-bit), beyond
-// kBinsMaxBytes or tp::kBinMaxGroups workgroups of the pre-pass; without a workspace (a failed
-// allocation, or growth under graph capture) no bins and no split tiles: every tile then takes all
-// of the call's poses itself.
+// kBinsMaxBytes or tp::kBinMaxGroups workgroups of the pre-pass.  Without room for the slots (a failed
+// allocation, or growth under graph capture) the tiles split in one level, whose pieces are added into
+// the zeroed tiles of the volume with float atomics: calls of up to 512 poses stay whole there.  Both
+// parts are at most 1.6 GB, and the workspace a quarter more.
 constexpr int64_t kBinsMinPoses = 16;
 constexpr size_t kBinsMaxBytes = size_t(1) << 30;
-int plan_scatter(const tp::Geom& g, const tp::TileSpec& ts, tp::ScatterWork& sw, bool weights, CallScratch& sc, hipStream_t s) {
+int plan_scatter(const tp::Geom& g, const tp::TileSpec& ts, bool cubic, TileOp op, tp::ScatterWork& sw, bool weights,
+                 CallScratch& sc, hipStream_t s) {
     TP_TRY(sc.get(s));
+    sw.split = scatter_split(g, ts, cubic, op, true);
     auto align = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t slots = align(size_t(g.B) * size_t(sw.split.pieces) * size_t(tp::slot_bytes(weights)));
+    size_t slots = align(size_t(g.B) * size_t(sw.split.pieces) * size_t(tp::slot_bytes(weights)));
     tp::BinGrid sb{};
     sb.nb[0] = (ts.ntc + 1) / 2;
     sb.nb[1] = (ts.ntr + 1) / 2;
@@ -670,14 +684,14 @@ int plan_scatter(const tp::Geom& g, const tp::TileSpec& ts, tp::ScatterWork& sw,
     if (g.P < kBinsMinPoses || g.P >= 65536 || counts + lists > kBinsMaxBytes ||
         g.B_rot * int64_t(sb.nb[1]) * sb.nb[2] * ((g.P + tp::kBinPoses - 1) / tp::kBinPoses) > tp::kBinMaxGroups)
         counts = lists = 0;
-    const size_t need = slots + counts + lists;
-    char* w = need ? static_cast<char*>(sc.bins(need, s)) : nullptr;
-    if (!w) {
-        sw.split = tp::PoseSplit{};
-        return TP_OK;
+    char* w = slots + counts > 0 ? static_cast<char*>(sc.bins(slots + counts + lists, s)) : nullptr;
+    if (w && slots) sw.part = w;
+    if (!w && slots) {
+        sw.split = scatter_split(g, ts, cubic, op, false);
+        slots = 0;
+        if (counts) w = static_cast<char*>(sc.bins(counts + lists, s));
     }
-    sw.part = w;
-    if (counts) {
+    if (w && counts) {
         sb.count = reinterpret_cast<int*>(w + slots);
         sb.list = reinterpret_cast<unsigned short*>(w + slots + counts);
         sw.bins = sb;
@@ -787,8 +801,7 @@ int project_forw(int dim, int dtype, const void* rec, int64_t B, int64_t D, int6
     }
     if (tiles) {
         tp::ForwWorks fw{};
-        tp::ScatterWork sw{};
-        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::project, fw, sw);
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::project, fw);
         TP_TRY(use_forw_tiles(g, ts, fw, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s));
         TP_TRY(launched(tp::launch_project3_forw_tiled(cubic, g, ts, fw, rec, rot, shifts, out, sc.p, 0, s, rec_half),
@@ -851,8 +864,8 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     if (tiles) {
         tp::ForwWorks fw{};
         tp::ScatterWork sw{};
-        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, fw, sw);
-        TP_TRY(plan_scatter(g, ts, sw, false, sc, s));
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, fw);
+        TP_TRY(plan_scatter(g, ts, cubic, TileOp::gradients, sw, false, sc, s));
         if (tiled_gradients) TP_TRY(use_forw_tiles(g, ts, fw, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, sw.bins));
         TP_TRY(fill_bins(cubic, g, ts, sw, rot, sc, s));
@@ -912,8 +925,8 @@ int backproject_forw(int dim, int dtype, const void* proj, int64_t B, int64_t P,
     if (tiles) {
         tp::ForwWorks fw{};
         tp::ScatterWork sw{};
-        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::backproject, fw, sw);
-        TP_TRY(plan_scatter(g, ts, sw, weights != nullptr, sc, s));
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::backproject, fw);
+        TP_TRY(plan_scatter(g, ts, cubic, TileOp::backproject, sw, weights != nullptr, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s, sw.bins));
         TP_TRY(fill_bins(cubic, g, ts, sw, rot, sc, s));
         TP_TRY(launched(tp::launch_scatter3_tiled(cubic, 0, g, ts, sw, proj, weights, rot, shifts, data, wrec, sc.p, 0, s),
@@ -970,8 +983,7 @@ int backproject_back(int dim, int dtype, const void* gdata, const void* gw, int6
     }
     if (tiles) {
         tp::ForwWorks fw{};
-        tp::ScatterWork sw{};
-        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, fw, sw);
+        const tp::TileSpec ts = tile_spec(g, cubic, TileOp::gradients, fw);
         TP_TRY(use_forw_tiles(g, ts, fw, sc, s));
         TP_TRY(call_poses(3, g, rot, ts.rho_unit, sc, s));
         TP_TRY(launched(tp::launch_bpback3_tiled(cubic, g, ts, fw, gdata, gw, proj, rot, shifts, gproj, gweights, grot,

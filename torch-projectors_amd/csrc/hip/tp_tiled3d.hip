@@ -31,7 +31,8 @@
 //                     them (with the Hermitian x = 0 mirror of the
 //                     backprojection): float atomics into a zeroed region
 //                     left 2 x 333 poses of 90 x 90 (cubic, oversampling 1.5,
-//                     eleven pieces) at 0.94 ms a step, the sums take it to 0.84.
+//                     eleven pieces) at 0.94 ms a step, the sums take it to 0.84;
+//                     they remain where a call has no workspace.
 //
 // Poses whose first two matrix columns a, b have singular values in
 // [kScaleMin, kScaleMax] take this path (pose_tiled3); the per-pixel kernels
@@ -269,13 +270,9 @@ struct Item {
 // The decoding of a work item into its tile and poses is scalar arithmetic on tables that are constant
 // during the kernel, loaded where it needs them.
 template <typename T> using Constant = const __attribute__((address_space(4))) T;
-template <typename T, typename S> __device__ __forceinline__ T scalar_load(S* p) {
-    static_assert(sizeof(T) % 4 == 0, "whole words");
-    T v;
-    Constant<unsigned>* q = (Constant<unsigned>*)p;
-#pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 4; ++i) reinterpret_cast<unsigned*>(&v)[i] = q[i];
-    return v;
+__device__ __forceinline__ Divisor load(Constant<Divisor>* p) { return Divisor{p->m, p->s}; }
+__device__ __forceinline__ PoseSplit::Box load(Constant<PoseSplit::Box>* p) {
+    return PoseSplit::Box{{p->lo[0], p->lo[1], p->lo[2]}, p->ext};
 }
 // The kernel's first argument, of type T, where it stands in memory.  As an ordinary argument, its fields
 // and what the decoding makes of them are loaded at the kernel's start and kept in scalar registers
@@ -292,10 +289,11 @@ __device__ __forceinline__ Item reach_item(Constant<ForwWork>* fw, int64_t w) {
     int l = 0;
 #pragma unroll
     for (int i = 1; i <= kSplitLevels; ++i) l += u >= fw->reach[i].begin;
-    const ReachLevel v = scalar_load<ReachLevel>(&fw->reach[l]);
-    const unsigned n = u - v.begin, b = v.by_per.of(n), q = n - b * v.per, t = v.by_k.of(q);
-    const TileAt f = scalar_load<TileAt>(fw->list + (v.first + t));
-    return Item{int64_t(b), f.d, f.r, f.c, int(q - t * v.k), int(v.k), false};
+    Constant<ReachLevel>* const v = &fw->reach[l];
+    const unsigned n = u - v->begin, b = load(&v->by_per).of(n), q = n - b * v->per, t = load(&v->by_k).of(q);
+    Constant<uint2>* const f = (Constant<uint2>*)(fw->list + (v->first + t));
+    const unsigned dr = f->x, c = f->y;
+    return Item{int64_t(b), int(dr & 0xffffu), int(dr >> 16), int(c & 0xffffu), int(q - t * v->k), int(v->k), false};
 }
 __device__ __forceinline__ Item item_of(int64_t w, int64_t B, int nd, int nr, int nc, int offd, int off,
                                         Constant<PoseSplit>* sp) {
@@ -312,17 +310,18 @@ __device__ __forceinline__ Item item_of(int64_t w, int64_t B, int nd, int nr, in
                 ++l;
             }
         }
-        const PoseSplit::Level v = scalar_load<PoseSplit::Level>(&sp->lv[l]);
+        Constant<PoseSplit::Level>* const v = &sp->lv[l];
+        const PoseSplit::Box box = load(&v->box);
         PoseSplit::Box in{};
-        if (l > 0) in = scalar_load<PoseSplit::Box>(&sp->lv[l - 1].box);  // (the boxes are nested: the next one in holds the others)
-        const unsigned b = v.by_pieces.of(u), q = u - b * unsigned(v.pieces), t = v.by_k.of(q), tr = v.by_c.of(t),
-                       td = v.by_r.of(tr);
+        if (l > 0) in = load(&sp->lv[l - 1].box);  // (the boxes are nested: the next one in holds the others)
+        const unsigned b = load(&v->by_pieces).of(u), q = u - b * unsigned(v->pieces), t = load(&v->by_k).of(q),
+                       tr = load(&v->by_c).of(t), td = load(&v->by_r).of(tr);
         it.b = b;
-        it.j = int(q - t * unsigned(v.k));
-        it.k = v.k;
-        it.kc = v.box.lo[2] + int(t - tr * unsigned(v.box.size(2)));
-        it.kr = v.box.lo[1] + int(tr - td * unsigned(v.box.size(1)));
-        it.kd = v.box.lo[0] + int(td);
+        it.j = int(q - t * unsigned(v->k));
+        it.k = v->k;
+        it.kc = box.lo[2] + int(t - tr * unsigned(box.size(2)));
+        it.kr = box.lo[1] + int(tr - td * unsigned(box.size(1)));
+        it.kd = box.lo[0] + int(td);
         it.skip = in.holds(it.kd, it.kr, it.kc);
     } else {
         const int64_t per_b = int64_t(nd) * nr * nc;
@@ -334,7 +333,7 @@ __device__ __forceinline__ Item item_of(int64_t w, int64_t B, int nd, int nr, in
         it.kd = offd + t / (nc * nr);
         it.j = 0;
         it.k = 1;
-        it.skip = scalar_load<PoseSplit::Box>(&sp->box).holds(it.kd, it.kr, it.kc);
+        it.skip = load(&sp->box).holds(it.kd, it.kr, it.kc);
     }
     return it;
 }
@@ -689,8 +688,10 @@ __attribute__((amdgpu_waves_per_eu(forw_waves_per_eu<CUBIC, GMODE, VS, GEN>())))
         const int64_t wi = xcd_item<kRunForw>(slot_i);
         if (wi >= items) continue;
         Constant<ForwWork>* const work = first_argument<ForwWork>();
+        int nr = nt, nd = ntd;
+        if constexpr (!GEN) asm("" : "+s"(nr), "+s"(nd));  // (nor are their products and reciprocals kept)
         const Item it = uniform(!GEN && work->list ? reach_item(work, wi)
-                                                   : item_of(wi, g.B, ntd, nt, nt, offd, off, &work->split));
+                                                   : item_of(wi, g.B, nd, nr, nr, offd, off, &work->split));
         if (it.skip) continue;
         const int64_t b = it.b;
         const int tc = org + it.kc * L, tr = org + it.kr * L, td = orgd + it.kd * LD;
@@ -1394,9 +1395,11 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
         // write every stored cell of the tile once: a piece of a split tile into its slot of the
         // workspace (k_finish3 sums them), other tiles into the volume.  GEN adds onto what the
         // rotation kernel wrote (one workgroup each, so by a plain read and write); without
-        // rotations in the call it stores.
+        // rotations in the call it stores.  Without a workspace a split tile's pieces are added into the
+        // volume, zero in those tiles (k_zero_split3).
+        const bool slotted = split && sw.part, adds = split && !sw.part;
         const bool onto = GEN && any_rot && (!split || dist2 <= (ts.rho_unit + 1.0f) * (ts.rho_unit + 1.0f));
-        if (GEN && any_rot && !touched && (onto || empty)) continue;
+        if (GEN && (any_rot || adds) && !touched && (onto || empty || adds)) continue;
         if (empty && split) continue;  // (k_finish3 reads no piece of a tile beyond every reach)
         __syncthreads();
         {
@@ -1404,19 +1407,23 @@ __global__ __launch_bounds__(kScatterThreads) __attribute__((amdgpu_waves_per_eu
             static_assert(NT % (SC * SR) == 0, "write-out lanes keep their column and row");
             const int lc = tid % SC, lr = (tid / SC) % SR;
             const int c = tc + lc, r = tr + lr;
-            if (split || (c < H && r <= half)) {
+            if (slotted || (c < H && r <= half)) {
                 // (a slot: the tile's values, then its weights)
                 char* const slot = sw.part + xcd_item<kRunScatter>(sl.s) * slot_bytes(WEIGHTS);
-                Cx<float>* const out = split ? reinterpret_cast<Cx<float>*>(slot) : dst;
-                float* const wout = split ? reinterpret_cast<float*>(slot + S3 * 8) : wdst;
-                const int64_t row = split ? lr * SC + lc : b * g.vol + int64_t(r < 0 ? r + N : r) * H + c;
-                const int plane = split ? SR * SC : N * H;
-                const int last = split ? SD - 1 : min(SD - 1, half - td);
+                Cx<float>* const out = slotted ? reinterpret_cast<Cx<float>*>(slot) : dst;
+                float* const wout = slotted ? reinterpret_cast<float*>(slot + S3 * 8) : wdst;
+                const int64_t row = slotted ? lr * SC + lc : b * g.vol + int64_t(r < 0 ? r + N : r) * H + c;
+                const int plane = slotted ? SR * SC : N * H;
+                const int last = slotted ? SD - 1 : min(SD - 1, half - td);
                 for (int ld = tid / (SC * SR); ld <= last; ld += NT / (SC * SR)) {
-                    const int d = split ? ld : td + ld;
+                    const int d = slotted ? ld : td + ld;
                     const int64_t idx = row + int64_t(d < 0 ? d + N : d) * plane;
                     const int a = (ld * SR + lr) * SC + ((lc + acc_swizzle(lr, ld)) & (SC - 1));
-                    if (onto) {
+                    if (adds) {
+                        atomic_add(&dst[idx].re, float(acc_re[a]));
+                        atomic_add(&dst[idx].im, float(acc_im[a]));
+                        if (WEIGHTS) atomic_add(&wdst[idx], float(acc_w[a]));
+                    } else if (onto) {
                         const Cx<float> o = out[idx];
                         out[idx] = Cx<float>{o.re + float(acc_re[a]), o.im + float(acc_im[a])};
                         if (WEIGHTS) wout[idx] += float(acc_w[a]);
@@ -1565,6 +1572,25 @@ __global__ __launch_bounds__(kBlock) void k_finish3(Geom g, TileSpec ts, Scatter
     }
 }
 
+// Zero the stored cells of the split tiles, one workgroup per tile of the outermost level's box (a scatter
+// without a workspace adds their pieces into them).
+template <bool WEIGHTS>
+__global__ __launch_bounds__(kBlock) void k_zero_split3(Geom g, PoseSplit::Box v, Cx<float>* __restrict__ dst,
+                                                        float* __restrict__ wdst) {
+    const int N = g.N, H = g.H, half = N / 2, nc = v.size(2), nr = v.size(1);
+    const int per_b = v.size(0) * nr * nc, t = int(blockIdx.x % unsigned(per_b));
+    const int64_t b = blockIdx.x / unsigned(per_b);
+    const int tc = (v.lo[2] + t % nc) * SC, tr = -half + 1 + (v.lo[1] + (t / nc) % nr) * SR,
+              td = -half + 1 + (v.lo[0] + t / (nc * nr)) * SD;
+    for (int e = threadIdx.x; e < S3; e += kBlock) {
+        const int c = tc + e % SC, r = tr + (e / SC) % SR, d = td + e / (SC * SR);
+        if (c >= H || r > half || d > half) continue;
+        const int64_t idx = b * g.vol + (int64_t(d < 0 ? d + N : d) * N + (r < 0 ? r + N : r)) * H + c;
+        dst[idx] = Cx<float>{0.f, 0.f};
+        if (WEIGHTS) wdst[idx] = 0.f;
+    }
+}
+
 // Pose bins (launch_pose_bins): one workgroup per rotation batch item, row of bins along c (bins
 // differ there only in their c extent) and block of kBinPoses poses, so each pose is loaded once per
 // row.  A lane tests its poses against every bin of the row with the tiles' plane test (a bit per
@@ -1710,6 +1736,14 @@ hipError_t forw_both(const Geom& g, const TileSpec& ts, const ForwWorks& fw, con
 template <bool CUBIC, int MODE, bool WEIGHTS, int KP, bool OSX>
 hipError_t scatter_launch(const Geom& g, const TileSpec& ts, const ScatterWork& sw, const void* src, const void* weights, const void* rot,
                           const void* shifts, void* dst, void* wdst, CallPoses* cp, int gl, hipStream_t s) {
+    const bool adds = sw.split.pieces > 0 && !sw.part;
+    if (adds) {
+        const PoseSplit::Box& v = sw.split.box;
+        hipLaunchKernelGGL(k_zero_split3<WEIGHTS>, dim3(unsigned(g.B * v.size(0) * v.size(1) * v.size(2))), dim3(kBlock),
+                           0, s, g, v, (Cx<float>*)dst, (float*)wdst);
+        const hipError_t ez = hipGetLastError();
+        if (ez != hipSuccess) return ez;
+    }
     // rotations write every tile (none: the other tiled poses store them); the other tiled
     // poses add onto them
     const int64_t work = g.B * (sw.split.pieces + int64_t(ts.ntd) * ts.ntr * ts.ntc);
@@ -1727,12 +1761,14 @@ hipError_t scatter_launch(const Geom& g, const TileSpec& ts, const ScatterWork& 
                        (Cx<float>*)dst, (float*)wdst, cp, gl);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const PoseSplit::Box& outer = sw.split.box;
+    ScatterWork fin = sw;
+    if (adds) fin.split = PoseSplit{};  // (no slots to sum)
+    const PoseSplit::Box& outer = fin.split.box;
     const int64_t red = kFinishParts * g.B * int64_t(outer.size(0)) * outer.size(1) * outer.size(2);
     int64_t blocks = 0;
     if (MODE == 0) blocks = std::min<int64_t>(65536, (g.B * int64_t(g.N) * g.N + kBlock - 1) / kBlock);
     if (red + blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_finish3<CUBIC, WEIGHTS, MODE == 0>), dim3(unsigned(red + blocks)), dim3(kBlock), 0, s, g, ts, sw, red,
+    hipLaunchKernelGGL((k_finish3<CUBIC, WEIGHTS, MODE == 0>), dim3(unsigned(red + blocks)), dim3(kBlock), 0, s, g, ts, fin, red,
                        (Cx<float>*)dst, (float*)wdst, cp);
     return hipGetLastError();
 }
