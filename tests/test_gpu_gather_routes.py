@@ -27,7 +27,7 @@ LEFT_OUT = ("test_pose_class_predicate_bounds", "test_fourier_transforms_replaye
             "test_2d_backprojection_replayed", "test_3d_scatters_replayed_without_a_workspace",
             "test_many_ranges_match_oracle", "test_precision_does_not_fall_with_the_pose_count",
             "test_strided_inputs_backprojection", "test_half_volume_through_autograd",
-            "test_tiled_gathers_past_the_per_pixel_sizes")
+            "test_tiled_gathers_past_the_per_pixel_sizes", "test_small_calls_run_per_pixel")
 
 
 def _has_gathers(param):

@@ -9,6 +9,7 @@ import pytest
 
 from tests.golden.cases import _case, make_inputs
 from tests.parity import check_outputs, scatter_cells
+from torch_projectors import capi
 
 pytestmark = pytest.mark.gpu
 
@@ -54,18 +55,35 @@ def test_pose_ranges_match_oracle(case, hip, oracle):
                   cells=scatter_cells(case["op"], args, oracle))
 
 
-# Calls just past the size where the tile-owner gathers take over from the per-pixel ones: small boxes
-# with many poses (the other tests' small calls run per pixel).
+@pytest.mark.parametrize("op,n,os_,P,cut", [
+    ("project_3d_to_2d_forw", 64, 2.0, 40, None), ("project_2d_forw", 1024, 2.0, 2, None),
+    ("project_3d_to_2d_back", 48, 1.0, 60, None), ("backproject_2d_to_3d_back", 48, 2.0, 60, 9.0),
+    ("project_2d_back", 64, 0.5, 40, None), ("backproject_2d_back", 100, 3.0, 40, 30.0)])
+def test_small_calls_run_per_pixel(op, n, os_, P, cut, hip, oracle):
+    case = _case("small", op, interp="linear", os=os_, cutoff=cut, B=1, P=P, n=n, seed=775000 + n)
+    args, tensors = make_inputs(case)
+    got = getattr(hip, op)(*args)
+    assert capi.lib().tp_last_gather_route() == capi.ROUTE_PER_PIXEL
+    exp = getattr(oracle, op)(*args)
+    check_outputs(op, got, exp, has_shifts=tensors.get("shifts") is not None, label=op,
+                  cells=scatter_cells(op, args, oracle))
+
+
+# Calls just past the size where the tile-owner gathers take over from the per-pixel ones (the other tests'
+# small calls run per pixel): volumes small and large for the caches, every oversampling range, cutoffs,
+# 2D images beyond an XCD's L2 and poses of many blocks.
 def _large_cases():
     out, seed = [], 772000
     for op, interp, n, os_, P, B, cut in (
-            ("project_3d_to_2d_forw", "linear", 30, 2.0, 3001, 1, None), ("project_3d_to_2d_forw", "linear", 32, 3.0, 700, 2, 9.5),
-            ("project_3d_to_2d_forw", "cubic", 24, 2.0, 1100, 1, None), ("project_3d_to_2d_forw", "cubic", 34, 1.3, 1500, 1, 15.0),
-            ("project_3d_to_2d_back", "linear", 30, 2.0, 3300, 1, None), ("project_3d_to_2d_back", "cubic", 26, 1.5, 1200, 1, None),
-            ("backproject_2d_to_3d_back", "linear", 30, 2.0, 3300, 1, None), ("backproject_2d_to_3d_back", "cubic", 28, 1.0, 500, 2, 12.0),
-            ("project_2d_forw", "cubic", 48, 3.0, 4000, 1, None), ("project_2d_forw", "linear", 256, 1.0, 1900, 1, None),
-            ("project_2d_back", "linear", 150, 1.5, 21, 2, None), ("project_2d_back", "cubic", 146, 2.0, 18, 1, 60.0),
-            ("backproject_2d_back", "linear", 150, 0.75, 21, 2, 50.0), ("backproject_2d_back", "cubic", 146, 2.0, 18, 1, None)):
+            ("project_3d_to_2d_forw", "linear", 66, 2.0, 1400, 1, None), ("project_3d_to_2d_forw", "linear", 63, 3.0, 1000, 1, None),
+            ("project_3d_to_2d_forw", "linear", 128, 1.3, 500, 1, 60.0),
+            ("project_3d_to_2d_forw", "cubic", 50, 2.0, 400, 1, None), ("project_3d_to_2d_forw", "cubic", 62, 1.3, 600, 2, 25.0),
+            ("project_3d_to_2d_back", "linear", 70, 2.0, 2100, 1, None), ("project_3d_to_2d_back", "cubic", 80, 1.5, 400, 1, None),
+            ("backproject_2d_to_3d_back", "linear", 70, 2.0, 2100, 1, None), ("backproject_2d_to_3d_back", "cubic", 90, 1.0, 500, 2, 40.0),
+            ("project_2d_forw", "cubic", 48, 3.0, 6000, 1, None), ("project_2d_forw", "linear", 513, 2.0, 65, 1, None),
+            ("project_2d_forw", "cubic", 514, 2.0, 10, 2, None),
+            ("project_2d_back", "linear", 150, 1.5, 21, 2, None), ("project_2d_back", "cubic", 200, 2.0, 18, 1, 90.0),
+            ("backproject_2d_back", "linear", 150, 0.75, 500, 2, 50.0), ("backproject_2d_back", "cubic", 146, 2.0, 18, 1, None)):
         seed += 1
         out.append(_case(f"large_{op}_{interp}_n{n}_os{os_:g}_P{P}", op, interp=interp, os=os_, cutoff=cut, B=B, P=P, n=n,
                          B_rot=B, seed=seed, weights=(seed % 2 == 0)))
@@ -85,6 +103,7 @@ def test_tiled_gathers_past_the_per_pixel_sizes(case, hip, oracle):
     args[at] = rot.requires_grad_(args[at].requires_grad)
     print(f"[large] {case['name']}", flush=True)
     got = getattr(hip, case["op"])(*args)
+    assert capi.lib().tp_last_gather_route() == capi.ROUTE_TILES
     exp = getattr(oracle, case["op"])(*args)
     check_outputs(case["op"], got, exp, has_shifts=tensors.get("shifts") is not None, label=case["name"],
                   cells=scatter_cells(case["op"], args, oracle))

@@ -355,34 +355,56 @@ void pose_ranges2(const tp::Geom& g, tp::TileSpec2& ts, int64_t ksplit) {
 // Calls small enough that the per-pixel gathers beat the tile-owner ones (fp32, complex-half volumes
 // too).  A tiled gather pays for its tiles whatever the call samples (staging, culling, two launches
 // that a call of rotations leaves at once, a zero fill or a completion pass); a per-pixel one is a
-// single launch that reads every tap through the caches.  The lines below were fitted to both sides
-// measured over 64 <= n <= 256, 8 to 4000 poses, in us (tiled / per pixel):
-//   forward, linear: 41 poses of 96 at oversampling 2, 30 / 10; 200 of 64 25 / 14; 200 of 128 56 / 58;
-//     40 of 256 216 / 56, 200 of them 286 / 270; at oversampling 1, whose samples share lines, 200 of 128
-//     44 / 24, 1000 of them 95 / 103; cubic, 40 of 128 at 2 84 / 73, 200 of them 117 / 319;
-//   forward 2D, linear: 256 of 64 24 / 10, 8 x 4000 of 64 489 / 414, 8 x 2000 of 128 706 / 741; cubic, 200
-//     of 128 44 / 26, 2000 of them 179 / 211;
-//   gradient gathers (a projection or backprojection with every gradient): 200 of 64 136 / 99, 1000 of
-//     64 263 / 206, 1000 of 128 595 / 601, at oversampling 1 200 of 256 416 / 534; cubic, 200 of 64
-//     268 / 273.  In 2D a pose of many blocks waits for its own sums' atomics: 50 of 256 133 / 164,
-//     so those boxes stay tiled.
+// single launch that reads every tap through the caches, cheaper per sample the smaller the volume
+// and, at small oversampling, the closer the samples.  The lines below were fitted to both sides
+// measured over 32 <= n <= 2048, oversampling 0.5 to 3, 2 to 60000 poses (393 calls: the slower side is
+// taken by at most 6 % in favour of per pixel, and where noted in favour of the tiles), in us (tiled /
+// per pixel):
+//   forward, linear: 100 poses of 48 at oversampling 2, 27 / 11; 1000 of 64 58 / 54, 2000 80 / 98; 100 of
+//     128 54 / 37, 300 of them 66 / 90; 100 of 256 246 / 146, 200 277 / 282; 200 of 512 1795 / 1473, 400
+//     2020 / 2889; at oversampling 1, whose samples share lines, 4000 of 64 130 / 80, 700 of 128 85 / 78, 1500
+//     137 / 155; cubic, 60 of 64 at 2 44 / 38, 150 52 / 64; 40 of 256 361 / 325, 100 470 / 753; 60 of 512
+//     2301 / 2608;
+//   forward 2D, linear: 8 x 4000 of 64 482 / 379, 8 x 2000 of 128 710 / 714, 8 x 300 of 256 452 / 432 and 600
+//     805 / 844; an image that outgrows an XCD's L2 costs a per-pixel sample twice as much: 10 of 1024 at
+//     oversampling 2 49 / 78, 100 312 / 682 (30 of 1024 at 1, 140 / 94); cubic, 500 of 128 73 / 61, 1000
+//     111 / 113; 10 of 1024 75 / 162;
+//   gradient gathers (with every gradient; projection, then backprojection): 1000 of 64 238 / 162 and
+//     167 / 111 (2000 of them, 368 / 249 and 262 / 205, still take the tiles); 200 of 128 234 / 173 and
+//     162 / 140, 500 338 / 293 (tiles) and 242 / 304; 200 of 256 906 / 814 and 744 / 645; cubic, 90 of 64
+//     168 / 147 and 105 / 75, 150 of 128 369 / 456 and 274 / 371.  2D: 600 of 64 78 / 65 and 60 / 46, 400 of 128
+//     109 / 131 and 78 / 84; a pose of many blocks waits for its own sums' atomics (60 of 200, 97 / 104
+//     and 71 / 74), so those boxes stay tiled.
 // Projections of a call's active pixels and the tiles that its samples reach:
 double active_samples(const tp::Geom& g) { return 0.785 * double(g.B) * double(g.P) * double(g.rect); }
+double reach_of(const tp::Geom& g) { return std::min(g.os * std::sqrt(std::max(0.0, g.cut2)), g.os * double(g.n)); }
 double reached_tiles(const tp::Geom& g) {
-    const double R = std::min(g.os * std::sqrt(std::max(0.0, g.cut2)), g.os * double(g.n));
+    const double R = reach_of(g);
     return 4.19 * R * R * R / double(tp::kTileEdge * tp::kTileEdge * tp::kTileEdgeD);
 }
+// (and cells: the volume's at the default cutoff)
+double reached_cells(const tp::Geom& g) { return std::min(double(g.vol), 4.0 * std::pow(reach_of(g), 3.0) + 1.0); }
+// 2 / oversampling within the measured range, 1 above it
+double samples_shared(const tp::Geom& g) { return std::min(4.0, std::max(1.0, 2.0 / g.os)); }
 bool small_forward(int dim, const tp::Geom& g, bool cubic) {
-    const double A = active_samples(g), apart = 2.0 / g.os;
-    if (dim == 2) return A < (cubic ? 4.5e6 * apart : 4.8e7);
-    const double tiles = double(g.B) * reached_tiles(g);
-    return A < (cubic ? 0.15e6 * apart * apart + 55.0 * tiles : 0.9e6 * apart * apart + 180.0 * tiles);
+    const double A = active_samples(g), shared = samples_shared(g);
+    if (dim == 2) {
+        const double vol = double(g.vol), large = std::sqrt(1e6 / vol);
+        const bool beyond_l2 = vol > double(1 << 18);
+        if (cubic) return A < (beyond_l2 ? 1.25e6 * large : 4.5e6) * shared;
+        if (beyond_l2) return A < 4e6 * large * std::min(4.0, shared * shared);
+        return A < (vol <= 40000.0 ? 9e7 : 5.5e7);
+    }
+    const double tiles = reached_tiles(g), cells = reached_cells(g);
+    if (cubic) return A < 0.15e6 * shared * shared * (1.0 + 0.2e6 / cells) + 44.0 * double(g.B) * tiles / (1.0 + tiles / 4e5);
+    return A < 0.75e6 * std::pow(shared, 1.5) * (1.0 + 1.3e6 / cells) + 150.0 * double(g.B) * tiles;
 }
 bool small_gradients(int dim, const tp::Geom& g, bool cubic) {
-    const double A = active_samples(g);
-    if (dim == 2) return A < (cubic ? 1.0e6 : 1.5e6) && g.chunks <= 40;
-    const double tiles = double(g.B) * reached_tiles(g) * std::min(4.0, g.os * g.os / 4.0);
-    return A < (cubic ? 0.25e6 + 40.0 * tiles : 1.0e6 + 300.0 * tiles);
+    const double A = active_samples(g), shared = samples_shared(g);
+    if (dim == 2) return A < (cubic ? 1.0e6 : 1.5e6) * shared && g.chunks <= 40;
+    const double tiles = double(g.B) * reached_tiles(g) * std::min(4.0, g.os * g.os / 4.0), cells = reached_cells(g);
+    return A < (cubic ? 0.25e6 * std::min(2.0, shared) * (1.0 + 0.4e6 / cells) + 40.0 * tiles
+                      : 1.0e6 * (1.0 + 1.7e6 / cells) + 270.0 * tiles);
 }
 
 // The calling thread's tp_set_gather_route, and the gathers its last call took.
