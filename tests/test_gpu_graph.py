@@ -165,9 +165,16 @@ def test_2d_backprojection_replayed(gpu, warm):
         assert _rel(data_g, data_e) <= 1e-5 and _rel(wrec_g, wrec_e) <= 1e-5
 
 
+@pytest.fixture(scope="module")
+def few_poses_stream(gpu):
+    """A stream whose eager calls have few poses, so that its workspace stays small (one for all tests that
+    need it: torch deals its streams from a pool of 32)."""
+    return torch.cuda.Stream()
+
+
 @pytest.mark.parametrize("interp", ["linear", "cubic"])
 @pytest.mark.parametrize("scaled", [False, True])
-def test_3d_scatters_replayed_without_a_workspace(gpu, interp, scaled):
+def test_3d_scatters_replayed_without_a_workspace(gpu, few_poses_stream, interp, scaled):
     """Scatters of 1300 poses captured after an eager call of ten: the stream's workspace has no room for the
     split tiles' slots, whose pieces are added into the zeroed tiles of the volume instead, by the kernels
     of the rotations and of the scaled poses."""
@@ -187,7 +194,7 @@ def test_3d_scatters_replayed_without_a_workspace(gpu, interp, scaled):
         data, wrec = T.backproject_2d_to_3d_forw(p, w[:, :count].contiguous(), r, None, interp, os_, None)
         return data, wrec, T.project_3d_to_2d_back(p, vol, r, None, interp, os_, None)[0]
 
-    stream = torch.cuda.Stream()
+    stream = few_poses_stream
     stream.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(stream):
         both(10)

@@ -19,8 +19,13 @@ def _rel(a, b):
     return ((a - b).norm() / b.norm()).item()
 
 
+@pytest.fixture(scope="module")
+def stream(gpu):
+    return torch.cuda.Stream()
+
+
 @pytest.mark.parametrize("interp,os_", [("linear", 2.0), ("cubic", 1.0)])
-def test_other_pose_counts_only_enqueue(gpu, interp, os_):
+def test_other_pose_counts_only_enqueue(gpu, stream, interp, os_):
     n, B, most = 48, 2, 640
     N = capi.rec_boxsize(n, os_)
     g = torch.Generator().manual_seed(515)
@@ -40,7 +45,6 @@ def test_other_pose_counts_only_enqueue(gpu, interp, os_):
 
     was = capi.lib().tp_set_gather_route(capi.ROUTE_TILES)
     try:
-        stream = torch.cuda.Stream()
         stream.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(stream):
             for P in (most, 320, 160, 80, 40, 20, 10):

@@ -11,6 +11,7 @@ tiled sources are compiled here for it. Three budgets are checked:
   workgroups per CU the compiler assumes must fit in 160 KB.
 * The kernels of the measured workloads keep their registers without spills (scratch 0).
 * The headline forward and backprojection keep four workgroups (16 waves) per CU.
+* The fused transforms' kernels keep their registers without spills too (their LDS is the launch's).
 """
 import os
 import re
@@ -62,8 +63,8 @@ def _report(src):
     return r.stderr
 
 
-def _kernels(text):
-    """{mangled name: {VGPRs, ScratchSize, Occupancy, LDS}} of the device functions in a report."""
+def _kernels(text, kind="_tiled"):
+    """{mangled name: {VGPRs, ScratchSize, Occupancy, LDS}} of the kernels of that kind in a report."""
     out, cur = {}, None
     for line in text.splitlines():
         m = re.search(r"Function Name: (\S+)", line)
@@ -77,7 +78,7 @@ def _kernels(text):
             m = re.search(pat, line)
             if m and key not in cur:
                 cur[key] = int(m.group(1))
-    return {k: v for k, v in out.items() if "_tiled" in k and "Occupancy" in v and "LDS" in v}
+    return {k: v for k, v in out.items() if kind in k and "Occupancy" in v and "LDS" in v}
 
 
 @pytest.fixture(scope="module")
@@ -112,3 +113,10 @@ def test_headline_kernels_keep_four_workgroups_per_cu(kernels, frag):
     (n, k), = [(n, k) for n, k in kernels.items() if frag in n]
     granular = -(-k["LDS"] // GRANULE) * GRANULE
     assert k["Occupancy"] >= 4 and 4 * granular <= LDS_PER_CU, (n, k)
+
+
+def test_fused_transforms_are_spill_free():
+    ks = _kernels(_report("tp_fft.hip"), "k_fft_")
+    assert ks, "no fused transforms in the resource report"
+    bad = {n: k["ScratchSize"] for n, k in ks.items() if k["ScratchSize"]}
+    assert not bad, bad

@@ -6,11 +6,11 @@
 // that are accumulated, and enqueues the kernels on the caller's stream.
 // The memory besides the caller's is kept per (device, stream) for the life
 // of the process: a small scratch area that the calls of the tiled kernels use
-// (tp::CallPoses: a summary of their poses and work counters), the
-// last lists of 3D forward tiles, and the 3D scatters' workspace (pose bins, partial sums of
-// split tiles).  Nothing is synchronised except where a call lists a new
-// geometry or outgrows that workspace.  tp_project_3d_to_2d_forw_noalloc uses a
-// static device array and neither list nor workspace.
+// (tp::CallPoses: a summary of their poses and work counters), the last lists of
+// 3D forward tiles, and the scatters' workspace (pose bins, partial sums of split
+// tiles and pose ranges).  Nothing is synchronised except where a call lists a
+// new geometry or outgrows that workspace.  tp_project_3d_to_2d_forw_noalloc uses
+// a static device array and neither list nor workspace.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -383,7 +383,10 @@ double reached_tiles(const tp::Geom& g) {
     return 4.19 * R * R * R / double(tp::kTileEdge * tp::kTileEdge * tp::kTileEdgeD);
 }
 // (and cells: the volume's at the default cutoff)
-double reached_cells(const tp::Geom& g) { return std::min(double(g.vol), 4.0 * std::pow(reach_of(g), 3.0) + 1.0); }
+double reached_cells(const tp::Geom& g) {
+    const double R = reach_of(g);
+    return std::min(double(g.vol), 4.0 * R * R * R + 1.0);
+}
 // 2 / oversampling within the measured range, 1 above it
 double samples_shared(const tp::Geom& g) { return std::min(4.0, std::max(1.0, 2.0 / g.os)); }
 bool small_forward(int dim, const tp::Geom& g, bool cubic) {
@@ -397,7 +400,7 @@ bool small_forward(int dim, const tp::Geom& g, bool cubic) {
     }
     const double tiles = reached_tiles(g), cells = reached_cells(g);
     if (cubic) return A < 0.15e6 * shared * shared * (1.0 + 0.2e6 / cells) + 44.0 * double(g.B) * tiles / (1.0 + tiles / 4e5);
-    return A < 0.75e6 * std::pow(shared, 1.5) * (1.0 + 1.3e6 / cells) + 150.0 * double(g.B) * tiles;
+    return A < 0.75e6 * shared * std::sqrt(shared) * (1.0 + 1.3e6 / cells) + 150.0 * double(g.B) * tiles;
 }
 bool small_gradients(int dim, const tp::Geom& g, bool cubic) {
     const double A = active_samples(g), shared = samples_shared(g);

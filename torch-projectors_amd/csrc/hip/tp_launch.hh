@@ -46,7 +46,7 @@ constexpr int kScTC = 16, kScTR = 8, kScTD = 12;        // scatter tiles (c, r, 
 // Pose bins of the scatter tile grid, filled per call by launch_pose_bins: for each block of
 // 2 x 2 x 2 tiles (a bin) and rotation batch item, the poses whose slice plane crosses the bin's
 // box, in no particular order (any matrix: the plane is spanned by its first two columns).  The
-// scatter's tiles outside the core then cull only their bin's poses instead of all P, in fewer and
+// scatter's whole tiles then cull only their bin's poses instead of all P, in fewer and
 // fuller phases.  list == nullptr: no bins (every tile culls all its poses).
 constexpr int kBinPoses = 1024;  // poses per workgroup of the bin pre-pass
 constexpr int64_t kBinMaxGroups = (int64_t(1) << 24) - 1;  // most workgroups of one bin pre-pass (256 lanes each

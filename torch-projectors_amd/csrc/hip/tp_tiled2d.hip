@@ -15,10 +15,11 @@
 // flips to (-c, -r) and conjugates), then enumerates exactly the samples of
 // each such pose whose stencil reaches the box: one lane per (pose, row)
 // computes the row's column interval, a wave prefix sum packs the samples of
-// KP poses densely onto the lanes.  Partial tiles of the pose ranges are
-// added into the zero-filled image with float atomics (once per cell and
-// range).  The x = 0 Hermitian completion of the backprojection is applied
-// afterwards by k_mirror2_x0.
+// KP poses densely onto the lanes.  Partial tiles of the pose ranges go to
+// slots of a workspace, which k_finish2 sums in fp64 into the image, with the
+// x = 0 Hermitian completion of the backprojection; without a workspace they
+// are added into the zero-filled image with float atomics (once per cell and
+// range) and k_mirror2_x0 completes it.
 //
 // Poses whose 2x2 matrix has singular values in [kScaleMin, kScaleMax]
 // (pose_tiled2: rotations, and scaled or sheared matrices) take this path;
