@@ -547,8 +547,10 @@ struct CallScratch {
             if (capturing) return nullptr;
             // (a size that the last attempt could not get is tried again after kBinsRetry calls: freeing
             // the workspace and waiting for the stream on each of them would cost more than it can give)
-            if (area->bins_failed && need >= area->bins_failed && area->bins_refused++ < kBinsRetry) return nullptr;
-            area->bins_failed = 0;
+            if (area->bins_failed && need >= area->bins_failed) {
+                if (area->bins_refused++ < kBinsRetry) return nullptr;
+                area->bins_failed = 0;
+            }
             if (hipStreamSynchronize(st) != hipSuccess) return nullptr;
             if (area->bins) {
                 if (area->bins_captured) area->bins_retired.push_back(area->bins);
