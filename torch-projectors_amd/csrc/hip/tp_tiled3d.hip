@@ -1842,9 +1842,11 @@ hipError_t forw_store(bool cubic, const Geom& g, const TileSpec& ts, const ForwW
 }  // namespace
 
 void forw_reach_tiles(const TileSpec& ts, const PoseSplit& ps, std::vector<TileAt>& out, int n[kSplitLevels + 1]) {
-    // the rotation kernel's test (dist2 > rho2: the tile holds no sample) with a margin, so that
-    // its own arithmetic drops no tile that the list leaves out
-    const float rho2 = (ts.rho_unit + 1.5f) * (ts.rho_unit + 1.5f);
+    // the rotation kernel's test (dist2 > rho2: the tile holds no sample) with a margin for its rounding,
+    // so that every tile the kernel would take is listed.  No wider: listed tiles that the kernel drops
+    // leave its workgroups uneven (half a voxel: cubic gradients of 512 backprojected poses of 256 x 256 at
+    // oversampling 1 took 1.209 ms against 1.131, the linear forward 0.198 against 0.192).
+    const float rho = ts.rho_unit + 1.0f, rho2 = rho * rho * 1.001f + 4.0f;
     auto axis2 = [&](int t, int edge) {
         const float lo = float(t) - ts.eps, hi = float(t + edge) + ts.eps;
         const float q = lo > 0.f ? lo : (hi < 0.f ? -hi : 0.f);
