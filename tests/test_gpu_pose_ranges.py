@@ -31,6 +31,13 @@ def _cases():
                 seed += 1
                 out.append(_case(f"{op}_{interp}_n{n}_os{os_:g}_P{P}", op, interp=interp, os=os_, cutoff=None, B=2, P=P,
                                  n=n, B_rot=2, seed=seed, weights=(seed % 2 == 0)))
+    # 3D batches whose work balances without levels: one level of two pieces, and the levels just below
+    for op, interp, B in (("project_3d_to_2d_forw", "cubic", 80), ("project_3d_to_2d_back", "cubic", 120),
+                          ("project_3d_to_2d_back", "cubic", 40), ("backproject_2d_to_3d_forw", "linear", 90),
+                          ("backproject_2d_to_3d_forw", "linear", 60), ("backproject_2d_to_3d_back", "cubic", 80)):
+        seed += 1
+        out.append(_case(f"{op}_{interp}_n16_B{B}_P520", op, interp=interp, os=2.0, cutoff=None, B=B, P=520, n=16, B_rot=B,
+                         seed=seed, weights=True))
     return out
 
 

@@ -160,21 +160,34 @@ constexpr double kMaxScatterPieces = double(1 << 15), kMaxGatherPieces = double(
 //     poses of 90 x 90 at oversampling 1.5, cubic forward and backward 1.59 -> 0.84 ms; 1000 poses of
 //     64 x 64 at 2, linear: backprojection 0.211 -> 0.124, projection with all gradients 0.549 -> 0.279 ms;
 //     1000 of 64 x 64 at 1, cubic backprojection 3.34 -> 0.65 ms.
-//   - in calls where that is 512 poses or more (and without `levels`), one level of 40 voxels with `range`
-//     poses per piece: there the levels measured slower (the headline backprojection 1.33 -> 1.39 ms:
-//     less of the projections' rows is shared by the pieces that run together).
+//   - in one level of 40 voxels with at most `range` poses per piece where that balances by itself: where
+//     its longest list, that of a core piece or of an unsplit tile next to the core, is below `balanced`
+//     times cross / per_slot over the workgroups.  Pieces that run together then share more of the
+//     projections' rows and there are fewer of them.  Both sides, at this ratio (one level / levels, ms):
+//       gathers     1.4 linear forward of 1400 x 256 x 256 at oversampling 1: 0.32 / 0.47; cubic gradients of a
+//                   backprojection, 700 of them: 1.29 / 1.54; 1.58 cubic, 1100 of 192 x 192 at 1.25: 0.53 /
+//                   0.57; 1.65 linear, 5000 of 96 x 96 at 2: 0.250 / 0.280; 1.71, 3000 of 160 x 160 at 1: 0.433 /
+//                   0.391; 2.2, 1100 of 192 x 192 at 1.5: 0.31 / 0.20; 2.7, 6000 of 128 x 128 at 1: 0.77 / 0.40;
+//       scatters    linear, 1.05 1100 of 256 x 256 at 1: 0.89 / 1.02; 1.24 700 of 192 x 192 at 1.5: 0.340 / 0.365;
+//                   1.57 800 of 256 x 256 at 1: 0.736 / 0.762, 8 x 333 of 64 x 64 at 2: 0.238 / 0.211; 3.2
+//                   6000 of 128 x 128 at 1: 2.19 / 1.54; cubic, 1.0 2048 of 256 x 256 at 1: 11.6 / 12.3; 1.35
+//                   1400 of them: 8.8 / 8.5; 1.54 1100 of 192 x 192 at 1.25: 3.72 / 4.04; 2.0 1024 of 256 x 256 at
+//                   1: 7.2 / 6.2; the headline backprojection, 0.7: 1.33 / 1.39.
+constexpr double kBalancedGather = 1.7, kBalancedScatter = 1.55;
 tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const int org[3], const int edge[3],
-                         double stencil, double per_slot, double least, int64_t range, double most, bool levels = true) {
-    constexpr double kSlots = 1024.0, kLongRange = 512.0;
+                         double stencil, double per_slot, double least, int64_t range, double most, double balanced) {
+    constexpr double kSlots = 1024.0, kCore = 40.0;
     const double h = 0.25 * (edge[0] + edge[1] + edge[2] + 3.0 * stencil);
     const double vt = double(edge[0]) * edge[1] * edge[2], R = std::max(reach, h);
     const double cross =
         double(g.B) * double(g.P) * 2.0 * M_PI / vt * (h * h * h / 3.0 + h * (R * R - h * h) / 2.0);
-    double target = std::max(least, cross / (kSlots * per_slot));
-    const bool one_level = !levels || target >= kLongRange;
-    if (one_level) target = double(range);
+    const double even = cross / (kSlots * per_slot);
+    const double core_list = double(g.P) / std::ceil(double(g.P) / double(range));
+    const double next_list = reach > kCore ? double(g.P) * std::min(1.0, h / (kCore + 6.0)) : 0.0;
+    const bool one_level = std::max(core_list, next_list) < balanced * even;
+    const double target = one_level ? double(range) : std::max(least, even);
     tp::PoseSplit ps{};
-    double r = one_level ? 40.0 : 16.0, p = 1.0;  // this level's half width; share of the poses that cross its tiles
+    double r = one_level ? kCore : 16.0, p = 1.0;  // this level's half width; share of the poses that cross its tiles
     double total = 0.0;
     for (int l = 0; l < (one_level ? 1 : tp::kSplitLevels); ++l, r *= 2.0) {
         // (21 poses in two pieces for a target of 16 cost more than they balanced)
@@ -193,7 +206,7 @@ tp::PoseSplit pose_split(const tp::Geom& g, double reach, const int n[3], const 
         total += double(g.B) * double(tiles) * double(k);
         if (total > most || k > tp::kMaxTilePieces || double(ps.pieces) + double(tiles) * double(k) > double(INT32_MAX))  // (twice as long until they fit)
             return pose_split(g, reach, n, org, edge, stencil, per_slot / 2.0, 2.0 * target, 2 * int64_t(target), most,
-                              levels);
+                              balanced);
         v.k = int(k);
         v.pieces = int(tiles * k);
         v.by_pieces = tp::divisor(unsigned(v.pieces));
@@ -220,7 +233,7 @@ tp::PoseSplit scatter_split(const tp::Geom& g, const tp::TileSpec& ts, bool cubi
               edge[3] = {tp::kScTD, tp::kScTR, tp::kScTC};
     return pose_split(g, double(ts.rho_unit), n, org, edge, cubic ? 3.0 : 1.0, cubic ? 1.5 : 1.0, cubic ? 16.0 : 48.0,
                       op == TileOp::backproject ? std::min<int64_t>(2048, std::max<int64_t>(512, g.P / 4)) : 512,
-                      kMaxScatterPieces, levels);
+                      kMaxScatterPieces, levels ? kBalancedScatter : INFINITY);
 }
 tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, tp::ForwWorks& fw) {
     constexpr int L = tp::kTileEdge;
@@ -257,8 +270,8 @@ tp::TileSpec tile_spec(const tp::Geom& g, bool cubic, TileOp op, tp::ForwWorks& 
     const double flo = op == TileOp::project ? 64.0 : 32.0;
     fw.rot.split =
         pose_split(g, rho_unit, nf, of, ef, 0.0, 0.5, flo, op == TileOp::project ? forw_poses_per_range(g.os) : 512,
-                   kMaxGatherPieces);
-    fw.gen.split = pose_split(g, rho_unit, nf2, of2, ef, 0.0, 0.5, flo, 512, kMaxGatherPieces);
+                   kMaxGatherPieces, kBalancedGather);
+    fw.gen.split = pose_split(g, rho_unit, nf2, of2, ef, 0.0, 0.5, flo, 512, kMaxGatherPieces, kBalancedGather);
     ts.rho = float(rho);
     ts.rho_unit = float(rho_unit);
     ts.os = float(g.os);
