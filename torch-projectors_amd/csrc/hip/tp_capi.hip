@@ -370,24 +370,25 @@ void pose_ranges2(const tp::Geom& g, tp::TileSpec2& ts, int64_t ksplit) {
 // that a call of rotations leaves at once, a zero fill or a completion pass); a per-pixel one is a
 // single launch that reads every tap through the caches, cheaper per sample the smaller the volume
 // and, at small oversampling, the closer the samples.  The lines below were fitted to both sides
-// measured over 32 <= n <= 2048, oversampling 0.5 to 3, 2 to 60000 poses (393 calls: the slower side is
-// taken by at most 6 % in favour of per pixel, and where noted in favour of the tiles), in us (tiled /
-// per pixel):
+// measured over 32 <= n <= 2048, oversampling 0.5 to 3, 2 to 60000 poses, 1 to 64 volumes (over 500 calls;
+// per pixel is taken where it is up to 12 % slower, the tiles where noted and in batches of small
+// gradient calls), in us (tiled / per pixel):
 //   forward, linear: 100 poses of 48 at oversampling 2, 27 / 11; 1000 of 64 58 / 54, 2000 80 / 98; 100 of
 //     128 54 / 37, 300 of them 66 / 90; 100 of 256 246 / 146, 200 277 / 282; 200 of 512 1795 / 1473, 400
-//     2020 / 2889; at oversampling 1, whose samples share lines, 4000 of 64 130 / 80, 700 of 128 85 / 78, 1500
-//     137 / 155; cubic, 60 of 64 at 2 44 / 38, 150 52 / 64; 40 of 256 361 / 325, 100 470 / 753; 60 of 512
-//     2301 / 2608;
-//   forward 2D, linear: 8 x 4000 of 64 482 / 379, 8 x 2000 of 128 710 / 714, 8 x 300 of 256 452 / 432 and 600
-//     805 / 844; an image that outgrows an XCD's L2 costs a per-pixel sample twice as much: 10 of 1024 at
-//     oversampling 2 49 / 78, 100 312 / 682 (30 of 1024 at 1, 140 / 94); cubic, 500 of 128 73 / 61, 1000
+//     2020 / 2889; 4 x 100 of 128 147 / 125, 4 x 130 155 / 160; at oversampling 1, whose samples share
+//     lines, 4000 of 64 130 / 80, 700 of 128 85 / 78, 1500 137 / 155; cubic, 60 of 64 at 2 44 / 38, 150 52
+//     / 64; 40 of 256 361 / 325, 100 470 / 753; 60 of 512 2301 / 2608; 8 x 24 of 128 427 / 381, 8 x 33 466
+//     / 502;
+//   forward 2D, linear: 8 x 4000 of 64 482 / 379, 8 x 2000 of 128 710 / 714, 8 x 300 of 256 452 / 432 and
+//     600 805 / 844; an image that outgrows an XCD's L2 costs a per-pixel sample twice as much: 10 of 1024
+//     at oversampling 2 49 / 78, 100 312 / 682 (30 of 1024 at 1, 140 / 94); cubic, 500 of 128 73 / 61, 1000
 //     111 / 113; 10 of 1024 75 / 162;
-//   gradient gathers (with every gradient; projection, then backprojection): 1000 of 64 238 / 162 and
-//     167 / 111 (2000 of them, 368 / 249 and 262 / 205, still take the tiles); 200 of 128 234 / 173 and
-//     162 / 140, 500 338 / 293 (tiles) and 242 / 304; 200 of 256 906 / 814 and 744 / 645; cubic, 90 of 64
-//     168 / 147 and 105 / 75, 150 of 128 369 / 456 and 274 / 371.  2D: 600 of 64 78 / 65 and 60 / 46, 400 of 128
-//     109 / 131 and 78 / 84; a pose of many blocks waits for its own sums' atomics (60 of 200, 97 / 104
-//     and 71 / 74), so those boxes stay tiled.
+//   gradient gathers (with every gradient; projection, then backprojection): 1000 of 64 238 / 162 and 167 /
+//     111 (2000 of them, 368 / 249 and 262 / 205, still take the tiles); 200 of 128 234 / 173 and 162 /
+//     140, 260 244 / 192 and 168 / 176, 500 338 / 293 (tiles) and 242 / 304; 200 of 256 906 / 814 and 744 /
+//     645; cubic, 90 of 64 168 / 147 and 105 / 75, 150 of 128 369 / 456 and 274 / 371.  2D: 600 of 64 78 /
+//     65 and 60 / 46, 400 of 128 109 / 131 and 78 / 84; a pose of many blocks waits for its own sums'
+//     atomics (60 of 200, 97 / 104 and 71 / 74), so those boxes stay tiled.
 // Projections of a call's active pixels and the tiles that its samples reach:
 double active_samples(const tp::Geom& g) { return 0.785 * double(g.B) * double(g.P) * double(g.rect); }
 double reach_of(const tp::Geom& g) { return std::min(g.os * std::sqrt(std::max(0.0, g.cut2)), g.os * double(g.n)); }
@@ -411,16 +412,17 @@ bool small_forward(int dim, const tp::Geom& g, bool cubic) {
         if (beyond_l2) return A < 4e6 * large * std::min(4.0, shared * shared);
         return A < (vol <= 40000.0 ? 9e7 : 5.5e7);
     }
-    const double tiles = reached_tiles(g), cells = reached_cells(g);
-    if (cubic) return A < 0.15e6 * shared * shared * (1.0 + 0.2e6 / cells) + 44.0 * double(g.B) * tiles / (1.0 + tiles / 4e5);
-    return A < 0.75e6 * shared * std::sqrt(shared) * (1.0 + 1.3e6 / cells) + 150.0 * double(g.B) * tiles;
+    const double tiles = reached_tiles(g), cells = reached_cells(g), each = double(g.B) * tiles;
+    if (cubic) return A < 0.15e6 * shared * shared * (1.0 + 0.2e6 / cells) + 55.0 * each / (1.0 + tiles / 2e5);
+    return A < 0.75e6 * shared * std::sqrt(shared) * (1.0 + 1.3e6 / cells) + 195.0 * each / (1.0 + tiles / 5e5);
 }
-bool small_gradients(int dim, const tp::Geom& g, bool cubic) {
+bool small_gradients(int dim, const tp::Geom& g, bool cubic, bool backprojection) {
     const double A = active_samples(g), shared = samples_shared(g);
     if (dim == 2) return A < (cubic ? 1.0e6 : 1.5e6) * shared && g.chunks <= 40;
     const double tiles = double(g.B) * reached_tiles(g) * std::min(4.0, g.os * g.os / 4.0), cells = reached_cells(g);
-    return A < (cubic ? 0.25e6 * std::min(2.0, shared) * (1.0 + 0.4e6 / cells) + 40.0 * tiles
-                      : 1.0e6 * (1.0 + 1.7e6 / cells) + 270.0 * tiles);
+    if (cubic) return A < 0.25e6 * std::min(2.0, shared) * (1.0 + 0.4e6 / cells) + 40.0 * tiles;
+    return A < (backprojection ? 0.85e6 * (1.0 + 2.1e6 / cells) + 240.0 * tiles
+                               : 1.0e6 * (1.0 + 1.7e6 / cells) + 270.0 * tiles);
 }
 
 // The calling thread's tp_set_gather_route, and the gathers its last call took.
@@ -899,7 +901,7 @@ int project_back(int dim, int dtype, const void* gproj, int64_t B, int64_t P, in
     CallScratch sc;
     // (complex-half volumes have no per-pixel gradients without the scatter)
     const bool per_pixel =
-        (tiles || tiles2) && (grot || gshift) && !rec_half && takes_per_pixel(small_gradients(dim, g, cubic));
+        (tiles || tiles2) && (grot || gshift) && !rec_half && takes_per_pixel(small_gradients(dim, g, cubic, false));
     const bool tiled_gradients = (grot || gshift) && !per_pixel;
     if (tiles) {
         tp::ForwWorks fw{};
@@ -1012,7 +1014,7 @@ int backproject_back(int dim, int dtype, const void* gdata, const void* gw, int6
     const bool cubic = interp == TP_CUBIC;
     bool tiles2 = use_tiles2(dim, dtype, os, n), tiles = use_tiles(dim, dtype, os, n);
     CallScratch sc;
-    if ((tiles || tiles2) && takes_per_pixel(small_gradients(dim, g, cubic))) {
+    if ((tiles || tiles2) && takes_per_pixel(small_gradients(dim, g, cubic, true))) {
         TP_TRY(sc.get(s));  // (a stream's first call is refused under capture, whatever its size)
         tiles = tiles2 = false;
     }
